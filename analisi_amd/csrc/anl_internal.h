@@ -103,6 +103,7 @@ struct anl_series {
     uint64_t nrows = 0;
     uint32_t ncols = 0;
     double *data = nullptr;
+    double2 *rec = nullptr;  // [nrows] 1/c, c = 1 .. nrows, in two parts (gk_reciprocals)
     // Green-Kubo scratch (splits, partial sums, output staging), grow-only;
     // calls on one series are stream-ordered on the caller's stream.
     void *work = nullptr;
@@ -147,9 +148,13 @@ void *series_workspace(anl_series *s, size_t bytes);
 // FP64 Green-Kubo epilogue (mean subtraction, running integrals, Schur
 // complement) over d[leff][narr] whose first ncur^2 columns hold C(l); the
 // mean and the integrals as the reference's serial scans, or as parallel
-// sums (different rounding) when serial_scans is false.
+// sums (different rounding) when serial_scans is false.  rec: 1/c for the
+// serial mean's counter (anl_series::rec).
 void gk_epilogue(double *d, uint32_t narr, uint32_t ncur, uint32_t leff, int subtract_mean, uint32_t start_mean,
-                 hipStream_t s, uint32_t nblocks, uint64_t stride, bool serial_scans);
+                 hipStream_t s, uint32_t nblocks, uint64_t stride, bool serial_scans, const double2 *rec);
+// rec[c-1] = {RN(1/c), the rest of 1/c}, c = 1 .. n: running means divide by
+// their counter through it.
+void gk_reciprocals(double2 *rec, uint64_t n, hipStream_t s);
 // Lag products of every block (split-BF16 MFMA) into d + b * leff * narr:
 // C(l) in the first ncur^2 columns, zeros elsewhere; scratch from the series.
 void gk_mfma_enqueue_blocks(anl_series *s, const uint32_t *idx_j, uint32_t ncur, uint32_t skip, uint32_t leff,

@@ -2,16 +2,17 @@
 // 156-356) on the device, in the reference's FP64 operation order so that the
 // correlation functions, their integrals and the transport coefficients match
 // the reference's values:
-//  * gk_lag_kernel: one thread per lag l holds the ncur^2 running means
+//  * gk_chain_kernel: a lane per (lag l, current pair ab, segment, block)
+//    holds the running mean
 //      JJ[ab] += ((Ja(t0).Jb(t0+l))/3 - JJ[ab]) / cont      (:200-228)
-//    over t0 = align, align+skip, .. < seg*(iseg+1) of each of the n_seg
-//    segments, and the running mean of the segment means (:230-237).
-//    Rows t0 are shared by all threads of a workgroup (broadcast loads), rows
-//    t0+l are consecutive across threads.
+//    over t0 = align, align+skip, .. < seg*(iseg+1) of its segment;
+//    gk_segments_kernel takes the running mean of the segment means
+//    (:230-237).
 //  * gk_mean_kernel / gk_integral_kernel / gk_schur_kernel: the serial
 //    epilogue (:259-356) as column-parallel prefix scans and a lag-parallel
 //    Schur complement of the symmetrised integral matrix.
 #include <algorithm>
+#include <type_traits>
 
 #include "anl_internal.h"
 
@@ -32,208 +33,665 @@ struct GkBlocks {
 
 struct GkArgs {
     const double *data;
+    const double2 *rec;  // [nrows] {RN(1/c), the rest of 1/c}, c = 1 ..
+    uint64_t nrows;
     uint32_t ncols;
     uint32_t ncur;
     uint32_t idx[GK_MAXC];
     uint32_t n_seg, skip, leff, narr;
+    uint32_t seg0;        // first segment of this launch
     uint64_t out_stride;
-    double *out;  // [block][leff][narr]
+    double *out;   // [block][leff][narr]
+    double *segm;  // segment means [block][segment][pair][lag], or null: fold into out
     GkBlocks bl;
 };
 
-template <int NC>
-__global__ __launch_bounds__(256) void gk_lag_kernel(const GkArgs a) {
-    const uint32_t it = blockIdx.x * blockDim.x + threadIdx.x;
-    if (it >= a.leff) return;
-    const uint32_t blk = blockIdx.y;
+// a / c for an integer c < 2^32 from y = {yh, yl}, yh = RN(1/c) and yl =
+// 1/c - yh to about 2^-50 of itself: the correctly rounded quotient, in two
+// operations.  yh + yl is 1/c to 2^-102 of it, and a yl rounds once, so the
+// last rounding sees a/c to better than 2^-100 of it.  With the quotient
+// scaled so that its rounding midpoints are odd integers M < 2^54, a/c is
+// never a midpoint (c M has 54 significant bits or more, a has 53), so
+// |a/c - M| >= 1/c > 2^-32, which is far more than 2^54 2^-100: both sides
+// round to the same number.  Needs |a| in (GK_TINY, inf): below it a yl may
+// lose bits to underflow, and inf * 0 is not a number.
+constexpr double GK_TINY = 0x1p-900;
+__device__ __forceinline__ double div_by(double a, double2 y) { return fma(a, y.x, a * y.y); }
+
+__global__ __launch_bounds__(256) void gk_reciprocal_kernel(double2 *__restrict__ rec, uint64_t n) {
+    const uint64_t k = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (k >= n) return;
+    const double c = (double)(k + 1), y = 1.0 / c;
+    rec[k] = make_double2(y, fma(-c, y, 1.0) / c);
+}
+
+// Lane J of each row of 16 lanes, in every lane of the row: what all lanes
+// need of 16 t0 sits in one register and costs a move each, where an LDS
+// broadcast moves 512 bytes through a port of 128 per clock.
+template <int J>
+__device__ __forceinline__ double row_lane(double v) {
+#ifdef __HIP_DEVICE_COMPILE__
+    const long long x = __builtin_bit_cast(long long, v);
+    const long long r = __builtin_amdgcn_update_dpp(0ll, x, 0x150 + J, 0xf, 0xf, true);  // row_newbcast:J
+    return __builtin_bit_cast(double, r);
+#else
+    return v;
+#endif
+}
+
+// Smallest |d| so far, by the high words read as FP32: their order is that of
+// the doubles (what reads as a NaN is 2^1017 or more, and either passes or
+// sends the steps to true divisions); one operation for two values.
+constexpr float GK_TINY_HI = 0x1.6p-112f;  // 0x07b00000, the high word of GK_TINY
+__device__ __forceinline__ void track_min(float &m, double d0, double d1) {
+    const int h0 = __double2hiint(d0), h1 = __double2hiint(d1);
+    asm("v_min3_f32 %0, |%1|, |%2|, %0" : "+v"(m) : "v"(h0), "v"(h1));
+}
+
+template <int N, int I = 0, class F>
+__device__ __forceinline__ void gk_for(F &&f) {  // f(integral_constant 0) .. f(integral_constant N-1)
+    if constexpr (I < N) {
+        f(std::integral_constant<int, I>{});
+        gk_for<N, I + 1>(f);
+    }
+}
+
+// One workgroup = 64 lags of one current pair, one segment and one block, a
+// running mean per lane:
+//     JJ += ((Ja(t0).Jb(t0+l))/3 - JJ) / cont            (:200-228)
+// The chain over t0 is serial (its roundings are the reference's): four
+// dependent FP64 operations per t0, 5.4 clocks each, and a wavefront issues
+// an instruction of any kind about every 4.3 clocks.  So wavefront 0 runs the
+// chain and nothing else, and wavefronts 1 to 3 form the terms Ja.Jb/3 of the
+// next round of T = 48 t0, 16 each, and hand them over in LDS (two buffers,
+// one barrier per round).  They also stage the rows: global loads two rounds
+// ahead into registers, then LDS.
+// LDS: Jb as one plane per component; with t0 stride 1 a lane's rows of two
+// consecutive t0 are adjacent and each row is stored with its successor, so
+// that one 16-byte read serves both (ds_read2_b64 of the two measured twice
+// the time).  LDS traffic is 20 clocks per t0.
+// Divisions by 3 and by cont are two operations each (div_by); steps outside
+// its range (a difference or product of zero included) take true divisions.
+// Rows of a round: contiguous where skip <= 64 (row rr of the round is
+// series row base + rr), else 64 rows per t0.
+// Measured, 2 currents: 5,000 lags x 95,001 t0 2.85 ms (47 to 50 clocks per
+// t0; one thread per lag with true divisions took 44.2 ms), 2,000 lags x 4
+// segments of 4,500 t0 0.16 ms (8.37 ms).
+constexpr uint32_t gk_rows(uint32_t T, uint32_t maxskip) { return 64 + (T - 1) * maxskip; }
+// doubles of a plane of at least n: planes start 12 banks apart, so that the
+// lanes of a store, which walk all planes, spread over the banks (with planes
+// a multiple of 64 banks apart the stores conflicted six ways and took half of
+// the LDS time)
+constexpr uint32_t gk_plane(uint32_t n) { return (n + 25) / 32 * 32 + 6; }
+
+template <uint32_t T, uint32_t MAXSKIP>
+__global__ __launch_bounds__(256, 1) void gk_chain_kernel(const GkArgs a) {
+    constexpr bool ONE = MAXSKIP == 1;
+    constexpr uint32_t ROWS = gk_rows(T, MAXSKIP), NC = ONE ? 2 : 1, PL = gk_plane(NC * ROWS), G = T / 16;
+    constexpr uint32_t NPT = 192, PF = (3 * ROWS + NPT - 1) / NPT;
+    static_assert(3 * T <= NPT && T % 16 == 0 && G <= 3, "16 t0 and one Ja value per producer");
+    __shared__ __align__(16) double Bs[2][3][PL];  // t0 stride 1: rows r and r + 1 at 2r
+    __shared__ double As[2][3][T];
+    __shared__ double Ys[4][2][T];
+    __shared__ __align__(16) double2 Xs[2][T / 2][64];  // terms of t0 2i, 2i + 1
+    const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63u, l16 = lane & 15u;
+    const uint32_t np = a.ncur * a.ncur, ntile = (a.leff + 63) / 64;
+    const uint32_t pair = blockIdx.x / ntile, tile = blockIdx.x - pair * ntile;
+    const uint32_t iseg = a.seg0 + blockIdx.y, blk = blockIdx.z;
     const uint64_t primo = a.bl.primo[blk];
-    const uint32_t n = a.bl.n[blk];
-    constexpr int NP = NC * NC;
-    double v[NP], JJ[NP];
+    const uint32_t seg = a.bl.n[blk] / a.n_seg;
+    const uint32_t first = seg * iseg + (seg * iseg) % a.skip, end = seg * (iseg + 1);  // :208
+    const uint32_t n0 = first < end ? (end - first + a.skip - 1) / a.skip : 0;
+    const uint32_t nst = (n0 + T - 1) / T;
+    double JJ = 0.0;
+    if (wave == 0) {
+        struct Sub {
+            double2 x[8];
+            double y0, y1;
+        };
+        float dmin = 1.0f;
+        auto read = [&](Sub &r, uint32_t k, uint32_t g) {
 #pragma unroll
-    for (int k = 0; k < NP; k++) v[k] = 0.0;
-    const uint32_t seg = n / a.n_seg;
-    uint32_t cont_JJ = 0;
-    for (uint32_t iseg = 0; iseg < a.n_seg; iseg++) {
-        ++cont_JJ;
-#pragma unroll
-        for (int k = 0; k < NP; k++) JJ[k] = 0.0;
-        uint32_t cont = 0;
-        const uint32_t allinea = (seg * iseg) + (seg * iseg) % a.skip;
-        for (uint32_t jm = allinea; jm < seg * (iseg + 1); jm += a.skip) {
-            cont++;
-            const double *la = a.data + (primo + jm) * a.ncols;
-            const double *lb = a.data + (primo + jm + it) * a.ncols;
-            double A[NC][3], B[NC][3];
-#pragma unroll
-            for (int c = 0; c < NC; c++)
-#pragma unroll
-                for (int x = 0; x < 3; x++) {
-                    A[c][x] = la[a.idx[c] + x];
-                    B[c][x] = lb[a.idx[c] + x];
-                }
-            const double dc = (double)cont;
-#pragma unroll
-            for (int j1 = 0; j1 < NC; j1++)
-#pragma unroll
-                for (int j2 = 0; j2 < NC; j2++) {
-                    const int k = j1 * NC + j2;
-                    double p = A[j1][0] * B[j2][0];
-                    p = p + A[j1][1] * B[j2][1];
-                    p = p + A[j1][2] * B[j2][2];
-                    const double delta = p / 3.0 - JJ[k];
-                    JJ[k] = JJ[k] + delta / dc;
-                }
-        }
-        const double dcj = (double)cont_JJ;
-#pragma unroll
-        for (int k = 0; k < NP; k++) v[k] = v[k] + (JJ[k] - v[k]) / dcj;
-    }
-    double *o = a.out + blk * a.out_stride + (uint64_t)it * a.narr;
-#pragma unroll
-    for (int k = 0; k < NP; k++) o[k] = v[k];
-    for (uint32_t k = NP; k < a.narr; k++) o[k] = 0.0;
-}
-
-// The serial scans over lags below read C(it) of every correlation column
-// through LDS: waves 1-3 of the workgroup load the next tile of lags (all
-// columns, coalesced) while the lanes of wave 0 that own a column scan the
-// current tile in the reference's order.  Tiles double-buffer; one barrier
-// per tile.
-// Each thread issues 8 global loads before the first LDS write, so a tile
-// costs about one memory latency rather than one per element.
-__device__ __forceinline__ void gk_load_tile(double *__restrict__ dst, const double *__restrict__ out, uint32_t narr,
-                                             uint32_t ncorr, uint32_t it0, uint32_t leff, uint32_t tl, uint32_t t,
-                                             uint32_t nt) {
-    constexpr uint32_t B = 8;
-    const uint32_t total = tl * ncorr;
-    for (uint32_t e0 = t; e0 < total; e0 += B * nt) {
-        double v[B];
-#pragma unroll
-        for (uint32_t j = 0; j < B; j++) {
-            const uint32_t e = e0 + j * nt;
-            const uint32_t k = e / ncorr, jj = e - k * ncorr;
-            const uint32_t it = it0 + k;
-            v[j] = (e < total && it < leff) ? out[(uint64_t)it * narr + jj] : 0.0;
-        }
-#pragma unroll
-        for (uint32_t j = 0; j < B; j++)
-            if (e0 + j * nt < total) dst[e0 + j * nt] = v[j];
-    }
-}
-
-// :259-277 subtract the mean of C over lags [start_mean, leff).
-__global__ __launch_bounds__(256) void gk_mean_kernel(double *__restrict__ out, uint32_t narr, uint32_t ncorr,
-                                                      uint32_t leff, uint32_t start_mean, uint64_t stride,
-                                                      uint32_t tl) {
-    extern __shared__ double tile[];  // [2][tl][ncorr], then [ncorr] means
-    out += blockIdx.y * stride;
-    const uint32_t t = threadIdx.x;
-    double *mean_lds = tile + 2 * tl * ncorr;
-    double m = 0.0;
-    uint32_t c = 0;
-    if (start_mean < leff) {
-        if (t >= 64) gk_load_tile(tile, out, narr, ncorr, start_mean, leff, tl, t - 64, blockDim.x - 64);
+            for (uint32_t j = 0; j < 8; j++) r.x[j] = Xs[k & 1u][8 * g + j][lane];
+            r.y0 = Ys[k & 3u][0][16 * g + l16];
+            r.y1 = Ys[k & 3u][1][16 * g + l16];
+        };
+        // the chain over the 16 steps in r, the operands of group g of round k
+        // read into n between its operations: each of them waits for the one
+        // before and leaves an issue slot (the barriers keep the order)
+        auto steps = [&](const Sub &r, Sub &n, uint32_t k, uint32_t g) {
+            const double2 *X = &Xs[k & 1u][8 * g][lane];
+            double dlast = 0.0;
+            gk_for<16>([&](auto jc) {
+                constexpr int j = decltype(jc)::value;
+                const double d = (j & 1 ? r.x[j / 2].y : r.x[j / 2].x) - JJ;
+                const double yl = row_lane<j>(r.y1);
+                __builtin_amdgcn_sched_barrier(0);
+                const double m = d * yl;
+                const double yh = row_lane<j>(r.y0);
+                __builtin_amdgcn_sched_barrier(0);
+                const double q = fma(d, yh, m);
+                if constexpr (j & 1) n.x[j / 2] = X[j / 2 * 64];
+                else if constexpr (j == 0) n.y0 = Ys[k & 3u][0][16 * g + l16];
+                else if constexpr (j == 2) n.y1 = Ys[k & 3u][1][16 * g + l16];
+                __builtin_amdgcn_sched_barrier(0);
+                JJ = JJ + q;
+                if constexpr (j & 1) track_min(dmin, dlast, d);
+                dlast = d;
+                __builtin_amdgcn_sched_barrier(0);
+            });
+        };
+        auto slow = [&](uint32_t k, uint32_t s0, uint32_t s1) {  // steps s0 .. s1 - 1 of round k with true divisions
+            for (uint32_t s = s0; s < s1; s++) {
+                const double2 x = Xs[k & 1u][s / 2][lane];
+                const double d = (s & 1 ? x.y : x.x) - JJ;
+                JJ = JJ + d / (double)(k * T + s + 1);
+            }
+        };
         __syncthreads();
-        uint32_t buf = 0;
-        for (uint32_t it0 = start_mean; it0 < leff; it0 += tl) {
-            if (t >= 64 && it0 + tl < leff)
-                gk_load_tile(tile + (buf ^ 1) * tl * ncorr, out, narr, ncorr, it0 + tl, leff, tl, t - 64,
-                             blockDim.x - 64);
-            if (t < ncorr) {
-                const double *col = tile + buf * tl * ncorr + t;
-                const uint32_t n = min(tl, leff - it0);
-                for (uint32_t k = 0; k < n; k++) {
-                    c++;
-                    const double d = col[k * ncorr] - m;
-                    m = m + d / (double)c;
+        __syncthreads();
+        for (uint32_t k = 0; k < nst; k++) {
+            const uint32_t cnt = min(T, n0 - k * T), full = cnt / 16;
+            const double J0 = JJ;
+            dmin = 1.0f;
+            Sub r0, r1;
+            if (full) read(r0, k, 0);
+            for (uint32_t g = 0; g < full; g += 2) {
+                steps(r0, r1, k, min(g + 1, G - 1));
+                if (g + 1 < full) steps(r1, r0, k, min(g + 2, G - 1));
+            }
+            if (__ballot(!(dmin > GK_TINY_HI) || !(fabs(JJ) < 0x1p1000))) {
+                JJ = J0;
+                slow(k, 0, 16 * full);
+            }
+            slow(k, 16 * full, cnt);  // the last round's remainder
+            __syncthreads();
+        }
+    } else {
+        const uint32_t p = threadIdx.x - 64u;  // producer thread
+        const uint32_t ca = a.idx[pair / a.ncur], cb = a.idx[pair % a.ncur];
+        const uint64_t ra = primo + first, rb = ra + (uint64_t)tile * 64u, last = a.nrows - 1;
+        const uint32_t skip = a.skip, rs = min(skip, 64u);
+        // this thread's loads of a round: PF values of Jb rows, one of Ja, one
+        // part of 1/cont.  Rows past the series' end are clamped to the last
+        // one (their lags are not used).
+        struct Regs {
+            double b[PF], a, y;
+        };
+        const double *pb[PF], *lb[PF];
+#pragma unroll
+        for (uint32_t j = 0; j < PF; j++) {
+            const uint32_t e = p + NPT * j, rr = e / 3, x = e - 3 * rr;
+            const uint64_t off = skip <= 64 ? rr : (uint64_t)(rr / 64) * skip + rr % 64;
+            pb[j] = a.data + (rb + off) * a.ncols + cb + x;
+            lb[j] = a.data + last * a.ncols + cb + x;
+        }
+        const uint32_t pa3 = min(p, 3 * T - 1), py = min(p, 2 * T - 1);
+        const double *pa = a.data + (ra + (uint64_t)(pa3 / 3) * skip) * a.ncols + ca + pa3 % 3;
+        const double *la = a.data + last * a.ncols + ca + pa3 % 3;
+        const double *pyr = reinterpret_cast<const double *>(a.rec) + py;
+        const double *ly = reinterpret_cast<const double *>(a.rec) + 2 * last + (py & 1u);
+        const uint64_t step = (uint64_t)T * skip * a.ncols;
+        auto fetch = [&](Regs &r) {  // the next round's
+#pragma unroll
+            for (uint32_t j = 0; j < PF; j++) {
+                r.b[j] = *(pb[j] < lb[j] ? pb[j] : lb[j]);
+                pb[j] += step;
+            }
+            r.a = *(pa < la ? pa : la);
+            pa += step;
+            r.y = *(pyr < ly ? pyr : ly);
+            pyr += 2 * T;
+        };
+        auto stash = [&](const Regs &r, uint32_t k) {
+#pragma unroll
+            for (uint32_t j = 0; j < PF; j++) {
+                const uint32_t e = p + NPT * j, rr = e / 3, x = e - 3 * rr;
+                if (rr < ROWS) {
+                    Bs[k & 1u][x][NC * rr] = r.b[j];
+                    if (ONE && rr) Bs[k & 1u][x][2 * rr - 1] = r.b[j];
                 }
             }
+            if (p < 3 * T) As[k & 1u][p % 3][p / 3] = r.a;
+            if (p < 2 * T) Ys[k & 3u][p & 1u][p / 2] = r.y;
+        };
+        const double2 third = make_double2(1.0 / 3.0, 0x1.5555555555555p-56);  // 1/3 - RN(1/3) = RN(1/3) 2^-54
+        const uint32_t w = wave - 1;
+        auto produce = [&](uint32_t k) {  // terms of t0 16w .. 16w + 15 of round k
+            if (w >= G) return;
+            const uint32_t buf = k & 1u;
+            const double A0 = As[buf][0][16 * w + l16], A1 = As[buf][1][16 * w + l16], A2 = As[buf][2][16 * w + l16];
+            double b[2][3][4];
+            auto read = [&](double (&r)[3][4], uint32_t s) {  // steps s .. s + 3
+#pragma unroll
+                for (uint32_t c = 0; c < 3; c++) {
+                    if (ONE) {
+                        const double2 *q = reinterpret_cast<const double2 *>(&Bs[buf][c][2 * (lane + s)]);
+                        const double2 u = q[0], v = q[2];
+                        r[c][0] = u.x, r[c][1] = u.y, r[c][2] = v.x, r[c][3] = v.y;
+                    } else {
+#pragma unroll
+                        for (uint32_t j = 0; j < 4; j++) r[c][j] = Bs[buf][c][(s + j) * rs + lane];
+                    }
+                }
+            };
+            read(b[0], 16 * w);
+            gk_for<4>([&](auto mc) {
+                constexpr int m = decltype(mc)::value;
+                if constexpr (m < 3) read(b[(m + 1) & 1], 16 * w + 4 * m + 4);
+                double pr[4], x[4];
+                gk_for<4>([&](auto jc) {
+                    constexpr int j = decltype(jc)::value;
+                    double q = row_lane<4 * m + j>(A0) * b[m & 1][0][j];
+                    q = q + row_lane<4 * m + j>(A1) * b[m & 1][1][j];
+                    pr[j] = q + row_lane<4 * m + j>(A2) * b[m & 1][2][j];
+                });
+#pragma unroll
+                for (uint32_t j = 0; j < 4; j++) x[j] = div_by(pr[j], third);
+                float least = 1.0f;
+                track_min(least, pr[0], pr[1]);
+                track_min(least, pr[2], pr[3]);
+                if (__ballot(!(least > GK_TINY_HI))) {
+#pragma unroll
+                    for (uint32_t j = 0; j < 4; j++) x[j] = pr[j] / 3.0;
+                }
+                Xs[buf][8 * w + 2 * m][lane] = make_double2(x[0], x[1]);
+                Xs[buf][8 * w + 2 * m + 1][lane] = make_double2(x[2], x[3]);
+            });
+        };
+        Regs r0{}, r1{};
+        fetch(r0);
+        if (nst > 1) fetch(r1);
+        stash(r0, 0);
+        if (nst > 2) fetch(r0);
+        __syncthreads();
+        // while round k - 1 is summed: form round k, stage round k + 1, load round k + 3
+        auto round = [&](Regs &r, uint32_t k) {
+            if (k < nst) produce(k);
+            if (k + 1 < nst) stash(r, k + 1);
+            if (k + 3 < nst) fetch(r);
             __syncthreads();
-            buf ^= 1;
+        };
+        for (uint32_t k = 0; k <= nst; k += 2) {
+            round(r1, k);
+            if (k + 1 <= nst) round(r0, k + 1);
+        }
+        return;
+    }
+    const uint32_t it = tile * 64 + lane;
+    if (it >= a.leff) return;
+    if (a.segm) {
+        a.segm[(((uint64_t)blk * a.n_seg + iseg) * np + pair) * a.leff + it] = JJ;
+        return;
+    }
+    double *o = a.out + blk * a.out_stride + (uint64_t)it * a.narr;
+    const double v = iseg ? o[pair] : 0.0;
+    o[pair] = v + (JJ - v) / (double)(iseg + 1);  // :230-237
+    if (it == 0 && pair == 0)  // the integrals start from zero
+        for (uint32_t k = np; k < a.narr; k++) o[k] = 0.0;
+}
+
+// The same chains for launches that fill the chip, t0 stride 1: one wavefront
+// = 64 lags of CH pairs (ja, jb0 ..) or, with one current, CH x 64 lags, CH
+// running means per lane that share Ja and 1/cont.  What bounds it is the
+// FP64 issue: 12 operations per mean and t0 and 5 / CH broadcast moves; the
+// LDS port is next (3 rows of 8 bytes per mean and t0: 12 of 16 clocks).  A
+// stage of 16 t0 goes through one LDS buffer: a wavefront's LDS operations
+// stay in order, so the next stage's values, loaded to registers while this
+// one is summed, are stored after its last read.  VALU busy 85% on 20,000
+// lags x 60,000 t0 x 8 blocks, 2 currents; 32 such blocks 95 ms per call
+// with its 72 MB copied to the host (186 ms with one thread per lag).
+template <int NCUR, int CH>
+__global__ __launch_bounds__(64, 3) void gk_dense_kernel(const GkArgs a) {
+    constexpr bool LAGS = NCUR == 1;                     // the CH means are lags 64 apart
+    constexpr uint32_t T = 16, CB = LAGS ? 1 : CH;       // columns of Jb
+    constexpr uint32_t ROWS = 64 * (LAGS ? CH : 1) + T - 1, PL = gk_plane(2 * ROWS), NB = 3 * CB;
+    constexpr uint32_t PF = (NB * ROWS + 63) / 64;
+    constexpr uint32_t NJB = LAGS ? 1 : (NCUR + CH - 1) / CH;  // groups of CH columns
+    __shared__ __align__(16) double Bs[NB][PL];
+    const uint32_t lane = threadIdx.x, l16 = lane & 15u;
+    constexpr uint32_t W = 64 * (LAGS ? CH : 1);
+    const uint32_t ntile = (a.leff + W - 1) / W;
+    uint32_t z = blockIdx.x;
+    const uint32_t tile = z % ntile;
+    z /= ntile;
+    const uint32_t jb0 = z % NJB * CH, ja = z / NJB;
+    const uint32_t iseg = a.seg0 + blockIdx.y, blk = blockIdx.z;
+    const uint32_t seg = a.bl.n[blk] / a.n_seg, n0 = seg;  // stride 1: every t0 of the segment
+    const uint64_t ra = a.bl.primo[blk] + (uint64_t)seg * iseg, rb = ra + (uint64_t)tile * W, last = a.nrows - 1;
+    // columns past the last current repeat it (their means are not stored)
+    uint32_t cb[CB];
+#pragma unroll
+    for (uint32_t c = 0; c < CB; c++) cb[c] = a.idx[min(jb0 + c, (uint32_t)NCUR - 1)];
+    const double *pb[PF], *lb[PF];
+#pragma unroll
+    for (uint32_t j = 0; j < PF; j++) {
+        const uint32_t e = lane + 64 * j, rr = e / NB, x = e - NB * rr;
+        uint32_t col = cb[0] + x;
+#pragma unroll
+        for (uint32_t c = 1; c < CB; c++) col = x >= 3 * c ? cb[c] + x - 3 * c : col;
+        pb[j] = a.data + (rb + rr) * a.ncols + col;
+        lb[j] = a.data + last * a.ncols + col;
+    }
+    const double *pa = a.data + (ra + l16) * a.ncols + a.idx[ja], *la = a.data + last * a.ncols + a.idx[ja];
+    const double2 *py = a.rec + l16, *ly = a.rec + last;
+    const uint64_t step = (uint64_t)T * a.ncols;
+    struct Lane {
+        double a[3];
+        double2 y;
+    };
+    double FB[PF];
+    auto fetch = [&](Lane &f) {
+#pragma unroll
+        for (uint32_t j = 0; j < PF; j++) {
+            FB[j] = *(pb[j] < lb[j] ? pb[j] : lb[j]);
+            pb[j] += step;
+        }
+        const double *q = pa < la ? pa : la;
+        f.a[0] = q[0], f.a[1] = q[1], f.a[2] = q[2];
+        pa += step;
+        f.y = *(py < ly ? py : ly);
+        py += T;
+    };
+    auto stash = [&]() {
+#pragma unroll
+        for (uint32_t j = 0; j < PF; j++) {
+            const uint32_t e = lane + 64 * j, rr = e / NB, x = e - NB * rr;
+            if (rr < ROWS) {
+                Bs[x][2 * rr] = FB[j];
+                if (rr) Bs[x][2 * rr - 1] = FB[j];
+            }
+        }
+    };
+    const double2 third = make_double2(1.0 / 3.0, 0x1.5555555555555p-56);
+    double JJ[CH];
+#pragma unroll
+    for (int c = 0; c < CH; c++) JJ[c] = 0.0;
+    const uint32_t nst = (n0 + T - 1) / T;
+    auto rows = [&](int c, int x, uint32_t s) {  // of steps s, s + 1 (s even) of mean c, component x
+        return *reinterpret_cast<const double2 *>(&Bs[LAGS ? x : 3 * c + x][2 * (lane + (LAGS ? 64 * c : 0) + s)]);
+    };
+    auto stage = [&](uint32_t k, const Lane &f) {
+        const uint32_t c0 = k * T, cnt = min(T, n0 - c0);
+        double J0[CH];
+        float dmin = 1.0f;
+        bool bad = cnt < T;
+#pragma unroll
+        for (int c = 0; c < CH; c++) J0[c] = JJ[c];
+        if (!bad) {
+            gk_for<8>([&](auto ic) {
+                constexpr int i = decltype(ic)::value;
+                double2 b[CH][3];
+#pragma unroll
+                for (int c = 0; c < CH; c++)
+#pragma unroll
+                    for (int x = 0; x < 3; x++) b[c][x] = rows(c, x, 2 * i);
+                double dl[CH];
+                gk_for<2>([&](auto hc) {
+                    constexpr int h = decltype(hc)::value, j = 2 * i + h;
+                    const double a0 = row_lane<j>(f.a[0]), a1 = row_lane<j>(f.a[1]), a2 = row_lane<j>(f.a[2]);
+                    const double2 y = make_double2(row_lane<j>(f.y.x), row_lane<j>(f.y.y));
+#pragma unroll
+                    for (int c = 0; c < CH; c++) {
+                        double q = a0 * (h ? b[c][0].y : b[c][0].x);
+                        q = q + a1 * (h ? b[c][1].y : b[c][1].x);
+                        q = q + a2 * (h ? b[c][2].y : b[c][2].x);
+                        const double d = div_by(q, third) - JJ[c];
+                        if constexpr (h == 1) track_min(dmin, dl[c], d);
+                        dl[c] = d;
+                        JJ[c] = JJ[c] + div_by(d, y);
+                    }
+                });
+            });
+            bad = !(dmin > GK_TINY_HI);
+#pragma unroll
+            for (int c = 0; c < CH; c++) bad = bad || !(fabs(JJ[c]) < 0x1p1000);
+        }
+        if (__ballot(bad)) {
+#pragma unroll
+            for (int c = 0; c < CH; c++) JJ[c] = J0[c];
+            for (uint32_t s = 0; s < cnt; s++) {
+                double A[3];
+#pragma unroll
+                for (int x = 0; x < 3; x++) A[x] = __shfl(f.a[x], (int)s);
+#pragma unroll
+                for (int c = 0; c < CH; c++) {
+                    double q[3];
+#pragma unroll
+                    for (int x = 0; x < 3; x++) {
+                        const double2 u = rows(c, x, s & ~1u);
+                        q[x] = A[x] * (s & 1 ? u.y : u.x);
+                    }
+                    const double d = ((q[0] + q[1]) + q[2]) / 3.0 - JJ[c];
+                    JJ[c] = JJ[c] + d / (double)(c0 + s + 1);
+                }
+            }
+        }
+    };
+    Lane f0{}, f1{};
+    if (nst) fetch(f0);
+    for (uint32_t k = 0; k < nst; k += 2) {
+        stash();
+        if (k + 1 < nst) fetch(f1);
+        stage(k, f0);
+        if (k + 1 < nst) {
+            stash();
+            if (k + 2 < nst) fetch(f0);
+            stage(k + 1, f1);
         }
     }
-    if (t < ncorr) mean_lds[t] = m;
+    const uint32_t np = a.ncur * a.ncur;
+#pragma unroll
+    for (int c = 0; c < CH; c++) {
+        const uint32_t it = tile * W + lane + (LAGS ? 64 * c : 0), pair = LAGS ? 0 : ja * NCUR + jb0 + c;
+        if (it >= a.leff || (!LAGS && jb0 + c >= NCUR)) continue;
+        if (a.segm) {
+            a.segm[(((uint64_t)blk * a.n_seg + iseg) * np + pair) * a.leff + it] = JJ[c];
+            continue;
+        }
+        double *o = a.out + blk * a.out_stride + (uint64_t)it * a.narr;
+        const double v = iseg ? o[pair] : 0.0;
+        o[pair] = v + (JJ[c] - v) / (double)(iseg + 1);  // :230-237
+        if (it == 0 && pair == 0)
+            for (uint32_t k = np; k < a.narr; k++) o[k] = 0.0;
+    }
+}
+
+// The running mean over the segments (:230-237) of the segment means.
+__global__ __launch_bounds__(256) void gk_segments_kernel(const GkArgs a) {
+    const uint32_t np = a.ncur * a.ncur, blk = blockIdx.y;
+    const uint32_t w = blockIdx.x * blockDim.x + threadIdx.x;
+    if (w >= np * a.leff) return;
+    const uint32_t pair = w / a.leff, it = w - pair * a.leff;
+    const double *m = a.segm + ((uint64_t)blk * a.n_seg * np + pair) * a.leff + it;
+    double v = 0.0;
+    for (uint32_t k = 0; k < a.n_seg; k++) v = v + (m[(uint64_t)k * np * a.leff] - v) / (double)(k + 1);
+    double *o = a.out + blk * a.out_stride + (uint64_t)it * a.narr;
+    o[pair] = v;
+    if (w == 0)
+        for (uint32_t k = np; k < a.narr; k++) o[k] = 0.0;
+}
+
+// The serial scans over lags below take the reference's order in wave 0 of
+// one workgroup per block, a lane per column, NC columns.  Waves 1 to 7 load a
+// tile of lags to registers while the tile before it is scanned, and prepare
+// its terms in LDS (two buffers, one barrier per tile), so that the scan
+// reads one LDS entry per lag, a batch ahead, and does only the operations
+// that depend on the lag before.
+constexpr uint32_t GK_SCAN = 512, GK_LOAD = GK_SCAN - 64;
+constexpr uint32_t gk_scan_tile(uint32_t nc) { return 768 / nc / 16 * 16; }  // lags
+constexpr uint32_t gk_scan_regs(uint32_t nc) { return ((gk_scan_tile(nc) + 1) * nc + GK_LOAD - 1) / GK_LOAD; }
+
+// Loader thread t's values C(it0 + e / NC)[e % NC], e = t + GK_LOAD j, of a
+// tile of n lags (clamped past the end).
+template <uint32_t NC>
+struct GkTile {
+    double v[gk_scan_regs(NC)];
+    __device__ __forceinline__ void load(const double *out, uint32_t narr, uint32_t it0, uint32_t n, uint32_t t) {
+#pragma unroll
+        for (uint32_t j = 0; j < gk_scan_regs(NC); j++) {
+            const uint32_t e = min(t + GK_LOAD * j, n * NC - 1);
+            v[j] = out[(uint64_t)(it0 + e / NC) * narr + e % NC];
+        }
+    }
+};
+
+// :259-277 the mean of C over lags [start_mean, leff) as the running mean
+// m += (C - m)/c, dividing through 1/c (div_by; a tile whose differences
+// leave its range takes true divisions), then subtracted from every lag.
+// 1,000 of 5,000 lags, 2 currents: 42 us (77 us with true divisions).
+template <uint32_t NC>
+__global__ __launch_bounds__(GK_SCAN) void gk_mean_kernel(double *__restrict__ out, uint32_t leff,
+                                                          uint32_t start_mean, uint64_t stride,
+                                                          const double2 *__restrict__ rec) {
+    constexpr uint32_t narr = 3 * NC + 2, TL = gk_scan_tile(NC), B = 8;
+    __shared__ __align__(16) double2 ys[2][TL + 2 * B];
+    __shared__ double cs[2][(TL + 2 * B) * NC];
+    __shared__ double means[NC];
+    out += blockIdx.y * stride;
+    const uint32_t t = threadIdx.x, nl = start_mean < leff ? leff - start_mean : 0, ntile = (nl + TL - 1) / TL;
+    double m = 0.0;
+    GkTile<NC> r;
+    double2 yr[2];
+    static_assert(TL <= 2 * GK_LOAD, "two 1/c per loader thread");
+    auto load = [&](uint32_t i) {
+        const uint32_t n = min(TL, nl - i * TL);
+        r.load(out, narr, start_mean + i * TL, n, t - 64);
+#pragma unroll
+        for (uint32_t j = 0; j < 2; j++) yr[j] = rec[i * TL + min(t - 64 + GK_LOAD * j, n - 1)];
+    };
+    if (t >= 64 && ntile) load(0);
+    for (uint32_t i = 0; i <= ntile; i++) {  // tile i is stored, tile i - 1 scanned
+        if (t >= 64 && i < ntile) {
+            const uint32_t n = min(TL, nl - i * TL);
+#pragma unroll
+            for (uint32_t j = 0; j < gk_scan_regs(NC); j++)
+                if (t - 64 + GK_LOAD * j < n * NC) cs[i & 1u][t - 64 + GK_LOAD * j] = r.v[j];
+#pragma unroll
+            for (uint32_t j = 0; j < 2; j++)
+                if (t - 64 + GK_LOAD * j < n) ys[i & 1u][t - 64 + GK_LOAD * j] = yr[j];
+            if (i + 1 < ntile) load(i + 1);
+        } else if (t < 64 && i > 0) {  // the whole wavefront, for the ballot; lanes past NC repeat the last column
+            const uint32_t c0 = (i - 1) * TL, n = min(TL, nl - c0);
+            const double *c = cs[(i - 1) & 1u] + min(t, NC - 1);
+            const double2 *y = ys[(i - 1) & 1u];
+            const double m0 = m;
+            double dmin = 1.0, v[B], vn[B];
+            double2 w[B], wn[B];
+            auto batch = [&](const double (&cv)[B], const double2 (&cw)[B], double (&nv)[B], double2 (&nw)[B],
+                             uint32_t k0) {
+#pragma unroll
+                for (uint32_t j = 0; j < B; j++) {
+                    nv[j] = c[(k0 + B + j) * NC];
+                    nw[j] = y[k0 + B + j];
+                    const double d = cv[j] - m;
+                    dmin = fmin(dmin, fabs(d));
+                    m = m + div_by(d, cw[j]);
+                }
+            };
+#pragma unroll
+            for (uint32_t j = 0; j < B; j++) {
+                v[j] = c[j * NC];
+                w[j] = y[j];
+            }
+            uint32_t k = 0;
+            for (; k + 2 * B <= n; k += 2 * B) {
+                batch(v, w, vn, wn, k);
+                batch(vn, wn, v, w, k + B);
+            }
+            uint32_t k1 = k;
+            if (__ballot(!(dmin > GK_TINY) || !(fabs(m) < 0x1p1000))) {
+                m = m0;
+                k1 = 0;
+            }
+            for (; k1 < n; k1++) {
+                const double d = c[k1 * NC] - m;
+                m = m + d / (double)(c0 + k1 + 1);
+            }
+        }
+        __syncthreads();
+    }
+    if (t < NC) means[t] = m;
     __syncthreads();
-    for (uint32_t e = t; e < leff * ncorr; e += blockDim.x) {
-        const uint32_t it = e / ncorr, jj = e - it * ncorr;
-        double *v = out + (uint64_t)it * narr + jj;
-        *v = *v - mean_lds[jj];
+#pragma unroll 8
+    for (uint32_t e = t; e < leff * NC; e += GK_SCAN) {
+        double *v = out + (uint64_t)(e / NC) * narr + e % NC;
+        *v = *v - means[e % NC];
     }
 }
 
 // :279-288 trapezoid I and Einstein E running integrals, per correlation
 // column: I(it) = (I(it-1) + C(it-1)/2) + C(it)/2, E(it) = (E(it-1) +
 // C(it-1) it/2) + C(it) it/2, with I(0) = E(0) = 0 as left by the lag loop.
-// The scan lanes write I and E of a tile into LDS; waves 1-3 store the
-// previous tile's results to HBM (coalesced) while they load the next tile's
-// C values, so the serial chain never waits on a global store.
-__global__ __launch_bounds__(256) void gk_integral_kernel(double *__restrict__ out, uint32_t narr, uint32_t ncorr,
-                                                          uint32_t leff, uint64_t stride, uint32_t tl) {
-    extern __shared__ double lds[];  // C in [2][tl][ncorr], then (I, E) out [2][tl][2 ncorr]
+// A lane scans one of the 2 NC sums; its two terms of a lag are one 16-byte
+// LDS entry.  5,000 lags, 2 currents: 80 us (210 us with I and E in one lane
+// and their terms formed by it).
+template <uint32_t NC>
+__global__ __launch_bounds__(GK_SCAN) void gk_integral_kernel(double *__restrict__ out, uint32_t leff,
+                                                              uint64_t stride) {
+    constexpr uint32_t narr = 3 * NC + 2, TL = gk_scan_tile(NC), NS = 2 * NC, B = 8;
+    __shared__ __align__(16) double2 terms[2][(TL + 2 * B) * NS];
+    __shared__ double res[2][TL * NS];
     if (leff < 2) return;
     out += blockIdx.y * stride;
-    double *cin = lds, *res = lds + 2 * tl * ncorr;
-    const uint32_t t = threadIdx.x, nres = 2 * ncorr;
-    double I = 0.0, E = 0.0, cprev = 0.0;
-    if (t < ncorr) {
-        I = out[ncorr + 2 * t];
-        E = out[ncorr + 2 * t + 1];
-        cprev = out[t];
-    }
-    const uint32_t ntile = (leff - 1 + tl - 1) / tl;  // tiles of lags 1 .. leff-1
-    if (t >= 64) gk_load_tile(cin, out, narr, ncorr, 1, leff, tl, t - 64, blockDim.x - 64);
-    __syncthreads();
-    for (uint32_t i = 0; i <= ntile; i++) {
-        const uint32_t buf = i & 1u;
+    const uint32_t t = threadIdx.x;
+    const uint32_t ntile = (leff - 1 + TL - 1) / TL;  // tiles of lags 1 .. leff-1
+    GkTile<NC> r;
+    // tile i reads C of one lag more, it0 - 1: C(it)'s terms belong to lag it
+    // (second) and to lag it + 1 (first)
+    auto load = [&](uint32_t i) { r.load(out, narr, i * TL, min(TL, leff - 1 - i * TL) + 1, t - 64); };
+    double s = t < NS ? out[NC + t] : 0.0;
+    if (t >= 64) load(0);
+    for (uint32_t i = 0; i <= ntile + 1; i++) {  // tile i is stored, tile i - 1 scanned, tile i - 2 written out
         if (t >= 64) {
-            if (i + 1 < ntile)
-                gk_load_tile(cin + (buf ^ 1u) * tl * ncorr, out, narr, ncorr, 1 + (i + 1) * tl, leff, tl, t - 64,
-                             blockDim.x - 64);
-            if (i >= 1) {  // results of tile i - 1
-                const uint32_t it0 = 1 + (i - 1) * tl, n = min(tl, leff - it0);
-                const double *src = res + (buf ^ 1u) * tl * nres;
-                for (uint32_t e = t - 64; e < n * nres; e += blockDim.x - 64) {
-                    const uint32_t k = e / nres, jj = e - k * nres;
-                    out[(uint64_t)(it0 + k) * narr + ncorr + jj] = src[e];
+            if (i < ntile) {
+                const uint32_t n = min(TL, leff - 1 - i * TL);
+                double2 *d = terms[i & 1u];
+#pragma unroll
+                for (uint32_t j = 0; j < gk_scan_regs(NC); j++) {
+                    const uint32_t e = t - 64 + GK_LOAD * j, k = e / NC, jj = e % NC, it = i * TL + k;
+                    const double v = r.v[j];
+                    if (k > 0 && k <= n) {
+                        d[(k - 1) * NS + 2 * jj].y = v / 2.0;
+                        d[(k - 1) * NS + 2 * jj + 1].y = v * (double)it / 2.0;
+                    }
+                    if (k < n) {
+                        d[k * NS + 2 * jj].x = v / 2.0;
+                        d[k * NS + 2 * jj + 1].x = v * (double)(it + 1) / 2.0;
+                    }
                 }
+                if (i + 1 < ntile) load(i + 1);
             }
-        } else if (t < ncorr && i < ntile) {
-            // batches of 16 lags: 16 LDS reads, one wait, the serial chain in
-            // registers, 16 paired LDS writes (a read-use-write per lag would
-            // wait out the LDS latency at every lag)
-            const uint32_t it0 = 1 + i * tl, n = min(tl, leff - it0);
-            const double *col = cin + buf * tl * ncorr + t;
-            double *dst = res + buf * tl * nres + 2 * t;
-            constexpr uint32_t B = 16;
-            auto step = [&](double v, uint32_t k, double &Io, double &Eo) {
-                const double dit = (double)(it0 + k);
-                const double In = I + cprev / 2.0;
-                I = In + v / 2.0;
-                const double En = E + cprev * dit / 2.0;
-                E = En + v * dit / 2.0;
-                cprev = v;
-                Io = I;
-                Eo = E;
-            };
-            uint32_t k0 = 0;
-            for (; k0 + B <= n; k0 += B) {
-                double v[B], Ib[B], Eb[B];
-#pragma unroll
-                for (uint32_t j = 0; j < B; j++) v[j] = col[(k0 + j) * ncorr];
-#pragma unroll
-                for (uint32_t j = 0; j < B; j++) step(v[j], k0 + j, Ib[j], Eb[j]);
+            if (i >= 2) {
+                const uint32_t it0 = 1 + (i - 2) * TL, n = min(TL, leff - it0);
+                const double *src = res[i & 1u];
+                for (uint32_t e = t - 64; e < n * NS; e += GK_LOAD)
+                    out[(uint64_t)(it0 + e / NS) * narr + NC + e % NS] = src[e];
+            }
+        } else if (t < NS && i > 0 && i <= ntile) {
+            const uint32_t n = min(TL, leff - 1 - (i - 1) * TL);
+            const double2 *src = terms[(i - 1) & 1u] + t;
+            double *dst = res[(i - 1) & 1u] + t;
+            double2 v[B], w[B];
+            auto batch = [&](const double2 (&c)[B], double2 (&nx)[B], uint32_t k0) {
 #pragma unroll
                 for (uint32_t j = 0; j < B; j++) {
-                    dst[(k0 + j) * nres] = Ib[j];
-                    dst[(k0 + j) * nres + 1] = Eb[j];
+                    nx[j] = src[(k0 + B + j) * NS];
+                    s = (s + c[j].x) + c[j].y;
+                    dst[(k0 + j) * NS] = s;
                 }
+            };
+#pragma unroll
+            for (uint32_t j = 0; j < B; j++) v[j] = src[j * NS];
+            uint32_t k = 0;
+            for (; k + 2 * B <= n; k += 2 * B) {
+                batch(v, w, k);
+                batch(w, v, k + B);
             }
-            for (; k0 < n; k0++) {  // tail of the last tile
-                double Io, Eo;
-                step(col[k0 * ncorr], k0, Io, Eo);
-                dst[k0 * nres] = Io;
-                dst[k0 * nres + 1] = Eo;
+            for (; k < n; k++) {  // tail of the last tile
+                const double2 c = src[k * NS];
+                s = (s + c.x) + c.y;
+                dst[k * NS] = s;
             }
         }
         __syncthreads();
@@ -512,7 +970,7 @@ static void gk_schur_launch(double *d, uint32_t narr, uint32_t ncur, uint32_t le
 }
 
 void gk_epilogue(double *d, uint32_t narr, uint32_t ncur, uint32_t leff, int subtract_mean, uint32_t start_mean,
-                 hipStream_t s, uint32_t nblocks, uint64_t stride, bool serial_scans) {
+                 hipStream_t s, uint32_t nblocks, uint64_t stride, bool serial_scans, const double2 *rec) {
     const uint32_t ncorr = ncur * ncur;
     if (!serial_scans) {
         if (subtract_mean) {
@@ -540,20 +998,52 @@ void gk_epilogue(double *d, uint32_t narr, uint32_t ncur, uint32_t leff, int sub
         gk_schur_launch(d, narr, ncur, leff, s, nblocks, stride);
         return;
     }
-    // lag tile of the scans: two buffers of tl x ncorr doubles, <= 64 KiB
-    const uint32_t tl = std::max(16u, 4096u / ncorr);
-    const size_t lds = (2 * (size_t)tl * ncorr + ncorr) * sizeof(double);
-    if (subtract_mean) {
-        hipLaunchKernelGGL(gk_mean_kernel, dim3(1, nblocks), dim3(256), lds, s, d, narr, ncorr, leff, start_mean,
-                           stride, tl);
-        ANL_HIP(hipGetLastError());
+    switch (ncorr) {
+#define ANL_GK_SCANS(NC)                                                                                            \
+    case NC:                                                                                                        \
+        if (subtract_mean)                                                                                          \
+            hipLaunchKernelGGL(gk_mean_kernel<NC>, dim3(1, nblocks), dim3(GK_SCAN), 0, s, d, leff, start_mean, stride, \
+                               rec);                                                                                \
+        hipLaunchKernelGGL(gk_integral_kernel<NC>, dim3(1, nblocks), dim3(GK_SCAN), 0, s, d, leff, stride);          \
+        break;
+        ANL_GK_SCANS(1)
+        ANL_GK_SCANS(4)
+        ANL_GK_SCANS(9)
+        ANL_GK_SCANS(16)
+#undef ANL_GK_SCANS
+        default: fail(ANL_ERR_ARG, "between 1 and 4 currents are supported");
     }
-    // integral: C tiles and (I, E) tiles, both double-buffered, <= 48 KiB
-    const uint32_t tli = std::max(16u, 1024u / ncorr);
-    const size_t ldsi = 6 * (size_t)tli * ncorr * sizeof(double);
-    hipLaunchKernelGGL(gk_integral_kernel, dim3(1, nblocks), dim3(256), ldsi, s, d, narr, ncorr, leff, stride, tli);
     ANL_HIP(hipGetLastError());
     gk_schur_launch(d, narr, ncur, leff, s, nblocks, stride);
+}
+
+size_t gk_fp64_scratch_bytes(uint32_t ncur, uint32_t leff, uint32_t n_seg, uint32_t nblocks) {
+    return n_seg > 1 ? (size_t)std::min(GK_MAXB, nblocks) * n_seg * ncur * ncur * leff * sizeof(double) : 0;
+}
+
+void gk_reciprocals(double2 *rec, uint64_t n, hipStream_t s) {
+    hipLaunchKernelGGL(gk_reciprocal_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, rec, n);
+    ANL_HIP(hipGetLastError());
+}
+
+// The segments of a block run side by side into scratch of the series and
+// are folded afterwards, when the scratch is there or can be had; else (more
+// scratch than the cap, or a stream under capture, where nothing can be
+// allocated) one launch per segment folds into the output.
+constexpr size_t GK_SEG_BYTES = 1ull << 30;
+
+// Wavefronts of 64 means from which a stride 1 launch takes gk_dense_kernel:
+// gk_chain_kernel's time for 20,000 t0 grows by 0.48 ms per 256 (one
+// per CU), the dense kernel's by 0.2-0.3 ms from 1.4 ms on (2.0 against
+// 2.7 ms at 1,024 and 2 currents, 2.9 against 2.6 ms at 2,048 and 4).
+constexpr uint64_t GK_DENSE_CHAINS = 1792;
+static bool gk_can_allocate(hipStream_t st) {
+    hipStreamCaptureStatus c = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &c) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    return c == hipStreamCaptureStatusNone;
 }
 
 void gk_fp64_enqueue_blocks(anl_series *s, const uint32_t *idx_j, uint32_t ncur, uint32_t skip, uint32_t leff,
@@ -561,10 +1051,16 @@ void gk_fp64_enqueue_blocks(anl_series *s, const uint32_t *idx_j, uint32_t ncur,
                             hipStream_t st) {
     const uint32_t narr = 3 * ncur * ncur + 2;
     const uint64_t stride = (uint64_t)leff * narr;
+    const size_t need = gk_fp64_scratch_bytes(ncur, leff, n_seg, nblocks);
+    double *segm = nullptr;
+    if (need && need <= GK_SEG_BYTES && n_seg <= 65535 && (need <= s->work_cap || gk_can_allocate(st)))
+        segm = (double *)series_workspace(s, need);
     for (uint32_t b0 = 0; b0 < nblocks; b0 += GK_MAXB) {
         const uint32_t nb = std::min(GK_MAXB, nblocks - b0);
         GkArgs a{};
         a.data = s->data;
+        a.rec = s->rec;
+        a.nrows = s->nrows;
         a.ncols = s->ncols;
         a.ncur = ncur;
         for (uint32_t c = 0; c < ncur; c++) a.idx[c] = idx_j[c];
@@ -574,18 +1070,34 @@ void gk_fp64_enqueue_blocks(anl_series *s, const uint32_t *idx_j, uint32_t ncur,
         a.narr = narr;
         a.out_stride = stride;
         a.out = d + b0 * stride;
+        a.segm = segm;
         for (uint32_t b = 0; b < nb; b++) {
             a.bl.primo[b] = primo[b0 + b];
             a.bl.n[b] = n[b0 + b];
         }
-        dim3 grid((leff + 255) / 256, nb);
-        switch (ncur) {
-            case 1: hipLaunchKernelGGL(gk_lag_kernel<1>, grid, dim3(256), 0, st, a); break;
-            case 2: hipLaunchKernelGGL(gk_lag_kernel<2>, grid, dim3(256), 0, st, a); break;
-            case 3: hipLaunchKernelGGL(gk_lag_kernel<3>, grid, dim3(256), 0, st, a); break;
-            default: hipLaunchKernelGGL(gk_lag_kernel<4>, grid, dim3(256), 0, st, a); break;
+        const dim3 grid((leff + 63) / 64 * ncur * ncur, segm ? n_seg : 1, nb);
+        for (uint32_t k = 0; k < (segm ? 1 : n_seg); k++) {
+            a.seg0 = k;
+            const uint64_t chains = (uint64_t)grid.x * grid.y * grid.z;
+            if (skip == 1 && chains > GK_DENSE_CHAINS) {
+                const uint32_t nt64 = (leff + 63) / 64, nt128 = (leff + 127) / 128;
+                switch (ncur) {
+#define ANL_GK_DENSE(N, C, X) hipLaunchKernelGGL((gk_dense_kernel<N, C>), dim3(X, grid.y, grid.z), dim3(64), 0, st, a)
+                    case 1: ANL_GK_DENSE(1, 2, nt128); break;
+                    case 2: ANL_GK_DENSE(2, 2, nt64 * 2); break;
+                    case 3: ANL_GK_DENSE(3, 3, nt64 * 3); break;
+                    default: ANL_GK_DENSE(4, 2, nt64 * 8); break;
+#undef ANL_GK_DENSE
+                }
+            } else if (skip == 1) hipLaunchKernelGGL((gk_chain_kernel<48, 1>), grid, dim3(256), 0, st, a);
+            else if (skip <= 8) hipLaunchKernelGGL((gk_chain_kernel<32, 8>), grid, dim3(256), 0, st, a);
+            else hipLaunchKernelGGL((gk_chain_kernel<16, 64>), grid, dim3(256), 0, st, a);
+            ANL_HIP(hipGetLastError());
         }
-        ANL_HIP(hipGetLastError());
+        if (segm) {
+            hipLaunchKernelGGL(gk_segments_kernel, dim3((ncur * ncur * leff + 255) / 256, nb), dim3(256), 0, st, a);
+            ANL_HIP(hipGetLastError());
+        }
     }
 }
 
@@ -636,7 +1148,8 @@ int anl_gk_calculate_blocks_async(anl_series *s, const uint32_t *idx_j, uint32_t
         if (form == ANL_GK_MFMA) gk_mfma_enqueue_blocks(s, idx_j, ncur, skip, leff, n_seg, primo, n, nblocks, out_dev, st);
         else gk_fp64_enqueue_blocks(s, idx_j, ncur, skip, leff, n_seg, primo, n, nblocks, out_dev, st);
         // the FP64 form keeps the reference's serial scans (bit-identical results)
-        gk_epilogue(out_dev, narr, ncur, leff, subtract_mean, start_mean, st, nblocks, stride, form == ANL_GK_FP64);
+        gk_epilogue(out_dev, narr, ncur, leff, subtract_mean, start_mean, st, nblocks, stride, form == ANL_GK_FP64,
+                    s->rec);
         if (mean_dev) mediavar_blocks(nullptr, out_dev, nullptr, nblocks, stride, mean_dev, var_dev, st);
     });
 }
@@ -666,10 +1179,13 @@ static int gk_calculate_host(anl_series *s, const uint32_t *idx_j, uint32_t ncur
         if (leff == 0) return;
         ensure_device();
         const size_t bytes = (size_t)leff * (3 * ncur * ncur + 2) * sizeof(double);
-        const size_t front = form == ANL_GK_MFMA ? gk_mfma_scratch_bytes(s, ncur, leff, n) : 0;
+        size_t front = form == ANL_GK_MFMA ? gk_mfma_scratch_bytes(s, ncur, leff, n)
+                                           : gk_fp64_scratch_bytes(ncur, leff, n_seg, 1);
+        if (form == ANL_GK_FP64 && front > GK_SEG_BYTES) front = 0;  // not used then
+        front = (front + 255) / 256 * 256;
         char *w = (char *)series_workspace(s, front + bytes);
         double *d = (double *)(w + front);
-        // the MFMA form takes its scratch from the front of the series scratch
+        // both forms take their scratch from the front of the series scratch
         int rc = anl_gk_calculate_blocks_async(s, idx_j, ncur, skip, tmax, n_seg, subtract_mean, start_mean, &primo,
                                                &n, 1, form, d, nullptr, nullptr, 0);
         if (rc != ANL_OK) throw Error{rc, anl_last_error()};

@@ -451,12 +451,17 @@ int anl_series_create(const double *data, uint64_t nrows, uint32_t ncols, anl_se
         if (!data || !out) fail(ANL_ERR_ARG, "null pointer passed to anl_series_create");
         if (nrows == 0 || ncols == 0) fail(ANL_ERR_ARG, "empty time series");
         ensure_device();
-        auto *s = new anl_series();
+        std::unique_ptr<anl_series, int (*)(anl_series *)> owner(new anl_series(), anl_series_destroy);
+        anl_series *s = owner.get();
         s->nrows = nrows;
         s->ncols = ncols;
         ANL_HIP(hipMalloc(&s->data, nrows * ncols * sizeof(double)));
         ANL_HIP(hipMemcpy(s->data, data, nrows * ncols * sizeof(double), hipMemcpyHostToDevice));
-        *out = s;
+        // a running mean over t0 counts to nrows at most
+        ANL_HIP(hipMalloc(&s->rec, nrows * sizeof(double2)));
+        gk_reciprocals(s->rec, nrows, nullptr);
+        ANL_HIP(hipStreamSynchronize(nullptr));  // calculations may run on other streams
+        *out = owner.release();
     });
 }
 
@@ -465,6 +470,7 @@ int anl_series_destroy(anl_series *s) {
         if (!s) return;
         (void)hipDeviceSynchronize();
         (void)hipFree(s->work);
+        (void)hipFree(s->rec);
         (void)hipFree(s->data);
         delete s;
     });
