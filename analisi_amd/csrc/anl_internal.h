@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -51,6 +52,35 @@ struct Cell {
     double xy, xz, yz;
 };
 
+// Device and pinned host memory of one calculation, kept for the next one of
+// the same trajectory.
+struct Scratch {
+    void *dev = nullptr, *pin = nullptr;
+    size_t dev_cap = 0, pin_cap = 0;
+};
+// The workspaces that no calculation holds: as many as calculations ran at
+// once (from several threads), at most 4, each at most SCRATCH_KEEP bytes.
+// A calculation returns its workspace when its stream has finished with it.
+constexpr size_t SCRATCH_KEEP = 64ull << 20;
+class ScratchPool {
+    std::mutex mu;
+    std::vector<Scratch> idle;
+
+   public:
+    Scratch take(size_t dev_bytes, size_t pin_bytes);
+    void give(const Scratch &s);
+    ~ScratchPool();
+};
+// A workspace for the scope; the destructor gives it back.
+struct ScratchLease {
+    ScratchPool &pool;
+    Scratch s;
+    ScratchLease(ScratchPool &p, size_t dev_bytes, size_t pin_bytes) : pool(p), s(p.take(dev_bytes, pin_bytes)) {}
+    ~ScratchLease() { pool.give(s); }
+    ScratchLease(const ScratchLease &) = delete;
+    ScratchLease &operator=(const ScratchLease &) = delete;
+};
+
 // g(r,t) screen parameters (16-bit fractional fixed point; see gofrt.hip).
 struct Screen {
     bool valid;            // preconditions hold for the whole trajectory
@@ -96,6 +126,8 @@ struct anl_traj {
     double screen_rmax = -1.0;
     uint32_t msd_tile = 16;             // lag tile of the MSD window kernel (anl_msd_set_tuning)
     uint32_t msd_waves = 4;             // its wavefronts per workgroup
+    bool msd_auto = true;               // neither was chosen: each calculation takes its own lag tile
+    anl::ScratchPool scratch;           // workspaces of the synchronous calculations
 };
 
 struct anl_series {

@@ -41,6 +41,64 @@ void ensure_device() {
     ANL_HIP(hipSetDevice(0));
 }
 
+Scratch ScratchPool::take(size_t dev_bytes, size_t pin_bytes) {
+    Scratch s;
+    {
+        std::lock_guard<std::mutex> lock(mu);
+        if (!idle.empty()) {  // the smallest that holds the calculation, else the largest, grown
+            size_t best = 0;
+            for (size_t k = 1; k < idle.size(); k++) {
+                const bool fits = idle[k].dev_cap >= dev_bytes, best_fits = idle[best].dev_cap >= dev_bytes;
+                if (fits != best_fits ? fits : fits == (idle[k].dev_cap < idle[best].dev_cap)) best = k;
+            }
+            s = idle[best];
+            idle.erase(idle.begin() + best);
+        }
+    }
+    try {
+        if (s.dev_cap < dev_bytes) {
+            (void)hipFree(s.dev);
+            s.dev = nullptr;
+            s.dev_cap = 0;
+            ANL_HIP(hipMalloc(&s.dev, dev_bytes));
+            s.dev_cap = dev_bytes;
+        }
+        if (s.pin_cap < pin_bytes) {
+            (void)hipHostFree(s.pin);
+            s.pin = nullptr;
+            s.pin_cap = 0;
+            ANL_HIP(hipHostMalloc(&s.pin, pin_bytes, hipHostMallocDefault));
+            s.pin_cap = pin_bytes;
+        }
+    } catch (...) {
+        give(s);
+        throw;
+    }
+    return s;
+}
+
+void ScratchPool::give(const Scratch &s) {
+    if (s.dev_cap + s.pin_cap <= SCRATCH_KEEP) {
+        std::lock_guard<std::mutex> lock(mu);
+        if (idle.size() < 4) {
+            try {
+                idle.push_back(s);
+                return;
+            } catch (...) {  // no memory for the list: free it
+            }
+        }
+    }
+    (void)hipFree(s.dev);
+    (void)hipHostFree(s.pin);
+}
+
+ScratchPool::~ScratchPool() {
+    for (const Scratch &s : idle) {
+        (void)hipFree(s.dev);
+        (void)hipHostFree(s.pin);
+    }
+}
+
 Cell cell_of(const double *b) {
     Cell c;
     for (int k = 0; k < 3; k++) {

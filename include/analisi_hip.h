@@ -236,21 +236,22 @@ int anl_msd_calculate_async(anl_traj *tr, uint32_t skip, uint32_t tmax, int cm_m
  * counterpart in the reference; it is for callers that cannot allocate
  * device memory (code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc).  Its scratch (block table, term counts,
- * partial sums: about 8 * leff * ceil(natoms/64) * ntypes bytes at t0
- * stride 1, ceil(natoms/256) at other strides) lives in a fixed 16 MiB
+ * partial sums: about 8 * leff * ceil(natoms/64) * ntypes bytes, at other t0
+ * strides than 1 with ceil(natoms/256) where that is over 8 MiB) lives in a fixed 16 MiB
  * device array per GPU, held until the process ends; larger calculations
  * fail with ANL_ERR_ARG before anything is launched.  The call synchronises
  * stream before returning.  Calls that overlap on one GPU share the array
  * and race. */
 int anl_msd_calculate_noalloc(anl_traj *tr, uint32_t skip, uint32_t tmax, int cm_msd, int cm_self, uint32_t n,
                               uint64_t primo, double *out_dev, void *stream);
-/* Launch shape of the MSD kernel for this trajectory: the lag tile R of the
- * t0-stride-1 kernel, which holds R frames of an atom in registers and loads
- * two frames per t0 for R updates, and its wavefronts per workgroup W; a
- * workgroup covers R * W lags of 64 atoms, streaming their frames once for
- * all of them.  (R, W) is one of (8,4) (12,4) (16,4) (24,4) (16,8) (24,8)
- * (12,12) (16,12) (8,16); default (16,4).  Lag tile 0 selects the
- * eight-lags-per-thread kernel that every other stride uses (W ignored).
+/* Launch shape of the MSD kernel for this trajectory: the lag tile R, R
+ * frames of an atom held in registers with two frames loaded per t0 for R
+ * updates, and its wavefronts per workgroup W (a workgroup covers R * W lags
+ * of 64 atoms; at t0 stride s > 1, R * W of the lags that are equal modulo
+ * s).  (R, W) is one of (8,4) (12,4) (16,4) (24,4) (16,8) (24,8) (12,12)
+ * (16,12) (8,16).  Until one is set each calculation takes its own tile by
+ * its sizes, and the shape reads as (16,4).  Lag tile 0 selects the
+ * eight-lags-per-thread kernel (W ignored).
  * All shapes with R > 0 give identical results (each (atom, lag) sum runs
  * over t0 in order with the same operations, and the workgroup sums its 64
  * atoms in slot order); tile 0 agrees with them to rounding (both within
