@@ -127,7 +127,7 @@ static void eig_sym3(const double G[3][3], double *lmin, double *lmax) {
 //  (3) |A delta| >= sqrt(lambda_min(A^T A)) |delta|, and rounding each 16-bit
 //      coordinate moves each component of q by at most 1 unit, so
 //      d <= rmax  =>  |q| <= rmax 2^16 / sqrt(lambda_min) + sqrt(3).
-static Screen make_screen(const Cell &c, bool box_const, uint32_t nt, double rmax) {
+static Screen make_screen(const Cell &c, bool box_const, uint32_t nt, double rmax, double *widths = nullptr) {
     Screen s{false, 0, "", 0.5, 0.0, 0.0, 0.0, 0.0};
     if (!box_const) {
         s.why_not = "the cell changes along the trajectory";
@@ -150,6 +150,7 @@ static Screen make_screen(const Cell &c, bool box_const, uint32_t nt, double rma
     for (int k = 0; k < 3; k++) {
         double n = std::sqrt(Ai[k][0] * Ai[k][0] + Ai[k][1] * Ai[k][1] + Ai[k][2] * Ai[k][2]);
         wmin = std::min(wmin, 1.0 / n);
+        if (widths) widths[k] = 1.0 / n;
     }
     double r = std::fabs(rmax) * (1 + 1e-9) + 1e-12;
     if (!(r < wmin * (0.5 - 4.0 / 65536.0))) {
@@ -911,6 +912,283 @@ __host__ __device__ __forceinline__ float cluster_threshold(float rho, float rma
         qn += (uint32_t)__popcll(M);                                        \
     }
 
+// g(r,t) of a cell that changes along the trajectory: the 16-bit screen with
+// the fractions of both frames taken in the cell of frame t0, the one the
+// reference's minimum image uses.  The fractions are formed as they are
+// needed, once per (workgroup, t0, j): 256 lanes share a j, so the 20 FP64
+// operations of a conversion are nothing beside the 256 distances.  The
+// arguments of make_screen, du_window and eval_candidate hold for each t0's
+// cell, whose constants come with the frame (CellScreen); a candidate near a
+// bin edge, rmin or rmax takes the reference's FP64 sequence.
+// Bound by VALU issue (65 % of the cycles; LDS 42 %): 5 instructions for a
+// pair's screen (per wavefront: 64 pairs), 6 for an append where a lane
+// passes, 35 per 64 candidates.  3,000 atoms in a tilted cell at rmax 0.31 of
+// its length (1.8e9 pairs, 14.6 % candidates): plain FP64 4.67 ms; this with
+// candidates straight to FP64 from positions in LDS 3.55 (six 8-byte gathers
+// a candidate); FP32 first 2.16; workgroups of one t0 1.76 (1,200 of two left
+// the second pass over the chip nearly empty); compares of 8 j together, the
+// queue's end as a scalar LDS address and entries taken from its top 1.43.
+// A 64 x 64 block of pairs is skipped when the boxes of its two groups of 64
+// slots are farther apart than rmax along a cell axis (in 16-bit fractions;
+// slots are in frame 0's k-d order).
+struct CellScreen {
+    double r0, r1, r2;                // 1 / cell lengths
+    uint32_t threshold;               // bound of |q|^2
+    uint32_t gap0, gap1, gap2;        // rmax in 16-bit units of each axis, plus the rounding
+    float cx, cxy, cxz, cy, cyz, cz;  // as in GofrtArgs, of this cell
+    float du_margin;
+    float pad;
+};
+struct GofrtCellArgs {
+    GofrtArgs g;
+    const CellScreen *cells;  // [F]
+};
+
+__device__ __forceinline__ uint32_t fix32(double s) {
+    return (uint32_t)(uint64_t)rint((s - floor(s)) * 4294967296.0);
+}
+// Rounded 32-bit fractions in a cell given by reciprocals: the error of s is
+// a few units of 2^-53 of |x| / L, as that of the divisions of to_fractional.
+template <bool TRI>
+__device__ __forceinline__ uint4 fractions32(const double4 &x, const double *b, const CellScreen &cs, uint32_t w) {
+    const double sc = (x.z - b[2]) * cs.r2;
+    const double sb = (x.y - b[1] - (TRI ? b[8] * sc : 0.0)) * cs.r1;
+    const double sa = (x.x - b[0] - (TRI ? b[6] * sb + b[7] * sc : 0.0)) * cs.r0;
+    return make_uint4(fix32(sa), fix32(sb), fix32(sc), w);
+}
+// {a | b << 16, c}: the 32-bit fractions rounded to 16 bits
+__device__ __forceinline__ uint2 round16(const uint4 &f) {
+    return make_uint2(((f.x + 0x8000u) >> 16) | ((f.y + 0x8000u) & 0xFFFF0000u), (f.z + 0x8000u) >> 16);
+}
+
+// The box of the wavefront's fractions: a centre and the largest offset from
+// it, per axis; lanes that are not `in` do not count.
+struct FracBox {
+    int c0, c1, c2, e0, e1, e2;
+};
+__device__ __forceinline__ FracBox frac_box(const uint2 f, bool in) {
+    const unsigned long long m = __ballot(in);
+    FracBox b{0, 0, 0, 0, 0, 0};
+    if (!m) return b;
+    const int l0 = __ffsll(m) - 1;
+    const uint32_t ra = __builtin_amdgcn_readlane((int)f.x, l0), rc = __builtin_amdgcn_readlane((int)f.y, l0);
+    int lo[3], hi[3];
+    lo[0] = hi[0] = in ? s16(f.x - ra) : 0;
+    lo[1] = hi[1] = in ? s16((f.x >> 16) - (ra >> 16)) : 0;
+    lo[2] = hi[2] = in ? s16(f.y - rc) : 0;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1)
+#pragma unroll
+        for (int k = 0; k < 3; k++) {
+            lo[k] = min(lo[k], __shfl_xor(lo[k], o));
+            hi[k] = max(hi[k], __shfl_xor(hi[k], o));
+        }
+    b.c0 = (int)(ra & 0xFFFFu) + (lo[0] + hi[0]) / 2;
+    b.c1 = (int)(ra >> 16) + (lo[1] + hi[1]) / 2;
+    b.c2 = (int)rc + (lo[2] + hi[2]) / 2;
+    b.e0 = (hi[0] - lo[0]) / 2 + 1;
+    b.e1 = (hi[1] - lo[1]) / 2 + 1;
+    b.e2 = (hi[2] - lo[2]) / 2 + 1;
+    return b;
+}
+// whether fractions of two boxes can be within gap of each other, modulo 1, on
+// one axis
+__device__ __forceinline__ bool axis_near(int ca, int ea, int cb, int eb, uint32_t gap) {
+    const int d = abs(s16((uint32_t)(ca - cb))), e = ea + eb;
+    return min(d - e, 65536 - d - e) <= (int)gap;
+}
+
+template <bool TRI>
+__global__ __launch_bounds__(WG, 4) void gofrt_cells_kernel(const GofrtCellArgs ca) {
+    constexpr int QC = SQCAP;
+    const GofrtArgs &a = ca.g;
+    extern __shared__ __align__(16) unsigned char smem[];
+    const WgId id = decode_wg(a.ntiles, a.nlag, a.nwork, a.per_xcd);
+    if (!id.valid) return;
+    const WorkItem w = a.work[id.work];
+    const BlockInfo b = a.blocks[w.block];
+    const uint32_t t = a.lag0 + id.lagi * a.every;
+    if (t >= b.leff) return;
+    uint4 *j32 = (uint4 *)smem;                       // fractions of the tile's j, .w = type | slot << 8
+    uint4 *i32 = j32 + WG;                            // and of the i
+    uint2 *jf = (uint2 *)(i32 + WG);                  // 16-bit fractions of the j
+    FracBox *jb = (FracBox *)(jf + WG);               // [WG / 64] their boxes
+    uint32_t *queue = (uint32_t *)(jb + WG / 64);     // [WG / 64][SQCAP]
+    uint32_t *requeue = queue + WG / 64 * SQCAP;      // [WG / 64][RQCAP]
+    double *thr = (double *)(requeue + WG / 64 * RQCAP);
+    int *rowch = (int *)(thr + a.nbin + 1);
+    unsigned *hist = (unsigned *)(rowch + 2 * a.nt * a.nt);
+    lds_setup_rows(a, hist, thr, rowch);
+
+    const uint32_t N = (uint32_t)a.N, tid = threadIdx.x, lane = tid & 63u;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    uint32_t *q = queue + wave * SQCAP;
+    uint32_t *rq = requeue + wave * RQCAP;
+    unsigned *sink = rq + (RQCAP - QSINK) + lane;
+    const uint32_t slot0 = id.tile * WG, slot = slot0 + tid;
+    bool active = slot < N;
+    if (active) {
+        const int o = a.orig_slot[slot];
+        active = o >= a.a0 && o < a.a1;
+    }
+    const uint32_t wi = (uint32_t)a.type_slot[min(slot, N - 1)] | slot << 8;
+    const unsigned long long amask = __ballot(active);
+    unsigned long long ncand = 0, nscr = 0, nre = 0;
+    // the candidate queue as LDS byte addresses: start, end, this lane's sink
+    const uint32_t qlo = lds_addr(q), qsink = qlo + 4u * ((uint32_t)(QC - QSINK) + lane);
+    uint32_t qa = qlo, rn = 0;
+    for (uint32_t k = w.k0; k < w.k1; k++) {
+        const uint64_t fi = b.primo + (uint64_t)k * a.skip, fj = fi + t;
+        const double *box = a.box + fi * 9;
+        const CellScreen cs = ca.cells[fi];
+        const double4 xi = a.pos[fi * N + min(slot, N - 1)];
+        const uint4 f32 = fractions32<TRI>(xi, box, cs, wi);
+        const uint2 f = round16(f32);
+        const FracBox ib = frac_box(f, active);
+        uint32_t th = active ? cs.threshold + 1u : 0u;  // strict: inactive lanes never pass
+        asm volatile("" : "+v"(th));  // kept as a value, not as a mask beside every comparison
+        // the reference's FP64 sequence
+        auto recheck = [&](uint32_t e, bool valid) {
+            if (valid) {
+                const uint32_t si = slot0 + (e & 0xFFu), sj = e >> 8;
+                const double4 x = a.pos[fi * N + si], y = a.pos[fj * N + sj];
+                const DevCell c = load_cell(box);
+                const double d2 = d2_ref<TRI>(x.x, x.y, x.z, y.x, y.y, y.z, c);
+                if (d2 >= a.lo && d2 <= a.rmax2 && d2 < a.Tn) {
+                    const int bb = bin_of(d2, thr, (int)a.nbin, a.rminf, a.inv_drf);
+                    atomicAdd(&hist[hidx((uint32_t)a.type_slot[si], (uint32_t)a.type_slot[sj], a.nt, a.nbin, (uint32_t)bb)], 1u);
+                }
+            }
+        };
+        // the queue's candidate e of this lane, in the j tile from j0
+        auto evaluate = [&](uint32_t e, bool valid, uint32_t j0) {
+            bool need = false;
+            if (valid) {
+                const uint4 ui = i32[e & 0xFFu], uj = j32[e >> 8];
+                const float fa = (float)(int)(ui.x - uj.x);
+                const float fb = (float)(int)(ui.y - uj.y);
+                const float fc = (float)(int)(ui.z - uj.z);
+                float dx, dy, dz;
+                if (TRI) {
+                    dz = cs.cz * fc;
+                    dy = fmaf(cs.cyz, fc, cs.cy * fb);
+                    dx = fmaf(cs.cxz, fc, fmaf(cs.cxy, fb, cs.cx * fa));
+                } else {
+                    dx = cs.cx * fa;
+                    dy = cs.cy * fb;
+                    dz = cs.cz * fc;
+                }
+                const float d2 = fmaf(dz, dz, fmaf(dy, dy, dx * dx));
+                const float u = (__builtin_amdgcn_sqrtf(d2) - a.rminf) * a.inv_drf;
+                need = fabsf(u - rintf(u)) < cs.du_margin;
+                const int bb = floor_i32(u);
+                const bool add = !need && (unsigned)bb < a.nbin;
+                atomicAdd(add ? &hist[hidx(ui.w, uj.w, a.nt, a.nbin, (uint32_t)bb)] : sink, 1u);
+            }
+            const unsigned long long m = __ballot(need);
+            if (m) {
+                if (need) rq[lane_slot(m, rn)] = (e & 0xFFu) | (j0 + (e >> 8)) << 8;
+                rn += (uint32_t)__popcll(m);
+                if (rn >= 64) {
+                    wave_sync_lds();
+                    rn -= 64;
+                    recheck(rq[rn + lane], true);
+                    nre += 64;
+                }
+            }
+        };
+        for (uint32_t j0 = 0; j0 < N; j0 += WG) {
+            __syncthreads();  // the previous tile's candidates are done
+            if (j0 == 0) i32[tid] = f32;
+            {
+                const uint32_t j = min(j0 + tid, N - 1);
+                const uint4 g32 = fractions32<TRI>(a.pos[fj * N + j], box, cs, (uint32_t)a.type_slot[j] | j << 8);
+                const uint2 g = round16(g32);
+                j32[tid] = g32;
+                jf[tid] = g;
+                const FracBox bx = frac_box(g, true);
+                if (lane == 0) jb[wave] = bx;
+            }
+            __syncthreads();
+            if (!amask) continue;  // no i in this wavefront
+            const uint32_t nj = min((uint32_t)WG, N - j0);
+            for (uint32_t g0 = 0; g0 < nj; g0 += 64) {
+                const FracBox bx = jb[g0 / 64];
+                if (!(axis_near(ib.c0, ib.e0, bx.c0, bx.e0, cs.gap0) && axis_near(ib.c1, ib.e1, bx.c1, bx.e1, cs.gap1) &&
+                      axis_near(ib.c2, ib.e2, bx.c2, bx.e2, cs.gap2)))
+                    continue;
+                const uint32_t ng = min(64u, nj - g0);
+                nscr += ng;
+                auto append = [&](bool pass, unsigned long long m, uint32_t j) {
+                    if (m) {
+                        uint32_t at = qa + 4u * lane_prefix(m);
+                        asm volatile("" : "+v"(at));  // every lane: a select, no branch
+                        *(lds_u32_t *)(size_t)(pass ? at : qsink) = j << 8 | tid;
+                        qa += 4u * (uint32_t)__popcll(m);
+                    }
+                };
+                auto drain = [&] {
+                    while (qa >= qlo + 256u) {
+                        wave_sync_lds();
+                        qa -= 256u;
+                        evaluate(*(lds_u32_t *)(size_t)(qa + 4u * lane), true, j0);
+                        ncand += 64;
+                        wave_sync_lds();
+                    }
+                };
+                uint32_t u = 0;
+                for (; u + 8 <= ng; u += 8) {
+                    uint4 r[4];
+                    bool pass[8];
+                    unsigned long long m[8];
+#pragma unroll
+                    for (int v = 0; v < 4; v++) r[v] = *reinterpret_cast<const uint4 *>(&jf[g0 + u + 2 * v]);
+#pragma unroll
+                    for (int v = 0; v < 8; v++) {
+                        pass[v] = sq16(f.x, v & 1 ? r[v / 2].z : r[v / 2].x, f.y, v & 1 ? r[v / 2].w : r[v / 2].y) < th;
+                        m[v] = __ballot(pass[v]);
+                    }
+#pragma unroll
+                    for (int v = 0; v < 8; v++) append(pass[v], m[v], g0 + u + v);
+                    drain();
+                }
+                if (u < ng) {  // the last atoms (the slots past them hold copies)
+                    for (; u < ng; u++) {
+                        const bool pass = sq16(f.x, jf[g0 + u].x, f.y, jf[g0 + u].y) < th;
+                        append(pass, __ballot(pass), g0 + u);
+                    }
+                    drain();
+                }
+            }
+            if (qa != qlo) {
+                const uint32_t n = (qa - qlo) >> 2;
+                wave_sync_lds();
+                evaluate(q[lane], lane < n, j0);
+                ncand += n;
+                qa = qlo;
+            }
+        }
+        wave_sync_lds();
+        recheck(rq[lane], lane < rn);
+        nre += rn;
+        rn = 0;
+        wave_sync_lds();
+        if (active) move_self_pair<TRI>(a, fi, fj, wi, box, thr, hist);
+    }
+    if (a.ncand) {
+        const unsigned long long na = (unsigned long long)__popcll(amask);
+        if (lane == 0 && na) {
+            atomicAdd(a.ncand + STAT_CANDIDATES, ncand);
+            atomicAdd(a.ncand + STAT_RECHECKS, nre);
+            atomicAdd(a.ncand + STAT_EXACT, nre);
+            atomicAdd(a.ncand + STAT_PAIRS_16, nscr * na);
+            atomicAdd(a.ncand + STAT_PAIRS_ALL, na * N * (w.k1 - w.k0));
+        }
+    }
+    __syncthreads();
+    lds_flush_rows(a, hist, rowch, w.block, t);
+}
+
 // CMODE, the cluster screen's j loop: 1 the groups left by the bounding-
 // sphere test, two per step; 2 the same with each step's columns cached in
 // LDS as FP32 offsets for the candidates' evaluation; 3 every 64 consecutive
@@ -1494,6 +1772,9 @@ struct anl_gofrt {
     int32_t *d_chan = nullptr;
     unsigned long long *d_ncand = nullptr;   // [NSTAT] statistics of the last launch (Stat)
     int last_form = -1;
+    // a changing cell: the screen of every frame's cell (prepare_cells)
+    CellScreen *d_cells = nullptr;
+    int cells = -1;               // -1 not looked at, 0 the screen does not apply, 1 it does
     // scratch for the work list
     BlockInfo *d_blocks = nullptr;
     WorkItem *d_work = nullptr;
@@ -1516,6 +1797,50 @@ int choose_form(anl_gofrt *g) {
     return ANL_GOFRT_FP64;
 }
 
+// Whether the automatic form of a trajectory with a changing cell takes
+// gofrt_cells_kernel: the screen's preconditions hold in every frame's cell.
+// From 256 atoms, one full tile of i (40 t0, 10 lags, plain -> this: 256 atoms
+// at rmax 0.3 and 0.49 of the cell length 218 -> 162 and 238 -> 188 us, 3,000
+// at 0.49, tilted, 8.33 -> 4.12 ms, 10,000 at 0.2 49.5 -> 11.2 ms); below,
+// most lanes of the tile idle and the launch is what a call costs.
+constexpr uint64_t CELLS_MIN_ATOMS = 256;
+bool use_cells(anl_gofrt *g) {
+    anl_traj *tr = g->tr;
+    if (g->form != ANL_GOFRT_AUTO || tr->box_const || tr->N < CELLS_MIN_ATOMS) return false;
+    if (g->cells < 0) {
+        std::vector<CellScreen> cells(tr->F);
+        g->cells = 1;
+        for (uint64_t f = 0; f < tr->F && g->cells; f++) {
+            const Cell c = cell_of(&tr->box_host[f * 9]);
+            double wd[3];
+            const Screen s = make_screen(c, true, tr->nt, g->rmax, wd);
+            // the fractions' rounding e_s (as in d2_window_fp64) stays below
+            // their quantisation, which the FP32 window's bound counts
+            const double lmin = std::min(c.L[0], std::min(c.L[1], c.L[2]));
+            const double tilt = std::max(std::fabs(c.xy), std::max(std::fabs(c.xz), std::fabs(c.yz))) / lmin;
+            const double lo = std::max(std::fabs(c.lo[0]), std::max(std::fabs(c.lo[1]), std::fabs(c.lo[2])));
+            const double e_s = 16.0 * std::ldexp(1.0, -53) * (1.0 + tilt) * (1.0 + tilt) * ((tr->pos_max + lo) / lmin + 1.0);
+            if (!s.valid || !(e_s < std::ldexp(1.0, -33))) {
+                g->cells = 0;
+                break;
+            }
+            uint32_t gap[3];
+            for (int k = 0; k < 3; k++)
+                gap[k] = (uint32_t)std::ceil((std::fabs(g->rmax) * (1 + 1e-9) + 1e-12) * 65536.0 / wd[k] * (1 + 1e-9)) + 4;
+            const double sc = std::ldexp(1.0, -32);
+            cells[f] = CellScreen{1.0 / c.L[0], 1.0 / c.L[1], 1.0 / c.L[2], s.threshold, gap[0], gap[1], gap[2],
+                                  (float)(c.L[0] * sc), (float)(c.xy * sc), (float)(c.xz * sc), (float)(c.L[1] * sc),
+                                  (float)(c.yz * sc), (float)(c.L[2] * sc),
+                                  du_window(s, tr->triclinic, g->rmin, g->rmax, g->dr, g->nbin), 0.0f};
+        }
+        if (g->cells) {
+            ANL_HIP(hipMalloc(&g->d_cells, cells.size() * sizeof(CellScreen)));
+            ANL_HIP(hipMemcpy(g->d_cells, cells.data(), cells.size() * sizeof(CellScreen), hipMemcpyHostToDevice));
+        }
+    }
+    return g->cells == 1;
+}
+
 struct Launch {
     std::vector<BlockInfo> blocks;
     std::vector<WorkItem> work;
@@ -1534,11 +1859,14 @@ Launch plan(anl_gofrt *g, const uint64_t *primo, const uint32_t *n, uint32_t nbl
     uint64_t target = g->tune.pairs_per_wg / ((uint64_t)WG * N);
     if (target < 1) target = 1;
     const uint64_t chunk = std::min(cap, target);
-    // a launch of fewer than 8 workgroups per CU (2,048 in all) leaves SIMDs
-    // idle: a small block splits its t0 range finer (the counts are sums of
-    // integers, so the split changes no result)
+    // a launch of fewer than 16 workgroups per CU (4,096 in all) leaves SIMDs
+    // idle or its last pass over the chip nearly empty: a small block splits
+    // its t0 range finer (the counts are sums of integers, so the split
+    // changes no result).  2,048 -> 4,096, rounded up: 1,000 atoms, 150 t0, 51
+    // lags 4.25 -> 4.02 ms; 3,000 atoms, 20 t0, 10 lags 2.16 -> 1.76; 8,192
+    // gains nothing more
     const uint64_t ntiles = (N + WG - 1) / WG;
-    const uint64_t want = (2048 + nblocks - 1) / nblocks;
+    const uint64_t want = (4096 + nblocks - 1) / nblocks;
     for (uint32_t bi = 0; bi < nblocks; bi++) {
         uint32_t leff = (n[bi] < g->lmax || g->lmax == 0) ? n[bi] : g->lmax;
         L.blocks.push_back(BlockInfo{primo[bi], leff, 0});
@@ -1552,7 +1880,7 @@ Launch plan(anl_gofrt *g, const uint64_t *primo, const uint32_t *n, uint32_t nbl
         uint64_t chunk_b = chunk;
         if (units * ((n0 + chunk - 1) / chunk) < want) {
             const uint64_t items = (want + units - 1) / units;
-            chunk_b = std::min(chunk, std::max<uint64_t>(1, (n0 + items - 1) / items));
+            chunk_b = std::min(chunk, std::max<uint64_t>(1, n0 / items));
         }
         for (uint64_t k = 0; k < n0; k += chunk_b)
             L.work.push_back(WorkItem{bi, (uint32_t)k, (uint32_t)std::min<uint64_t>(n0, k + chunk_b), 0});
@@ -1586,6 +1914,7 @@ struct GofrtPrepared {
     bool triclinic = false;
     int unroll = 4;
     int cluster = 0;  // as GofrtTuning::cluster, 0 when the cluster screen cannot be used
+    bool cells = false;  // gofrt_cells_kernel
     // device work list and block table owned by this launch (block engine)
     BlockInfo *own_blocks = nullptr;
     WorkItem *own_work = nullptr;
@@ -1714,12 +2043,6 @@ GofrtPrepared gofrt_prepare(anl_gofrt *g, const Launch &L, uint64_t out_len, int
     const uint64_t total = (uint64_t)ntiles * nlag * L.work.size();
     const uint64_t per = (total + 7) / 8;
     if (8 * per >= (1ull << 32)) fail(ANL_ERR_ARG, "too many workgroups (reduce the trajectory block)");
-    a.ntiles = ntiles;
-    a.nlag = nlag;
-    a.nwork = (uint32_t)L.work.size();
-    const bool remap = g->tune.xcd && form == ANL_GOFRT_SCREENED;
-    a.per_xcd = remap ? (uint32_t)per : 0u;
-    P.grid = dim3((uint32_t)(remap ? 8 * per : total));
     // channel table (FP64 form) or histogram-offset table (screened form, two
     // entries per type pair), bin-edge table, histogram
     const size_t common = (g->nbin + 1) * sizeof(double) +
@@ -1728,6 +2051,15 @@ GofrtPrepared gofrt_prepare(anl_gofrt *g, const Launch &L, uint64_t out_len, int
     auto screened_lds = [&](int qcap, bool cluster) {
         return (cluster ? 2 : 1) * WG * sizeof(uint4) + (WG / 64) * (qcap + RQCAP) * sizeof(uint32_t) + common;
     };
+    const size_t cells_lds = screened_lds(SQCAP, true) + WG * sizeof(uint2) + WG / 64 * sizeof(FracBox) +
+                             tr->nt * tr->nt * sizeof(int);
+    const bool cells = form == ANL_GOFRT_FP64 && cells_lds <= 160 * 1024 && use_cells(g);
+    a.ntiles = ntiles;
+    a.nlag = nlag;
+    a.nwork = (uint32_t)L.work.size();
+    const bool remap = g->tune.xcd && (form == ANL_GOFRT_SCREENED || cells);
+    a.per_xcd = remap ? (uint32_t)per : 0u;
+    P.grid = dim3((uint32_t)(remap ? 8 * per : total));
     // the cluster screen needs the larger queue; without room it is not used
     const bool colc = g->tune.cluster == 2 || g->tune.cluster == 4;
     const int qcl = colc ? SQCAP_CLC : SQCAP_CL;
@@ -1735,12 +2067,16 @@ GofrtPrepared gofrt_prepare(anl_gofrt *g, const Launch &L, uint64_t out_len, int
                             screened_lds(qcl, colc) <= 160 * 1024;
     P.lds = form == ANL_GOFRT_FP64 ? common : (cluster_ok ? screened_lds(qcl, colc) : screened_lds(SQCAP, false));
     if (P.lds > 160 * 1024) fail(ANL_ERR_ARG, "histogram does not fit in LDS (reduce nbin or types)");
+    if (cells) {
+        P.cells = true;
+        P.lds = cells_lds;
+    }
     P.form = form;
     P.out_len = out_len;
     P.triclinic = tr->triclinic;
     P.unroll = g->tune.unroll;
     P.cluster = cluster_ok ? g->tune.cluster : 0;
-    g->last_form = form;
+    g->last_form = P.cells ? ANL_GOFRT_SCREENED : form;
     return P;
 }
 
@@ -1750,7 +2086,11 @@ void gofrt_enqueue(anl_gofrt *g, const GofrtPrepared &P, unsigned long long *out
     zero_u64(out, P.out_len, s);
     zero_u64(g->d_ncand, NSTAT, s);
     if (P.grid.x == 0) return;
-    if (P.form == ANL_GOFRT_FP64) {
+    if (P.cells) {
+        const GofrtCellArgs c{a, g->d_cells};
+        if (P.triclinic) hipLaunchKernelGGL(gofrt_cells_kernel<true>, P.grid, dim3(WG), P.lds, s, c);
+        else hipLaunchKernelGGL(gofrt_cells_kernel<false>, P.grid, dim3(WG), P.lds, s, c);
+    } else if (P.form == ANL_GOFRT_FP64) {
         if (P.triclinic) hipLaunchKernelGGL(gofrt_fp64_kernel<true>, P.grid, dim3(WG), P.lds, s, a);
         else hipLaunchKernelGGL(gofrt_fp64_kernel<false>, P.grid, dim3(WG), P.lds, s, a);
     } else {
@@ -1891,6 +2231,7 @@ int anl_gofrt_destroy(anl_gofrt *g) {
         (void)hipFree(g->d_thr);
         (void)hipFree(g->d_chan);
         (void)hipFree(g->d_ncand);
+        (void)hipFree(g->d_cells);
         (void)hipFree(g->d_blocks);
         (void)hipFree(g->d_work);
         delete g;

@@ -37,7 +37,8 @@ extern "C" {
 #define ANL_GOFRT_FP64 0       /* plain FP64 evaluation of every ordered pair */
 #define ANL_GOFRT_SCREENED 1   /* 16-bit fixed-point screen of every pair, exact FP64
                                   evaluation of every candidate (same counts) */
-#define ANL_GOFRT_AUTO 2       /* SCREENED when its preconditions hold, else FP64 */
+#define ANL_GOFRT_AUTO 2       /* SCREENED when its preconditions hold (in a changing cell: in every
+                                * frame's, from 256 atoms), else FP64 */
 
 /* Message of the last failed call on this thread ("" if none). */
 const char *anl_last_error(void);
