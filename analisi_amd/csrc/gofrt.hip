@@ -1762,6 +1762,8 @@ struct GofrtTuning {
 struct anl_gofrt {
     anl_traj *tr = nullptr;
     GofrtTuning tune;
+    bool tuned = false;           // the caller or the environment set the shape, or the autotuner did
+    int fits = -1;                // clusters_fit, -1 not looked at
     double rmin = 0, rmax = 0, dr = 0, rmin2 = 0, rmax2 = 0;
     uint32_t nbin = 0, lmax = 0, skip = 1, every = 1;
     int form = ANL_GOFRT_AUTO;
@@ -1839,6 +1841,46 @@ bool use_cells(anl_gofrt *g) {
         }
     }
     return g->cells == 1;
+}
+
+// Whether the cluster screen pays for a launch shape nobody chose, from frame
+// 0's groups: `unfit`, the share of wavefronts too wide for it (they fall back
+// to the 16-bit screen in a kernel with fewer registers left for it), and
+// `near`, the volume a compact wavefront cannot skip over that of the cell.  A
+// wavefront's radius is taken as half the extent of its two groups' spheres.
+// The line near + unfit = 0.9 is where 6 t0 x 6 lags of 4,000 to 40,000 atoms
+// and 40 x 10 of 1,000 to 8,000, rmax 0.04 to 0.35 of a cubic cell, broke
+// even.  Cluster against 16-bit: 4,000 atoms 290 / 325 us at 0.57, 476 / 428 at
+// 1.5; 12,000 1.61 / 1.75 ms at 0.85, 2.29 / 2.17 at 1.35; 24,000 6.08 / 6.97
+// at 0.82, 10.5 / 8.84 at 1.23; 1,000 atoms 547 / 411 us at 1.4 (rmax 0.1 of
+// the cell) and 635 / 477 at 2 and more.
+bool clusters_fit(anl_gofrt *g, float rho_cap) {
+    if (g->fits < 0) {
+        anl_traj *tr = g->tr;
+        const uint64_t ng = (tr->N + 31) / 32;
+        std::vector<uint4> gr(ng);
+        ANL_HIP(hipMemcpy(gr.data(), tr->jgroups, ng * sizeof(uint4), hipMemcpyDeviceToHost));
+        const Cell &c = tr->cell0;
+        auto wrap = [](uint32_t x) { return (double)(int16_t)(x & 0xFFFFu) * 0x1p-16; };
+        uint64_t fit = 0, all = 0;
+        double reach = 0;
+        for (uint64_t k = 0; k < ng; k += 2, all++) {
+            const uint4 a = gr[k], b = gr[std::min(k + 1, ng - 1)];
+            const double sa = wrap(a.x - b.x), sb = wrap((a.x >> 16) - (b.x >> 16)), sc = wrap(a.y - b.y);
+            const double x = c.L[0] * sa + c.xy * sb + c.xz * sc, y = c.L[1] * sb + c.yz * sc, z = c.L[2] * sc;
+            float ra, rb;
+            std::memcpy(&ra, &a.z, sizeof(float));
+            std::memcpy(&rb, &b.z, sizeof(float));
+            const double rho = 0.5 * (std::sqrt(x * x + y * y + z * z) + ra + rb);
+            fit += rho < rho_cap;
+            reach += rho + std::fabs(g->rmax) + 0.5 * (ra + rb);
+        }
+        reach /= (double)all;
+        const double near = 4.0 / 3.0 * 3.14159265358979 * reach * reach * reach / (c.L[0] * c.L[1] * c.L[2]);
+        const double unfit = 1.0 - (double)fit / (double)all;
+        g->fits = near + unfit < 0.9;
+    }
+    return g->fits == 1;
 }
 
 struct Launch {
@@ -2064,7 +2106,7 @@ GofrtPrepared gofrt_prepare(anl_gofrt *g, const Launch &L, uint64_t out_len, int
     const bool colc = g->tune.cluster == 2 || g->tune.cluster == 4;
     const int qcl = colc ? SQCAP_CLC : SQCAP_CL;
     const bool cluster_ok = g->tune.cluster != 0 && form == ANL_GOFRT_SCREENED && a.rho_cap > 0 &&
-                            screened_lds(qcl, colc) <= 160 * 1024;
+                            screened_lds(qcl, colc) <= 160 * 1024 && (g->tuned || clusters_fit(g, a.rho_cap));
     P.lds = form == ANL_GOFRT_FP64 ? common : (cluster_ok ? screened_lds(qcl, colc) : screened_lds(SQCAP, false));
     if (P.lds > 160 * 1024) fail(ANL_ERR_ARG, "histogram does not fit in LDS (reduce nbin or types)");
     if (cells) {
@@ -2180,7 +2222,10 @@ int anl_gofrt_create(anl_traj *tr, double rmin, double rmax, uint32_t nbin, uint
         g->form = form;
         if (const char *e = std::getenv("ANL_GOFRT_UNROLL")) g->tune.unroll = std::atoi(e) == 8 ? 8 : 4;
         if (const char *e = std::getenv("ANL_GOFRT_XCD")) g->tune.xcd = std::atoi(e) != 0;
-        if (const char *e = std::getenv("ANL_GOFRT_CLUSTER")) g->tune.cluster = std::min(4, std::max(0, std::atoi(e)));
+        if (const char *e = std::getenv("ANL_GOFRT_CLUSTER")) {
+            g->tune.cluster = std::min(4, std::max(0, std::atoi(e)));
+            g->tuned = true;
+        }
         if (const char *e = std::getenv("ANL_GOFRT_PAIRS_PER_WG")) {
             long long v = std::atoll(e);
             if (v > 0) g->tune.pairs_per_wg = (uint64_t)v;
@@ -2393,6 +2438,7 @@ int anl_gofrt_set_tuning(anl_gofrt *g, int unroll, int xcd, uint64_t pairs_per_w
         if (!g) fail(ANL_ERR_ARG, "null handle");
         if (unroll != 4 && unroll != 8) fail(ANL_ERR_ARG, "unroll must be 4 or 8");
         if (pairs_per_wg == 0) fail(ANL_ERR_ARG, "pairs_per_wg must be positive");
+        g->tuned = true;
         g->tune.unroll = unroll;
         g->tune.xcd = xcd != 0;
         g->tune.pairs_per_wg = pairs_per_wg;
@@ -2443,6 +2489,8 @@ int anl_gofrt_autotune(anl_gofrt *g, uint64_t primo, uint32_t nlag_probe, const 
         const uint64_t len = (uint64_t)g->leff * nch_of(g->tr) * g->nbin;
         if (len == 0) return;
         const GofrtTuning saved = g->tune;
+        const bool saved_tuned = g->tuned;
+        g->tuned = true;  // the candidates' modes as they are
         unsigned long long *d = nullptr;
         hipEvent_t e0 = nullptr, e1 = nullptr;
         ANL_HIP(hipMalloc(&d, len * sizeof(unsigned long long)));
@@ -2476,6 +2524,7 @@ int anl_gofrt_autotune(anl_gofrt *g, uint64_t primo, uint32_t nlag_probe, const 
             }
         } catch (...) {
             g->tune = saved;
+            g->tuned = saved_tuned;
             if (e0) (void)hipEventDestroy(e0);
             if (e1) (void)hipEventDestroy(e1);
             (void)hipFree(d);
