@@ -70,6 +70,7 @@ SIGNATURES = [
     ("anl_series_destroy", _i, [_vp]),
     ("anl_gk_calculate", _i, [_vp, _vp, _u32, _u32, _u32, _u32, _u32, _i, _u32, _u64, _vp]),
     ("anl_gk_calculate_mfma", _i, [_vp, _vp, _u32, _u32, _u32, _u32, _u32, _i, _u32, _u64, _vp]),
+    ("anl_gk_calculate_blocks", _i, [_vp, _vp, _u32, _u32, _u32, _u32, _i, _u32, _vp, _vp, _u32, _i, _vp, _vp, _vp]),
     ("anl_gk_calculate_blocks_async", _i, [_vp, _vp, _u32, _u32, _u32, _u32, _i, _u32, _vp, _vp, _u32, _i, _vp, _vp,
                                           _vp, _vp]),
     ("anl_gk_calculate_async", _i, [_vp, _vp, _u32, _u32, _u32, _u32, _u32, _i, _u32, _u64, _vp, _vp]),
@@ -476,17 +477,13 @@ class DeviceSeries:
         nb = len(pr)
         leff = int(nn[0]) if (int(nn[0]) < tmax or tmax == 0) else tmax
         narr = 3 * ncur * ncur + 2
-        out = DeviceBuffer(nb * leff * narr * 8)
-        mean = DeviceBuffer(leff * narr * 8) if stats else None
-        var = DeviceBuffer(leff * narr * 8) if stats else None
-        check(lib().anl_gk_calculate_blocks_async(self.handle, _ptr(idx), ncur, skip, tmax, n_seg,
-                                                  int(bool(subtract_mean)), start_mean, _ptr(pr), _ptr(nn), nb,
-                                                  GK_MFMA if mfma else GK_FP64, out.ptr,
-                                                  mean.ptr if stats else None, var.ptr if stats else None, None))
-        res = out.to_host((nb, leff, narr))
-        if not stats:
-            return res, None, None
-        return res, mean.to_host((leff, narr)), var.to_host((leff, narr))
+        out = np.empty((nb, leff, narr))
+        mean = np.empty((leff, narr)) if stats else None
+        var = np.empty((leff, narr)) if stats else None
+        check(lib().anl_gk_calculate_blocks(self.handle, _ptr(idx), ncur, skip, tmax, n_seg, int(bool(subtract_mean)),
+                                            start_mean, _ptr(pr), _ptr(nn), nb, GK_MFMA if mfma else GK_FP64, _ptr(out),
+                                            _ptr(mean) if stats else None, _ptr(var) if stats else None))
+        return out, mean, var
 
     def set_gk_shape(self, tiles_per_wave, chunk_steps, waves_per_group):
         check(lib().anl_gk_set_tuning(self.handle, tiles_per_wave, chunk_steps, waves_per_group))

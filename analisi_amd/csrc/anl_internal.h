@@ -4,8 +4,11 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <algorithm>
+#include <exception>
 #include <mutex>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "../../include/analisi_hip.h"
@@ -51,6 +54,35 @@ struct Cell {
     double L[3];
     double xy, xz, yz;
 };
+
+// f(thread, begin, end) over [0, n) on up to `most` threads, at least
+// `grain` elements each; on the calling thread alone when n is small.
+constexpr unsigned HOST_THREADS = 16;
+template <class F>
+void parallel(uint64_t n, uint64_t grain, F f, unsigned most = HOST_THREADS) {
+    const uint64_t nth = std::min<uint64_t>(std::min(most, std::max(1u, std::thread::hardware_concurrency())),
+                                            std::max<uint64_t>(1, n / grain));
+    std::vector<std::thread> pool;
+    std::vector<std::exception_ptr> failed(nth);
+    const auto run = [&](unsigned th, uint64_t i0, uint64_t i1) {
+        try {
+            f(th, i0, i1);
+        } catch (...) {
+            failed[th] = std::current_exception();
+        }
+    };
+    uint64_t own = n / nth;
+    try {
+        pool.reserve(nth);
+        for (uint64_t k = nth; k-- > 1;) pool.emplace_back(run, (unsigned)k, n * k / nth, n * (k + 1) / nth);
+    } catch (...) {  // no more threads: the calling one takes what is left
+        own = n * (nth - pool.size()) / nth;
+    }
+    run(0, 0, own);
+    for (auto &t : pool) t.join();
+    for (auto &e : failed)
+        if (e) std::rethrow_exception(e);
+}
 
 // Device and pinned host memory of one calculation, kept for the next one of
 // the same trajectory.
@@ -115,6 +147,7 @@ struct anl_traj {
     uint2 *frac16 = nullptr;            // [F][N] {a | b<<16, c} 16-bit fractions, lazily built
     uint4 *frac32 = nullptr;            // [F][N] {a, b, c, type | slot << 8} 32-bit fractions, lazily built
     int32_t *frac_order = nullptr;      // [F][N] slot held by each screen slot, until the fractions are built
+    std::mutex screen_mutex;            // held while the screen's order and fractions are built
     double4 *pos_scr = nullptr;         // [F][N] positions in each frame's screen order (with the fractions)
     uint4 *jgroups = nullptr;           // [F][ceil(N/32)] bounding spheres of 32 consecutive screen slots:
                                         // {centre a | b << 16, centre c, radius (float bits, A), 0}
@@ -140,6 +173,7 @@ struct anl_series {
     // calls on one series are stream-ordered on the caller's stream.
     void *work = nullptr;
     size_t work_cap = 0;
+    anl::ScratchPool scratch;  // outputs of anl_gk_calculate_blocks
     // launch shape of the MFMA lag products: tiles per wavefront, MFMA steps
     // per FP32 chunk, wavefronts per workgroup (anl_gk_set_tuning)
     uint32_t gk_q = 8, gk_cs = 16, gk_wg = 4;
@@ -151,6 +185,7 @@ Cell cell_of(const double *box9);
 // (int)floorf((float)((sqrt(d2) - rmin) / dr)) is >= k, computed on the host
 // with IEEE double arithmetic (gofrt.cpp:114-115, sphericalbase.cpp:52-53).
 std::vector<double> bin_edges(double rmin, double rmax, uint32_t nbin, double dr);
+void build_screen_order(anl_traj *tr);
 void build_frac16(anl_traj *tr, hipStream_t s);
 
 // Prepared launches for the block engine: all host work (checks, plans,

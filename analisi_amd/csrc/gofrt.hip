@@ -2252,6 +2252,7 @@ int anl_gofrt_create(anl_traj *tr, double rmin, double rmax, uint32_t nbin, uint
                 k[FP64K_YZ] = cl.yz * f;
                 k[FP64K_Z] = cl.L[2] * f;
                 k[FP64K_EPS] = d2_window_fp64(sc, cl, tr->pos_max, rmax);
+                if (form != ANL_GOFRT_FP64) build_screen_order(tr);
             }
             ANL_HIP(hipMalloc(&g->d_thr, t.size() * sizeof(double)));
             ANL_HIP(hipMemcpy(g->d_thr, t.data(), t.size() * sizeof(double), hipMemcpyHostToDevice));

@@ -1,10 +1,12 @@
 // Runtime of libanalisi_hip: errors, device selection, trajectory and time
 // series mirrors, block statistics kernels.
 #include <algorithm>
+#include <atomic>
 #include <array>
 #include <thread>
 #include <cmath>
 #include <cstring>
+#include <exception>
 #include <memory>
 #include <numeric>
 
@@ -195,7 +197,54 @@ __global__ void jgroup_kernel(const uint2 *__restrict__ frac16, uint64_t natoms,
     out[k] = make_uint4(ca | (cb << 16), cc, __float_as_uint(R), 0u);
 }
 
+static void kd_order(int32_t *order, const std::array<float, 3> *fr, size_t lo, size_t hi, const double len[3]);
+
+// Screen order, per frame: the bisection of the slot order applied to that
+// frame's positions, so that the atoms of one wavefront stay compact in every
+// frame while they diffuse.  frac_order[f][s] = slot of the atom at screen slot
+// s.  Only the screened g(r,t) needs it (constant cell): its handle builds it,
+// from the device's positions, and every other calculation does without (the
+// first MSD over a new trajectory, 8,192 atoms x 1,000 frames: 124 -> 32 ms, with the
+// checks and the staging of the positions on several threads).
+void build_screen_order(anl_traj *tr) {
+    std::lock_guard<std::mutex> lock(tr->screen_mutex);
+    if (tr->frac16 || tr->frac_order) return;
+    const uint64_t N = tr->N, F = tr->F;
+    const double len[3] = {tr->cell0.L[0], tr->cell0.L[1], tr->cell0.L[2]};
+    const uint64_t chunk = std::min<uint64_t>(F, std::max<uint64_t>(1, (64u << 20) / (N * sizeof(double4))));
+    std::vector<double4> pos(chunk * N);
+    std::vector<int32_t> ford(F * N);
+    for (uint64_t f0 = 0; f0 < F; f0 += chunk) {
+        const uint64_t nf = std::min(chunk, F - f0);
+        ANL_HIP(hipMemcpy(pos.data(), tr->pos + f0 * N, nf * N * sizeof(double4), hipMemcpyDeviceToHost));
+        parallel(nf, 1, [&](unsigned, uint64_t i0, uint64_t i1) {
+                std::vector<std::array<float, 3>> fs(N);
+                for (uint64_t f = i0; f < i1; f++) {
+                    for (uint64_t sl = 0; sl < N; sl++) {
+                        const double4 x = pos[f * N + sl];
+                        double s3[3];
+                        to_fractional(tr->cell0, x.x, x.y, x.z, s3);
+                        for (int c = 0; c < 3; c++) fs[sl][c] = (float)(s3[c] - std::floor(s3[c]));
+                    }
+                    int32_t *o = ford.data() + (f0 + f) * N;
+                    std::iota(o, o + N, 0);
+                    kd_order(o, fs.data(), 0, N, len);
+                }
+            });
+    }
+    int32_t *d = nullptr;
+    ANL_HIP(hipMalloc(&d, F * N * sizeof(int32_t)));
+    const hipError_t e = hipMemcpy(d, ford.data(), F * N * sizeof(int32_t), hipMemcpyHostToDevice);
+    if (e != hipSuccess) {
+        (void)hipFree(d);
+        ANL_HIP(e);
+    }
+    tr->frac_order = d;
+}
+
 void build_frac16(anl_traj *tr, hipStream_t s) {
+    build_screen_order(tr);
+    std::lock_guard<std::mutex> lock(tr->screen_mutex);
     if (tr->frac16) return;
     uint64_t total = tr->F * tr->N;
     ANL_HIP(hipMalloc(&tr->frac16, total * sizeof(uint2)));
@@ -318,7 +367,7 @@ struct Uploader {
     hipEvent_t done[2] = {nullptr, nullptr};
     size_t cap;
     int k = 0;
-    explicit Uploader(size_t bytes) : cap(std::max<size_t>(bytes, 1 << 16)) {
+    explicit Uploader(size_t bytes) : cap(std::max<size_t>(bytes, 256 << 10)) {
         ANL_HIP(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));
         for (int i = 0; i < 2; i++) {
             ANL_HIP(hipHostMalloc(&stage[i], cap, hipHostMallocDefault));
@@ -354,6 +403,16 @@ struct Uploader {
         }
     }
     void finish() { ANL_HIP(hipStreamSynchronize(s)); }
+    // after finish(): one staging buffer becomes the first pinned workspace of
+    // the trajectory's calculations (allocating another would cost the first
+    // of them 0.35 ms)
+    void keep(ScratchPool &pool) {
+        Scratch w;
+        w.pin = stage[0];
+        w.pin_cap = cap;
+        stage[0] = nullptr;
+        pool.give(w);
+    }
 };
 
 }  // namespace anl
@@ -382,13 +441,21 @@ int anl_traj_create(const double *pos, const double *box, uint32_t box_stride, c
             for (uint32_t k = 6; k < box_stride; k++)
                 if (!std::isfinite(box[f * box_stride + k])) fail(ANL_ERR_ARG, "cell tilts must be finite");
         const double bound = 1e4 * 2 * lmin;
-        double pos_max = 0.0;
-        for (uint64_t i = 0; i < nframes * natoms * 3; i++) {
-            const double v = std::fabs(pos[i]);
-            if (!(v <= bound))
-                fail(ANL_ERR_ARG, "positions must be finite and within 10^4 (shortest) cell lengths of the origin");
-            pos_max = std::max(pos_max, v);
-        }
+        std::atomic<bool> refused{false};
+        std::vector<double> part(HOST_THREADS, 0.0);
+        parallel(nframes * natoms * 3, 1 << 18, [&](unsigned th, uint64_t i0, uint64_t i1) {
+            double m = 0.0;
+            bool bad = false;
+            for (uint64_t i = i0; i < i1; i++) {
+                const double v = std::fabs(pos[i]);
+                bad |= !(v <= bound);
+                m = v > m ? v : m;
+            }
+            part[th] = std::max(part[th], m);
+            if (bad) refused = true;
+        });
+        if (refused) fail(ANL_ERR_ARG, "positions must be finite and within 10^4 (shortest) cell lengths of the origin");
+        const double pos_max = *std::max_element(part.begin(), part.end());
         ensure_device();
         // on any failure below (a device allocation, an upload) everything
         // allocated so far is released with the trajectory
@@ -431,17 +498,23 @@ int anl_traj_create(const double *pos, const double *box, uint32_t box_stride, c
             tr->type_of_slot[s] = type_id[order[s]];
             tr->type_count[type_id[order[s]]]++;
         }
-        // permuted, padded positions, staged frame by frame in pinned memory
-        Uploader up(natoms * sizeof(double4));
-        ANL_HIP(hipMalloc(&tr->pos, nframes * natoms * sizeof(double4)));
-        for (uint64_t f = 0; f < nframes; f++) {
-            const double *p = pos + f * natoms * 3;
+        // permuted, padded positions, staged in pinned memory, as many frames
+        // at a time as fit
+        const size_t frame = natoms * sizeof(double4);
+        Uploader up(std::max<size_t>(frame, std::min<size_t>(nframes * frame, 4u << 20)));
+        ANL_HIP(hipMalloc(&tr->pos, nframes * frame));
+        const uint64_t batch = up.cap / frame;
+        for (uint64_t f0 = 0; f0 < nframes; f0 += batch) {
+            const uint64_t nf = std::min(batch, nframes - f0);
             double4 *buf = (double4 *)up.next();
-            for (uint64_t s = 0; s < natoms; s++) {
-                const double *x = p + (uint64_t)order[s] * 3;
-                buf[s] = make_double4(x[0], x[1], x[2], 0.0);
-            }
-            up.send(tr->pos + f * natoms, natoms * sizeof(double4));
+            parallel(nf * natoms, 1 << 15, [&](unsigned, uint64_t i0, uint64_t i1) {
+                for (uint64_t i = i0, f = i0 / natoms, s = i0 % natoms; i < i1; i++) {
+                    const double *x = pos + ((f0 + f) * natoms + (uint64_t)order[s]) * 3;
+                    buf[i] = make_double4(x[0], x[1], x[2], 0.0);
+                    if (++s == natoms) s = 0, f++;
+                }
+            });
+            up.send(tr->pos + f0 * natoms, nf * frame);
         }
         ANL_HIP(hipMalloc(&tr->box, nframes * 9 * sizeof(double)));
         up.put(tr->box, tr->box_host.data(), nframes * 9 * sizeof(double));
@@ -449,39 +522,12 @@ int anl_traj_create(const double *pos, const double *box, uint32_t box_stride, c
         up.put(tr->type_slot, tr->type_of_slot.data(), natoms * sizeof(int32_t));
         ANL_HIP(hipMalloc(&tr->orig_slot, natoms * sizeof(int32_t)));
         up.put(tr->orig_slot, order.data(), natoms * sizeof(int32_t));
-        // screen order, per frame (the screened g(r,t) needs a constant
-        // cell): the same bisection of that frame's positions, so that the
-        // atoms of one wavefront stay compact in every frame while they
-        // diffuse.  frac_order[f][s] = slot of the atom at screen slot s.
-        if (tr->box_const) {
-            std::vector<int32_t> ford(nframes * natoms);
-            const unsigned nth = std::max(1u, std::min(16u, std::thread::hardware_concurrency()));
-            std::vector<std::thread> pool;
-            for (unsigned k = 0; k < nth; k++)
-                pool.emplace_back([&, k] {
-                    std::vector<std::array<float, 3>> fs(natoms);
-                    for (uint64_t f = k; f < nframes; f += nth) {
-                        const double *p = pos + f * natoms * 3;
-                        for (uint64_t sl = 0; sl < natoms; sl++) {
-                            const double *x = p + (uint64_t)order[sl] * 3;
-                            double s3[3];
-                            to_fractional(tr->cell0, x[0], x[1], x[2], s3);
-                            for (int c = 0; c < 3; c++) fs[sl][c] = (float)(s3[c] - std::floor(s3[c]));
-                        }
-                        int32_t *o = ford.data() + f * natoms;
-                        std::iota(o, o + natoms, 0);
-                        kd_order(o, fs.data(), 0, natoms, len);
-                    }
-                });
-            for (auto &t : pool) t.join();
-            ANL_HIP(hipMalloc(&tr->frac_order, nframes * natoms * sizeof(int32_t)));
-            up.put(tr->frac_order, ford.data(), nframes * natoms * sizeof(int32_t));
-        }
         if (pos_cm) {
             ANL_HIP(hipMalloc(&tr->cm, nframes * ntypes * 3 * sizeof(double)));
             up.put(tr->cm, pos_cm, nframes * ntypes * 3 * sizeof(double));
         }
         up.finish();
+        up.keep(tr->scratch);
         *out = owner.release();
     });
 }

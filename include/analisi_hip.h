@@ -305,6 +305,12 @@ int anl_gk_calculate_blocks_async(anl_series *s, const uint32_t *idx_j, uint32_t
                                   uint32_t tmax, uint32_t n_seg, int subtract_mean, uint32_t start_mean,
                                   const uint64_t *primo, const uint32_t *n, uint32_t nblocks, int form,
                                   double *out_dev, double *mean_dev, double *var_dev, void *stream);
+/* The same to host memory, synchronous; mean_host and var_host both or
+ * neither. */
+int anl_gk_calculate_blocks(anl_series *s, const uint32_t *idx_j, uint32_t ncur, uint32_t skip, uint32_t tmax,
+                            uint32_t n_seg, int subtract_mean, uint32_t start_mean, const uint64_t *primo,
+                            const uint32_t *n, uint32_t nblocks, int form, double *out_host, double *mean_host,
+                            double *var_host);
 /* Stream-ordered variants writing [leff][3*ncur^2+2] FP64 to device memory.
  * Scratch lives in the series (grow-only; growing synchronises the device),
  * so the calls on one series must be ordered on one stream. */
