@@ -399,8 +399,13 @@ struct GofrtArgs {
     unsigned long long *ncand;   // [NSTAT] launch statistics, see the Stat enum
     const double *thr;           // [nbin+1] bin edges, then the FP64 window constants (FP64K_*)
     const int32_t *chan;         // [nt*nt]
+    // work list and block table; without them (null) one block `block0` whose t0
+    // indices [wk0, wk1) are cut into chunks of `chunk`
     const WorkItem *work;
     const BlockInfo *blocks;
+    BlockInfo block0;
+    uint32_t wk0, wk1, chunk;
+    uint32_t stage;                   // plain form, SPLIT: LDS offset of the staged j
     uint64_t N;
     uint64_t out_block_stride;   // leff_max * nch * nbin
     uint32_t nt, nbin, nch, half, skip, every;
@@ -415,6 +420,9 @@ struct GofrtArgs {
     unsigned long long *nrecheck;
     float cx, cxy, cxz, cy, cyz, cz;  // cell matrix entries times 2^-32
     float du_margin;                  // bins: |u - nearest integer| below this -> FP64
+    double d2_end;                    // d2 <= rmax2 && d2 < Tn  <=>  d2 < d2_end
+    float bin_margin;                 // bins: error bound of the plain form's FP32 quotient, twice
+    float zero_d2;                    // d2 up to this is in bin 0 (an atom with itself at lag 0), < 0: none
     float du_m0, du_m1;               // mode 2: window m0 + m1 (rho + dq) of the offset evaluation
     // cluster screen (see cluster_threshold): cell entries times 2^-16,
     // largest usable cluster radius, quantisation bound, rmax
@@ -449,6 +457,17 @@ __device__ __forceinline__ WgId decode_wg(uint32_t ntiles, uint32_t nlag, uint32
     return w;
 }
 
+__device__ __forceinline__ WorkItem work_item(const GofrtArgs &a, uint32_t k, BlockInfo &b) {
+    if (a.work) {
+        const WorkItem w = a.work[k];
+        b = a.blocks[w.block];
+        return w;
+    }
+    b = a.block0;
+    const uint32_t k0 = a.wk0 + k * a.chunk;
+    return WorkItem{0, k0, min(a.wk1, k0 + a.chunk), 0};
+}
+
 #include "min_image.h"
 
 __device__ __forceinline__ int bin_of(double d2, const double *T, int nbin, float rminf, float inv_drf) {
@@ -461,14 +480,7 @@ __device__ __forceinline__ int bin_of(double d2, const double *T, int nbin, floa
     return b;
 }
 
-__device__ __forceinline__ void lds_setup(const GofrtArgs &a, unsigned *hist, double *thr, int *chan) {
-    const int nh = (int)(a.nch * a.nbin);
-    for (int k = threadIdx.x; k < nh; k += WG) hist[k] = 0u;
-    for (int k = threadIdx.x; k <= (int)a.nbin; k += WG) thr[k] = a.thr[k];
-    for (int k = threadIdx.x; k < (int)(a.nt * a.nt); k += WG) chan[k] = a.chan[k];
-}
-
-// Screened form: the workgroup's histogram rows are the ordered type pairs of
+// The workgroup's histogram rows are the ordered type pairs of
 // distinct atoms (row ti nt + tj) and the types of an atom paired with itself
 // (row nt^2 + ti): nt (nt + 1) rows, as many as the reference's channels, so
 // that a candidate's row is arithmetic (hidx) and the flush folds the rows
@@ -516,8 +528,10 @@ __device__ __forceinline__ int floor_i32(float x) {
     return r;
 }
 
-// The screened form's flush: row r of the workgroup's histogram adds to its
-// channel rowch[r] (see lds_setup_rows), from a rotated start as lds_flush.
+// Row r of the workgroup's histogram adds to its channel rowch[r] (see
+// lds_setup_rows).  Workgroups of one (block, lag) flush into the same
+// counters, often at the same time (they start and end together): each starts
+// at its own offset, so that their atomics meet different addresses.
 __device__ __forceinline__ void lds_flush_rows(const GofrtArgs &a, const unsigned *hist, const int *rowch,
                                                uint32_t block, uint32_t t) {
     const int nh = (int)(a.nch * a.nbin);
@@ -531,73 +545,233 @@ __device__ __forceinline__ void lds_flush_rows(const GofrtArgs &a, const unsigne
     }
 }
 
-// Workgroups of one (block, lag) flush into the same counters, often at the
-// same time (they start and end together): each starts at its own offset,
-// so that their atomics meet different addresses.
-__device__ __forceinline__ void lds_flush(const GofrtArgs &a, const unsigned *hist, uint32_t block, uint32_t t) {
-    const int nh = (int)(a.nch * a.nbin);
-    unsigned long long *o = a.out + (uint64_t)block * a.out_block_stride + (uint64_t)t * nh;
-    const int rot = (int)((blockIdx.x * 977u) % (uint32_t)nh);
-    for (int k0 = threadIdx.x; k0 < nh; k0 += WG) {
-        const int k = k0 + rot < nh ? k0 + rot : k0 + rot - nh;
-        unsigned v = hist[k];
-        if (v) atomicAdd(o + k, (unsigned long long)v);
-    }
+__device__ __forceinline__ void wave_sync_lds() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// grid: x = i tile (256 slots), y = lag index, z = work item (block, t0 range)
-template <bool TRI>
-__global__ __launch_bounds__(WG) void gofrt_fp64_kernel(const GofrtArgs a) {
+constexpr int SPLIT_WG = 512;  // threads of a workgroup of the split plain form
+// LDS of a wavefront's 32 staged j: x, y, z and histogram row
+constexpr uint32_t STAGE_J = 32 * (3 * sizeof(double) + sizeof(uint32_t));
+
+// The plain form: every ordered pair with the reference's FP64 sequence.  A
+// lane owns an i atom and takes 4 j at a time, whose chains run side by side
+// (min_image_batch), while the next 4 are loaded.  The bin is the floor of an FP32 quotient
+// where that is farther than bin_margin from an integer (twice its error),
+// otherwise from the table of edges.
+// SPLIT: 64 i per workgroup, a t0 per pair of wavefronts, which share its j
+// (see FP64_SPLIT_ATOMS).
+// The plain form of a large system is bound by VALU issue, of a small one by
+// the length of a wavefront's chain.  256 i per workgroup, one j after the
+// other, the image's loops branching for each pair -> this: 3,000 atoms, 60 t0
+// x 12 lags, all pairs in range 16.9 -> 8.9 ms (tilted 19.1 -> 11.4; positions
+// ten cells out 96 -> 57), 3 % in range 10.4 -> 7.2; 56 atoms in three types,
+// 70 t0 x 10 lags: the kernel 52 -> 28 us.
+template <bool TRI, bool SPLIT>
+__global__ __launch_bounds__(SPLIT ? SPLIT_WG : WG) void gofrt_fp64_kernel(const GofrtArgs a) {
+    constexpr int U = 4;
+    constexpr uint32_t NTH = SPLIT ? SPLIT_WG : WG;
     extern __shared__ unsigned char smem[];
     const WgId id = decode_wg(a.ntiles, a.nlag, a.nwork, a.per_xcd);
     if (!id.valid) return;
-    const WorkItem w = a.work[id.work];
-    const BlockInfo b = a.blocks[w.block];
+    BlockInfo b;
+    const WorkItem w = work_item(a, id.work, b);
     const uint32_t t = a.lag0 + id.lagi * a.every;
     if (t >= b.leff) return;
     double *thr = (double *)smem;
-    int *chan = (int *)(thr + a.nbin + 1);
-    unsigned *hist = (unsigned *)(chan + a.nt * a.nt);
-    lds_setup(a, hist, thr, chan);
+    int *rowch = (int *)(thr + a.nbin + 1);                // [nt*nt] channel offset of a row of distinct atoms
+    unsigned *hist = (unsigned *)(rowch + a.nt * a.nt);
+    const uint32_t nh = a.nch * a.nbin;
+    for (uint32_t k = threadIdx.x; k < nh; k += NTH) hist[k] = 0u;
+    for (uint32_t k = threadIdx.x; k <= a.nbin; k += NTH) thr[k] = a.thr[k];
+    for (uint32_t k = threadIdx.x; k < a.nt * a.nt; k += NTH) rowch[k] = a.chan[k] * (int)a.nbin;
     __syncthreads();
 
-    const uint64_t N = a.N;
-    const uint64_t slot = (uint64_t)id.tile * WG + threadIdx.x;
+    const uint32_t N = (uint32_t)a.N, nbin = a.nbin, nt = a.nt;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t slot = id.tile * (SPLIT ? 64u : (uint32_t)WG) + (SPLIT ? threadIdx.x & 63u : threadIdx.x);
     bool active = slot < N;
-    int ti = 0;
+    uint32_t ti = 0;
     if (active) {
-        int o = a.orig_slot[slot];
+        const int o = a.orig_slot[slot];
         active = o >= a.a0 && o < a.a1;
-        ti = a.type_slot[slot];
+        ti = (uint32_t)a.type_slot[slot];
     }
-    const int nbin = (int)a.nbin;
-    // every ordered pair of an active i is evaluated: N per t0
-    const unsigned long long npairs = (unsigned long long)__popcll(__ballot(active)) * N * (w.k1 - w.k0);
-    for (uint32_t k = w.k0; k < w.k1; k++) {
-        const uint64_t fi = b.primo + (uint64_t)k * a.skip;
-        const uint64_t fj = fi + t;
-        const DevCell c = load_cell(a.box + fi * 9);
-        const double4 *__restrict__ pj = a.pos + fj * N;
-        if (active) {
-            const double4 xi = a.pos[fi * N + slot];
-            for (uint64_t j = 0; j < N; j++) {
-                const double4 xj = pj[j];
-                double d2 = d2_ref<TRI>(xi.x, xi.y, xi.z, xj.x, xj.y, xj.z, c);
-                if (d2 >= a.lo && d2 <= a.rmax2 && d2 < a.Tn) {
-                    int bb = bin_of(d2, thr, nbin, a.rminf, a.inv_drf);
-                    int tj = a.type_slot[j];
-                    int ch = chan[ti * a.nt + tj] + (slot == j ? (int)a.half : 0);
-                    atomicAdd(&hist[ch * nbin + bb], 1u);
+    const unsigned nact = (unsigned)__popcll(__ballot(active));
+    const uint32_t row0 = ti * nt * nbin, rowself = (nt * nt + ti) * nbin;
+    // d2 <= rmax2 and d2 < Tn as one comparison
+    const double hi = a.d2_end, lo = a.lo;
+    const float rminf = a.rminf, inv_drf = a.inv_drf, margin = a.bin_margin, zero_d2 = a.zero_d2;
+    uint32_t nt0 = 0;
+    // U pairs of this lane's atom at xi; js: slot of the first j, nv: how many there are
+    auto pairs = [&](const double4 &xi, const double (&yx)[U], const double (&yy)[U], const double (&yz)[U],
+                     const uint32_t (&row)[U], uint32_t js, uint32_t nv, const DevCell &c) {
+        double x0[U], x1[U], x2[U];
+#pragma unroll
+        for (int v = 0; v < U; v++) {
+            x0[v] = xi.x - yx[v];
+            x1[v] = xi.y - yy[v];
+            x2[v] = xi.z - yz[v];
+        }
+        min_image_batch<TRI, U>(x0, x1, x2, c);
+        if constexpr (!SPLIT) {
+            // many wavefronts per SIMD: a pair out of range costs nothing more
+#pragma unroll
+            for (int v = 0; v < U; v++) {
+                const double d2 = d2_of(x0[v], x1[v], x2[v]);
+                if (d2 >= lo && d2 < hi && (uint32_t)v < nv) {
+                    const float u = (__builtin_amdgcn_sqrtf((float)d2) - rminf) * inv_drf;
+                    int bb = floor_i32(u);
+                    if (!(fabsf(u - rintf(u)) > margin)) bb = bin_of(d2, thr, (int)nbin, rminf, inv_drf);
+                    atomicAdd(&hist[(slot == js + v ? rowself : row0 + row[v]) + (uint32_t)bb], 1u);
+                }
+            }
+            return;
+        }
+        // few wavefronts: no branches within the four
+        double d2[U];
+        bool in[U], any = false;
+#pragma unroll
+        for (int v = 0; v < U; v++) {
+            d2[v] = d2_of(x0[v], x1[v], x2[v]);
+            in[v] = (d2[v] >= lo) & (d2[v] < hi) & ((uint32_t)v < nv);
+            any |= in[v];
+        }
+        if (!__any(any)) return;
+        // every lane adds: 1 to its bin, or 0 to a word of its own
+        uint32_t need = 0;
+#pragma unroll
+        for (int v = 0; v < U; v++) {
+            const float f2 = (float)d2[v], u = (__builtin_amdgcn_sqrtf(f2) - rminf) * inv_drf;
+            const bool sure = (fabsf(u - rintf(u)) > margin) | (f2 <= zero_d2), count = in[v] & sure;
+            need |= in[v] & !sure ? 1u << v : 0u;
+            const uint32_t at = (slot == js + v ? rowself : row0 + row[v]) + (uint32_t)floor_i32(u);
+            atomicAdd(count ? &hist[at] : (unsigned *)smem + (threadIdx.x & 63u), count ? 1u : 0u);
+        }
+        if (__any(need != 0))
+#pragma unroll 1
+            for (int v = 0; v < U; v++)
+                if (need >> v & 1u) {
+                    double e = d2[0];
+                    uint32_t r = row[0];
+#pragma unroll
+                    for (int q = 1; q < U; q++) {
+                        e = q == v ? d2[q] : e;
+                        r = q == v ? row[q] : r;
+                    }
+                    const uint32_t bb = (uint32_t)bin_of(e, thr, (int)nbin, rminf, inv_drf);
+                    atomicAdd(&hist[(slot == js + v ? rowself : row0 + r) + bb], 1u);
+                }
+    };
+    if constexpr (SPLIT) {
+        // every second group of 32 j, from LDS (the wavefront's own); the next
+        // group (of this frame or the next t0's) is on its way meanwhile
+        const uint32_t lane = threadIdx.x & 63u, jl = lane & 31u, jw = 32u * (wave & 1u);
+        constexpr uint32_t KSTEP = SPLIT_WG / 128;
+        double *sx = (double *)(smem + a.stage) + wave * (STAGE_J / 8), *sy = sx + 32, *sz = sy + 32;
+        uint32_t *srow = (uint32_t *)(sz + 32);
+        uint32_t k = w.k0 + (wave >> 1);
+        double4 xn, xin;
+        uint32_t tn;
+        DevCell cn;
+        auto fetch_j = [&](uint64_t fj, uint32_t j0) {
+            const uint32_t j = min(j0 + jl, N - 1);
+            xn = a.pos[fj * N + j];
+            tn = (uint32_t)a.type_slot[j];
+        };
+        auto fetch_i = [&](uint32_t kk) {
+            const uint64_t fi = b.primo + (uint64_t)kk * a.skip;
+            xin = a.pos[fi * N + min(slot, N - 1)];
+            cn = load_cell(a.box + fi * 9);
+            fetch_j(fi + t, jw);
+        };
+        if (nact && k < w.k1) fetch_i(k);
+        for (; nact && k < w.k1; k += KSTEP) {
+            const double4 xi = xin;
+            const DevCell c = cn;
+            if (!(wave & 1u)) nt0++;
+            for (uint32_t j0 = jw; j0 < N; j0 += 64) {
+                sx[jl] = xn.x;
+                sy[jl] = xn.y;
+                sz[jl] = xn.z;
+                srow[jl] = tn * nbin;
+                if (j0 + 64 < N) fetch_j(b.primo + (uint64_t)k * a.skip + t, j0 + 64);
+                else if (k + KSTEP < w.k1) fetch_i(k + KSTEP);
+                wave_sync_lds();
+                const uint32_t nj = min(32u, N - j0);
+                if (active)
+                    for (uint32_t j = 0; j < nj; j += U) {
+                        double yx[U], yy[U], yz[U];
+                        uint32_t row[U];
+#pragma unroll
+                        for (int v = 0; v < U; v++) {
+                            yx[v] = sx[j + v];
+                            yy[v] = sy[j + v];
+                            yz[v] = sz[j + v];
+                            row[v] = srow[j + v];
+                        }
+                        pairs(xi, yx, yy, yz, row, j0 + j, nj - j, c);
+                    }
+                wave_sync_lds();
+            }
+            if (jw >= N && k + KSTEP < w.k1) fetch_i(k + KSTEP);
+        }
+    } else {
+        for (uint32_t k = w.k0; k < w.k1; k++) {
+            const uint64_t fi = b.primo + (uint64_t)k * a.skip;
+            const uint64_t fj = fi + t;
+            DevCell c = load_cell(a.box + fi * 9);
+            // in vector registers: the scalar ones hold the atoms loaded ahead
+            asm("" : "+v"(c.lh0), "+v"(c.lh1), "+v"(c.lh2), "+v"(c.L0), "+v"(c.L1), "+v"(c.L2));
+            if (TRI) asm("" : "+v"(c.xy), "+v"(c.xz), "+v"(c.yz));
+            const double4 *__restrict__ pj = a.pos + fj * N;
+            nt0++;
+            if (active) {
+                const double4 xi = a.pos[fi * N + slot];
+                // the next U atoms are loaded (scalar loads) before these are worked on
+                double4 xn[U];
+                uint32_t tn[U];
+                auto fetch = [&](uint32_t j) {
+#pragma unroll
+                    for (int v = 0; v < U; v++) {
+                        xn[v] = pj[min(j + v, N - 1)];
+                        tn[v] = (uint32_t)a.type_slot[min(j + v, N - 1)];
+                    }
+                };
+                fetch(0);
+                for (uint32_t j = 0; j < N; j += U) {
+                    double yx[U], yy[U], yz[U];
+                    uint32_t row[U];
+#pragma unroll
+                    for (int v = 0; v < U; v++) {
+                        yx[v] = xn[v].x;
+                        yy[v] = xn[v].y;
+                        yz[v] = xn[v].z;
+                        row[v] = tn[v] * nbin;
+                    }
+                    fetch(j + U);
+                    pairs(xi, yx, yy, yz, row, j, N - j, c);
                 }
             }
         }
     }
-    if ((threadIdx.x & 63u) == 0 && a.ncand && npairs) {
+    if ((threadIdx.x & 63u) == 0 && a.ncand && nact && nt0) {
+        const unsigned long long npairs = (unsigned long long)nact * N * nt0;
         atomicAdd(a.ncand + STAT_PAIRS_FP64, npairs);
         atomicAdd(a.ncand + STAT_PAIRS_ALL, npairs);
     }
     __syncthreads();
-    lds_flush(a, hist, w.block, t);
+    // rows to channels and a rotated start, as lds_flush_rows
+    unsigned long long *o = a.out + (uint64_t)w.block * a.out_block_stride + (uint64_t)t * nh;
+    const uint32_t rot = (blockIdx.x * 977u) % nh;
+    for (uint32_t k0 = threadIdx.x; k0 < nh; k0 += NTH) {
+        const uint32_t k = k0 + rot < nh ? k0 + rot : k0 + rot - nh;
+        const unsigned v = hist[k];
+        const uint32_t r = k / nbin, self = nt * nt;
+        const uint32_t ch = r < self ? (uint32_t)rowch[r] : (uint32_t)rowch[(r - self) * (nt + 1)] + a.half * nbin;
+        if (v) atomicAdd(o + ch + (k - r * nbin), (unsigned long long)v);
+    }
 }
 
 typedef short short2_t __attribute__((ext_vector_type(2)));
@@ -851,13 +1025,6 @@ __device__ __forceinline__ void uadd(unsigned long long &c, unsigned long long v
     }
 }
 
-__device__ __forceinline__ void wave_sync_lds() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
-
 typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
 
@@ -1005,8 +1172,8 @@ __global__ __launch_bounds__(WG, 4) void gofrt_cells_kernel(const GofrtCellArgs 
     extern __shared__ __align__(16) unsigned char smem[];
     const WgId id = decode_wg(a.ntiles, a.nlag, a.nwork, a.per_xcd);
     if (!id.valid) return;
-    const WorkItem w = a.work[id.work];
-    const BlockInfo b = a.blocks[w.block];
+    BlockInfo b;
+    const WorkItem w = work_item(a, id.work, b);
     const uint32_t t = a.lag0 + id.lagi * a.every;
     if (t >= b.leff) return;
     uint4 *j32 = (uint4 *)smem;                       // fractions of the tile's j, .w = type | slot << 8
@@ -1202,8 +1369,8 @@ __global__ __launch_bounds__(WG, CLUSTER ? 4 : 1) void gofrt_screened_kernel(con
     extern __shared__ unsigned char smem[];
     const WgId id = decode_wg(a.ntiles, a.nlag, a.nwork, a.per_xcd);
     if (!id.valid) return;
-    const WorkItem w = a.work[id.work];
-    const BlockInfo b = a.blocks[w.block];
+    BlockInfo b;
+    const WorkItem w = work_item(a, id.work, b);
     const uint32_t t = a.lag0 + id.lagi * a.every;
     if (t >= b.leff) return;
     uint4 *fi_lds = (uint4 *)smem;                          // [WG]
@@ -1801,11 +1968,12 @@ int choose_form(anl_gofrt *g) {
 
 // Whether the automatic form of a trajectory with a changing cell takes
 // gofrt_cells_kernel: the screen's preconditions hold in every frame's cell.
-// From 256 atoms, one full tile of i (40 t0, 10 lags, plain -> this: 256 atoms
-// at rmax 0.3 and 0.49 of the cell length 218 -> 162 and 238 -> 188 us, 3,000
-// at 0.49, tilted, 8.33 -> 4.12 ms, 10,000 at 0.2 49.5 -> 11.2 ms); below,
-// most lanes of the tile idle and the launch is what a call costs.
-constexpr uint64_t CELLS_MIN_ATOMS = 256;
+// From 769 atoms (more than three tiles of i; 40 t0, 10 lags, plain -> this at
+// rmax 0.3 and 0.49 of the cell length: 600 atoms 243 -> 285 us (0.15) and 342
+// -> 442, 800 481 -> 389 and 504 -> 568, 1,000 658 -> 491 and 715 -> 679, 2,000
+// at 0.49 2.29 -> 1.84 ms, 3,000 tilted 6.16 -> 4.08, 10,000 at 0.2 42.5 ->
+// 11.2); below, the plain form's smaller tiles fill the chip better.
+constexpr uint64_t CELLS_MIN_ATOMS = 769;
 bool use_cells(anl_gofrt *g) {
     anl_traj *tr = g->tr;
     if (g->form != ANL_GOFRT_AUTO || tr->box_const || tr->N < CELLS_MIN_ATOMS) return false;
@@ -1885,20 +2053,40 @@ bool clusters_fit(anl_gofrt *g, float rho_cap) {
 
 struct Launch {
     std::vector<BlockInfo> blocks;
-    std::vector<WorkItem> work;
+    std::vector<WorkItem> work;   // empty for one block: [k0, k1) in chunks, from the arguments
+    uint32_t k0 = 0, k1 = 0, chunk = 1;
+    uint32_t nwork = 0;
     uint32_t leff_max = 0;
+    uint32_t tile = WG;           // i atoms of a workgroup
 };
+
+// The plain FP64 form of a system of at most FP64_SPLIT_ATOMS atoms gives a
+// workgroup 64 i atoms and each pair of its eight wavefronts its own t0: with
+// 256 i most lanes, or whole wavefronts, would idle, and a workgroup's flush of
+// the histogram would serve one t0 only.  60 t0 x 12 lags, 256 i -> this: 64
+// atoms 54 -> 46 us a call, 300 217 -> 181, 600 551 -> 511, 800 (tilted) 1,137
+// -> 1,016, 1,000 1,129 -> 1,170.
+constexpr uint64_t FP64_SPLIT_ATOMS = 768;
+// LDS of the plain form without the staged j
+size_t fp64_lds(const anl_gofrt *g) {
+    const size_t nt = g->tr->nt;
+    return (g->nbin + 1) * sizeof(double) + nt * nt * sizeof(int) + (size_t)nch_of(g->tr) * g->nbin * sizeof(unsigned);
+}
+size_t fp64_stage(const anl_gofrt *g) { return (fp64_lds(g) + 15) / 16 * 16; }
 
 // Splits every block's t0 range into chunks: a chunk bounds the LDS counters
 // (each t0 adds at most 256*N to one bin: 256*N*chunk < 2^32) and sets the
 // work per workgroup (the tuned number of pair evaluations), finer where the
 // launch would not fill the chip.
-Launch plan(anl_gofrt *g, const uint64_t *primo, const uint32_t *n, uint32_t nblocks, int single_k) {
+Launch plan(anl_gofrt *g, const uint64_t *primo, const uint32_t *n, uint32_t nblocks) {
     Launch L;
     const uint64_t N = g->tr->N;
+    const bool split = choose_form(g) == ANL_GOFRT_FP64 && N <= FP64_SPLIT_ATOMS &&
+                       fp64_stage(g) + SPLIT_WG / 64 * STAGE_J <= 160 * 1024 && !use_cells(g);
+    if (split) L.tile = 64;
     uint64_t cap = (0xFFFFFFFFull / ((uint64_t)WG * N));
     if (cap < 1) cap = 1;
-    uint64_t target = g->tune.pairs_per_wg / ((uint64_t)WG * N);
+    uint64_t target = g->tune.pairs_per_wg / ((uint64_t)L.tile * N);
     if (target < 1) target = 1;
     const uint64_t chunk = std::min(cap, target);
     // a launch of fewer than 16 workgroups per CU (4,096 in all) leaves SIMDs
@@ -1907,26 +2095,29 @@ Launch plan(anl_gofrt *g, const uint64_t *primo, const uint32_t *n, uint32_t nbl
     // changes no result).  2,048 -> 4,096, rounded up: 1,000 atoms, 150 t0, 51
     // lags 4.25 -> 4.02 ms; 3,000 atoms, 20 t0, 10 lags 2.16 -> 1.76; 8,192
     // gains nothing more
-    const uint64_t ntiles = (N + WG - 1) / WG;
+    const uint64_t ntiles = (N + L.tile - 1) / L.tile;
     const uint64_t want = (4096 + nblocks - 1) / nblocks;
     for (uint32_t bi = 0; bi < nblocks; bi++) {
         uint32_t leff = (n[bi] < g->lmax || g->lmax == 0) ? n[bi] : g->lmax;
         L.blocks.push_back(BlockInfo{primo[bi], leff, 0});
         L.leff_max = std::max(L.leff_max, leff);
-        if (single_k >= 0) {
-            L.work.push_back(WorkItem{bi, (uint32_t)single_k, (uint32_t)single_k + 1, 0});
-            continue;
-        }
         uint32_t n0 = (n[bi] + g->skip - 1) / g->skip;  // t0 = 0, skip, ... < n
         const uint64_t units = ntiles * std::max<uint64_t>(1, (leff + g->every - 1) / g->every);
         uint64_t chunk_b = chunk;
         if (units * ((n0 + chunk - 1) / chunk) < want) {
             const uint64_t items = (want + units - 1) / units;
-            chunk_b = std::min(chunk, std::max<uint64_t>(1, n0 / items));
+            chunk_b = std::min(chunk, std::max<uint64_t>(split ? std::min<uint64_t>(4, n0) : 1, n0 / items));
+        }
+        if (nblocks == 1) {
+            L.k1 = n0;
+            L.chunk = (uint32_t)std::max<uint64_t>(1, chunk_b);
+            L.nwork = (uint32_t)((n0 + (uint64_t)L.chunk - 1) / L.chunk);
+            return L;
         }
         for (uint64_t k = 0; k < n0; k += chunk_b)
             L.work.push_back(WorkItem{bi, (uint32_t)k, (uint32_t)std::min<uint64_t>(n0, k + chunk_b), 0});
     }
+    L.nwork = (uint32_t)L.work.size();
     return L;
 }
 
@@ -1957,20 +2148,18 @@ struct GofrtPrepared {
     int unroll = 4;
     int cluster = 0;  // as GofrtTuning::cluster, 0 when the cluster screen cannot be used
     bool cells = false;  // gofrt_cells_kernel
+    bool split = false;  // gofrt_fp64_kernel: a t0 per wavefront
     // device work list and block table owned by this launch (block engine)
     BlockInfo *own_blocks = nullptr;
     WorkItem *own_work = nullptr;
 };
 
-__global__ void fill_u64_kernel(unsigned long long *__restrict__ p, uint64_t len) {
-    uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+// Clears the output and the launch counters (a kernel: the launch may be
+// captured into a graph).
+__global__ void clear_kernel(unsigned long long *__restrict__ p, uint64_t len, unsigned long long *__restrict__ stat) {
+    const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < len) p[i] = 0ull;
-}
-
-static void zero_u64(unsigned long long *p, uint64_t len, hipStream_t s) {
-    if (len == 0) return;
-    hipLaunchKernelGGL(fill_u64_kernel, dim3((unsigned)((len + 255) / 256)), dim3(256), 0, s, p, len);
-    ANL_HIP(hipGetLastError());
+    if (i < NSTAT) stat[i] = 0ull;
 }
 
 // own = true: the work list and block table go to buffers owned by the
@@ -1985,7 +2174,9 @@ GofrtPrepared gofrt_prepare(anl_gofrt *g, const Launch &L, uint64_t out_len, int
     if (form == ANL_GOFRT_SCREENED) build_frac16(tr, s);
     BlockInfo *d_blocks = nullptr;
     WorkItem *d_work = nullptr;
-    if (own) {
+    if (L.work.empty()) {
+        if (!own) ANL_HIP(hipDeviceSynchronize());  // the counters (d_ncand) belong to one launch at a time
+    } else if (own) {
         ANL_HIP(hipMalloc(&P.own_blocks, std::max<size_t>(1, L.blocks.size()) * sizeof(BlockInfo)));
         d_blocks = P.own_blocks;
         hipError_t e = hipMalloc(&P.own_work, std::max<size_t>(1, L.work.size()) * sizeof(WorkItem));
@@ -2013,9 +2204,11 @@ GofrtPrepared gofrt_prepare(anl_gofrt *g, const Launch &L, uint64_t out_len, int
         d_blocks = g->d_blocks;
         d_work = g->d_work;
     }
-    ANL_HIP(hipMemcpyAsync(d_blocks, L.blocks.data(), L.blocks.size() * sizeof(BlockInfo), hipMemcpyHostToDevice, s));
-    ANL_HIP(hipMemcpyAsync(d_work, L.work.data(), L.work.size() * sizeof(WorkItem), hipMemcpyHostToDevice, s));
-    ANL_HIP(hipStreamSynchronize(s));  // the host vectors die with L
+    if (!L.work.empty()) {
+        ANL_HIP(hipMemcpyAsync(d_blocks, L.blocks.data(), L.blocks.size() * sizeof(BlockInfo), hipMemcpyHostToDevice, s));
+        ANL_HIP(hipMemcpyAsync(d_work, L.work.data(), L.work.size() * sizeof(WorkItem), hipMemcpyHostToDevice, s));
+        ANL_HIP(hipStreamSynchronize(s));  // the host vectors die with L
+    }
 
     GofrtArgs &a = P.a;
     a.pos = tr->pos;
@@ -2030,6 +2223,10 @@ GofrtPrepared gofrt_prepare(anl_gofrt *g, const Launch &L, uint64_t out_len, int
     a.chan = g->d_chan;
     a.work = d_work;
     a.blocks = d_blocks;
+    a.block0 = L.blocks.empty() ? BlockInfo{0, 0, 0} : L.blocks[0];
+    a.wk0 = L.k0;
+    a.wk1 = L.k1;
+    a.chunk = L.chunk;
     a.N = tr->N;
     a.nt = tr->nt;
     a.nbin = g->nbin;
@@ -2041,6 +2238,12 @@ GofrtPrepared gofrt_prepare(anl_gofrt *g, const Launch &L, uint64_t out_len, int
     a.lo = g->lo;
     a.rmax2 = g->rmax2;
     a.Tn = g->thr[g->nbin];
+    a.d2_end = std::min(std::nextafter(g->rmax2, HUGE_VAL), a.Tn);
+    // (float)d2, the square root, the subtraction, 1/dr and the product round
+    // at most 2^-23 of a value below umax = nbin + 1 + rmin/dr each, as does
+    // the reference's own u
+    a.bin_margin = (float)(2.0 * 6.0 * std::ldexp(1.0, -23) * (g->nbin + 1.0 + g->rmin / g->dr) + 1e-6);
+    a.zero_d2 = g->rmin == 0.0 && g->thr[1] > 0x1p-140 ? 0.0f : -1.0f;
     a.rminf = (float)g->rmin;
     a.inv_drf = (float)(1.0 / g->dr);
     a.threshold = form == ANL_GOFRT_SCREENED ? tr->screen_cache.threshold : 0;
@@ -2079,14 +2282,16 @@ GofrtPrepared gofrt_prepare(anl_gofrt *g, const Launch &L, uint64_t out_len, int
         a.inv_w16 = form == ANL_GOFRT_SCREENED ? (float)(65536.0 / tr->screen_cache.wmin * (1 + 1e-6)) : 0.0f;
         a.smin16 = form == ANL_GOFRT_SCREENED ? (float)(tr->screen_cache.smin * std::ldexp(1.0, -16) * (1 - 1e-6)) : 0.0f;
     }
-    const uint32_t ntiles = (uint32_t)((tr->N + WG - 1) / WG);
+    const uint32_t ntiles = (uint32_t)((tr->N + L.tile - 1) / L.tile);
+    P.split = L.tile != WG;
     const uint32_t nlag = nlag_force ? nlag_force : (L.leff_max + g->every - 1) / g->every;
     a.lag0 = lag0;
-    const uint64_t total = (uint64_t)ntiles * nlag * L.work.size();
+    const uint64_t total = (uint64_t)ntiles * nlag * L.nwork;
     const uint64_t per = (total + 7) / 8;
     if (8 * per >= (1ull << 32)) fail(ANL_ERR_ARG, "too many workgroups (reduce the trajectory block)");
-    // channel table (FP64 form) or histogram-offset table (screened form, two
-    // entries per type pair), bin-edge table, histogram
+    // histogram-offset table (screened forms: two entries per type pair; the
+    // plain form, whose room stays as it was, reads a.chan when it flushes),
+    // bin-edge table, histogram
     const size_t common = (g->nbin + 1) * sizeof(double) +
                           (size_t)(form == ANL_GOFRT_FP64 ? 1 : 2) * tr->nt * tr->nt * sizeof(int) +
                           (size_t)a.nch * g->nbin * sizeof(unsigned);
@@ -2098,7 +2303,7 @@ GofrtPrepared gofrt_prepare(anl_gofrt *g, const Launch &L, uint64_t out_len, int
     const bool cells = form == ANL_GOFRT_FP64 && cells_lds <= 160 * 1024 && use_cells(g);
     a.ntiles = ntiles;
     a.nlag = nlag;
-    a.nwork = (uint32_t)L.work.size();
+    a.nwork = L.nwork;
     const bool remap = g->tune.xcd && (form == ANL_GOFRT_SCREENED || cells);
     a.per_xcd = remap ? (uint32_t)per : 0u;
     P.grid = dim3((uint32_t)(remap ? 8 * per : total));
@@ -2109,6 +2314,11 @@ GofrtPrepared gofrt_prepare(anl_gofrt *g, const Launch &L, uint64_t out_len, int
                             screened_lds(qcl, colc) <= 160 * 1024 && (g->tuned || clusters_fit(g, a.rho_cap));
     P.lds = form == ANL_GOFRT_FP64 ? common : (cluster_ok ? screened_lds(qcl, colc) : screened_lds(SQCAP, false));
     if (P.lds > 160 * 1024) fail(ANL_ERR_ARG, "histogram does not fit in LDS (reduce nbin or types)");
+    P.lds = std::max<size_t>(P.lds, 64 * sizeof(unsigned));  // the plain form adds 0 to words 0 .. 63
+    if (P.split) {
+        a.stage = (uint32_t)fp64_stage(g);
+        P.lds = fp64_stage(g) + SPLIT_WG / 64 * STAGE_J;
+    }
     if (cells) {
         P.cells = true;
         P.lds = cells_lds;
@@ -2125,16 +2335,18 @@ GofrtPrepared gofrt_prepare(anl_gofrt *g, const Launch &L, uint64_t out_len, int
 void gofrt_enqueue(anl_gofrt *g, const GofrtPrepared &P, unsigned long long *out, hipStream_t s) {
     GofrtArgs a = P.a;
     a.out = out;
-    zero_u64(out, P.out_len, s);
-    zero_u64(g->d_ncand, NSTAT, s);
+    hipLaunchKernelGGL(clear_kernel, dim3((unsigned)((std::max<uint64_t>(P.out_len, NSTAT) + 255) / 256)), dim3(256), 0, s,
+                       out, P.out_len, g->d_ncand);
+    ANL_HIP(hipGetLastError());
     if (P.grid.x == 0) return;
     if (P.cells) {
         const GofrtCellArgs c{a, g->d_cells};
         if (P.triclinic) hipLaunchKernelGGL(gofrt_cells_kernel<true>, P.grid, dim3(WG), P.lds, s, c);
         else hipLaunchKernelGGL(gofrt_cells_kernel<false>, P.grid, dim3(WG), P.lds, s, c);
     } else if (P.form == ANL_GOFRT_FP64) {
-        if (P.triclinic) hipLaunchKernelGGL(gofrt_fp64_kernel<true>, P.grid, dim3(WG), P.lds, s, a);
-        else hipLaunchKernelGGL(gofrt_fp64_kernel<false>, P.grid, dim3(WG), P.lds, s, a);
+        auto kernel = P.triclinic ? (P.split ? gofrt_fp64_kernel<true, true> : gofrt_fp64_kernel<true, false>)
+                                  : (P.split ? gofrt_fp64_kernel<false, true> : gofrt_fp64_kernel<false, false>);
+        hipLaunchKernelGGL(kernel, P.grid, dim3(P.split ? SPLIT_WG : WG), P.lds, s, a);
     } else {
         const bool u8 = P.unroll == 8;
 #define ANL_SCREENED(T, U, C, K) hipLaunchKernelGGL((gofrt_screened_kernel<T, U, C, K>), P.grid, dim3(WG), P.lds, s, a)
@@ -2168,7 +2380,7 @@ namespace anl {
 void *gofrt_prepare_blocks(anl_gofrt *g, const uint64_t *primo, const uint32_t *n, uint32_t nblocks,
                            uint32_t *leff_max, hipStream_t s) {
     check_lengths(g, primo, n, nblocks);
-    Launch L = plan(g, primo, n, nblocks, -1);
+    Launch L = plan(g, primo, n, nblocks);
     const uint64_t len = (uint64_t)nblocks * L.leff_max * nch_of(g->tr) * g->nbin;
     auto *P = new GofrtPrepared(gofrt_prepare(g, L, len, INT32_MIN, INT32_MAX, s, 0, 0, true));
     if (leff_max) *leff_max = L.leff_max;
@@ -2196,6 +2408,51 @@ void launch(anl_gofrt *g, const Launch &L, unsigned long long *out, uint64_t out
             hipStream_t s, uint32_t lag0 = 0, uint32_t nlag_force = 0) {
     GofrtPrepared P = gofrt_prepare(g, L, out_len, a0, a1, s, lag0, nlag_force);
     gofrt_enqueue(g, P, out, s);
+}
+
+__global__ void copy_out_kernel(const unsigned long long *__restrict__ src, uint64_t len,
+                                unsigned long long *__restrict__ dst) {
+    const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < len) dst[i] = src[i];
+}
+
+// A launch whose counts go to the host: take(counts, first, n) in order, once
+// per piece.  The device and pinned memory are the trajectory's pooled
+// workspace.  Up to 512 KiB a kernel writes the pinned memory itself: the copy
+// engine's start costs more than the bytes (192 KB: 20 us less per call); a
+// large output passes through 8 MiB at a time.
+template <class Take>
+void launch_to_host(anl_gofrt *g, const Launch &L, uint64_t len, int a0, int a1, uint32_t lag0, uint32_t nlag_force,
+                    Take take) {
+    const uint64_t piece = std::min<uint64_t>(len, (8u << 20) / sizeof(unsigned long long));
+    ScratchLease w(g->tr->scratch, len * sizeof(unsigned long long), piece * sizeof(unsigned long long));
+    auto *d = (unsigned long long *)w.s.dev, *h = (unsigned long long *)w.s.pin;
+    hipStream_t s = 0;
+    try {
+        launch(g, L, d, len, a0, a1, s, lag0, nlag_force);
+        for (uint64_t at = 0; at < len; at += piece) {
+            const uint64_t n = std::min(piece, len - at);
+            if (n <= (512u << 10) / sizeof(unsigned long long)) {
+                hipLaunchKernelGGL(copy_out_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, d + at, n, h);
+                ANL_HIP(hipGetLastError());
+            } else {
+                ANL_HIP(hipMemcpyAsync(h, d + at, n * sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
+            }
+            ANL_HIP(hipStreamSynchronize(s));
+            take(h, at, n);
+        }
+    } catch (...) {
+        (void)hipStreamSynchronize(s);  // the workspace goes back unused
+        throw;
+    }
+}
+
+template <class Take>
+void calculate_to_host(anl_gofrt *g, uint64_t primo, Take take) {
+    ensure_device();
+    check_lengths(g, &primo, &g->n, 1);
+    const uint64_t len = (uint64_t)g->leff * nch_of(g->tr) * g->nbin;
+    if (len) launch_to_host(g, plan(g, &primo, &g->n, 1), len, INT32_MIN, INT32_MAX, 0, 0, take);
 }
 
 }  // namespace
@@ -2298,7 +2555,7 @@ int anl_gofrt_calculate_async(anl_gofrt *g, uint64_t primo, uint64_t *counts_dev
         if (!g || !counts_dev) fail(ANL_ERR_ARG, "null pointer passed to anl_gofrt_calculate_async");
         ensure_device();
         check_lengths(g, &primo, &g->n, 1);
-        Launch L = plan(g, &primo, &g->n, 1, -1);
+        Launch L = plan(g, &primo, &g->n, 1);
         if (L.leff_max == 0) return;
         uint64_t len = (uint64_t)L.leff_max * nch_of(g->tr) * g->nbin;
         launch(g, L, (unsigned long long *)counts_dev, len, INT32_MIN, INT32_MAX, (hipStream_t)stream);
@@ -2308,22 +2565,17 @@ int anl_gofrt_calculate_async(anl_gofrt *g, uint64_t primo, uint64_t *counts_dev
 int anl_gofrt_calculate(anl_gofrt *g, uint64_t primo, uint64_t *counts_host) {
     return guard([&] {
         if (!g || !counts_host) fail(ANL_ERR_ARG, "null pointer passed to anl_gofrt_calculate");
-        ensure_device();
-        check_lengths(g, &primo, &g->n, 1);
-        uint64_t len = (uint64_t)g->leff * nch_of(g->tr) * g->nbin;
-        if (len == 0) return;
-        unsigned long long *d = nullptr;
-        ANL_HIP(hipMalloc(&d, len * sizeof(unsigned long long)));
-        try {
-            Launch L = plan(g, &primo, &g->n, 1, -1);
-            launch(g, L, d, len, INT32_MIN, INT32_MAX, 0);
-            ANL_HIP(hipMemcpy(counts_host, d, len * sizeof(unsigned long long), hipMemcpyDeviceToHost));
-
-        } catch (...) {
-            (void)hipFree(d);
-            throw;
-        }
-        (void)hipFree(d);
+        calculate_to_host(g, primo, [&](const unsigned long long *c, uint64_t at, uint64_t n) {
+            std::memcpy(counts_host + at, c, n * sizeof(uint64_t));
+        });
+    });
+}
+int anl_gofrt_calculate_scaled(anl_gofrt *g, uint64_t primo, double scale, double *out_host) {
+    return guard([&] {
+        if (!g || !out_host) fail(ANL_ERR_ARG, "null pointer passed to anl_gofrt_calculate_scaled");
+        calculate_to_host(g, primo, [&](const unsigned long long *c, uint64_t at, uint64_t n) {
+            for (uint64_t k = 0; k < n; k++) out_host[at + k] = (double)c[k] * scale;
+        });
     });
 }
 
@@ -2339,19 +2591,10 @@ int anl_gofrt_calc_single_th(anl_gofrt *g, int t, int imedia, int a0, int a1, ui
         Launch L;
         L.leff_max = g->leff;
         L.blocks.push_back(BlockInfo{primo + (uint64_t)imedia, g->leff, 0});
-        L.work.push_back(WorkItem{0, 0, 1, 0});
-        unsigned long long *d = nullptr;
-        ANL_HIP(hipMalloc(&d, len * sizeof(unsigned long long)));
-        std::vector<uint64_t> h(len);
-        try {
-            launch(g, L, d, len, a0, a1, 0, (uint32_t)t, 1);
-            ANL_HIP(hipMemcpy(h.data(), d, len * sizeof(unsigned long long), hipMemcpyDeviceToHost));
-        } catch (...) {
-            (void)hipFree(d);
-            throw;
-        }
-        (void)hipFree(d);
-        for (uint64_t k = 0; k < len; k++) counts_host[k] += h[k];
+        L.k1 = L.nwork = 1;
+        launch_to_host(g, L, len, a0, a1, (uint32_t)t, 1, [&](const unsigned long long *c, uint64_t at, uint64_t n) {
+            for (uint64_t k = 0; k < n; k++) counts_host[at + k] += c[k];
+        });
     });
 }
 
@@ -2362,7 +2605,7 @@ int anl_gofrt_calculate_blocks_async(anl_gofrt *g, const uint64_t *primo, const 
             fail(ANL_ERR_ARG, "bad arguments to anl_gofrt_calculate_blocks_async");
         ensure_device();
         check_lengths(g, primo, n, nblocks);
-        Launch L = plan(g, primo, n, nblocks, -1);
+        Launch L = plan(g, primo, n, nblocks);
         uint64_t len = (uint64_t)nblocks * L.leff_max * nch_of(g->tr) * g->nbin;
         launch(g, L, (unsigned long long *)counts_dev, len, INT32_MIN, INT32_MAX, (hipStream_t)stream);
     });
@@ -2483,7 +2726,8 @@ int anl_gofrt_autotune(anl_gofrt *g, uint64_t primo, uint32_t nlag_probe, const 
         // probe lags: at least nlag_probe, and enough for >= 4096 workgroups
         // (several waves of residency), so that the probe behaves like the run
         const uint32_t nlag_all = (g->leff + g->every - 1) / g->every;
-        const uint64_t per_lag = (uint64_t)((g->tr->N + WG - 1) / WG) * plan(g, &primo, &g->n, 1, -1).work.size();
+        const Launch L1 = plan(g, &primo, &g->n, 1);
+        const uint64_t per_lag = (uint64_t)((g->tr->N + L1.tile - 1) / L1.tile) * L1.nwork;
         const uint64_t fill = (4096 + per_lag - 1) / std::max<uint64_t>(per_lag, 1);
         const uint32_t nlag = (uint32_t)std::max<uint64_t>(
             1, std::min<uint64_t>(std::max<uint64_t>(nlag_probe, fill), nlag_all));
@@ -2508,7 +2752,7 @@ int anl_gofrt_autotune(anl_gofrt *g, uint64_t primo, uint32_t nlag_probe, const 
             ANL_HIP(hipEventCreate(&e1));
             for (uint32_t c = 0; c < ncand; c++) {
                 set(c);
-                Launch L = plan(g, &primo, &g->n, 1, -1);
+                Launch L = plan(g, &primo, &g->n, 1);
                 GofrtPrepared P = gofrt_prepare(g, L, len, INT32_MIN, INT32_MAX, 0, 0, nlag);
                 gofrt_enqueue(g, P, d, 0);
                 ANL_HIP(hipEventRecord(e0, 0));

@@ -553,9 +553,13 @@ class Gofrt : public VectorOp<Gofrt<TFLOAT, T>, TFLOAT> {
         calc_init((int)primo);
         // timesteps primo .. primo + n - 1 + leff - 1 must be on the device
         const size_t off = traiettoria->window_offset(primo, (size_t)ntimesteps + leff - 1);
-        std::vector<uint64_t> counts(data_length);
-        anl_check(anl_gofrt_calculate(h(), off, counts.data()));
-        for (unsigned int k = 0; k < data_length; k++) vdata[k] = (TFLOAT)counts[k] * incr;
+        if constexpr (std::is_same<TFLOAT, double>::value) {
+            anl_check(anl_gofrt_calculate_scaled(h(), off, incr, vdata));
+        } else {
+            std::vector<uint64_t> counts(data_length);
+            anl_check(anl_gofrt_calculate(h(), off, counts.data()));
+            for (unsigned int k = 0; k < data_length; k++) vdata[k] = (TFLOAT)counts[k] * incr;
+        }
         calc_end();
     }
     void calc_init(int primo) {  // gofrt.cpp:74-93

@@ -85,6 +85,61 @@ __device__ __forceinline__ void min_image_ref(double &x0, double &x1, double &x2
     }
 }
 
+// min_image_ref of U pairs side by side: every step is branch-free (s * L is L
+// with the sign of x: exact; a lane that does not need the step keeps its
+// value), and an axis is stepped again while some lane of the wavefront needs
+// it, so that the U chains overlap.  The same operations in the same order.
+template <bool TRI, int U>
+__device__ __forceinline__ void min_image_batch(double (&x0)[U], double (&x1)[U], double (&x2)[U], const DevCell &c) {
+    auto flip = [](double v, double sign) {  // v, or -v where sign is negative
+        return __longlong_as_double(__double_as_longlong(v) ^ (__double_as_longlong(sign) & (long long)0x8000000000000000ull));
+    };
+    int guard = 0;  // as in min_image_ref
+    unsigned long long more;
+#pragma clang loop unroll(disable)
+    do {
+        more = 0;
+#pragma unroll
+        for (int v = 0; v < U; v++) {
+            const bool t = fabs(x2[v]) > c.lh2;
+            const double s = x2[v], n2 = s - copysign(c.L2, s);
+            x2[v] = t ? n2 : s;
+            if (TRI) {
+                const double n1 = x1[v] - flip(c.yz, s), n0 = x0[v] - flip(c.xz, s);
+                x1[v] = t ? n1 : x1[v];
+                x0[v] = t ? n0 : x0[v];
+            }
+            more |= __ballot(fabs(x2[v]) > c.lh2);
+        }
+    } while (more && ++guard < (1 << 20));
+#pragma clang loop unroll(disable)
+    do {
+        more = 0;
+#pragma unroll
+        for (int v = 0; v < U; v++) {
+            const bool t = fabs(x1[v]) > c.lh1;
+            const double s = x1[v], n1 = s - copysign(c.L1, s);
+            x1[v] = t ? n1 : s;
+            if (TRI) {
+                const double n0 = x0[v] - flip(c.xy, s);
+                x0[v] = t ? n0 : x0[v];
+            }
+            more |= __ballot(fabs(x1[v]) > c.lh1);
+        }
+    } while (more && ++guard < (2 << 20));
+#pragma clang loop unroll(disable)
+    do {
+        more = 0;
+#pragma unroll
+        for (int v = 0; v < U; v++) {
+            const bool t = fabs(x0[v]) > c.lh0;
+            const double s = x0[v], n0 = s - copysign(c.L0, s);
+            x0[v] = t ? n0 : s;
+            more |= __ballot(fabs(x0[v]) > c.lh0);
+        }
+    } while (more && ++guard < (3 << 20));
+}
+
 // basetrajectory.h:200-219: x = xi - xj, minimum image, d2 = 0 + x0^2 + x1^2
 // + x2^2 with separate products and sums.
 __device__ __forceinline__ double d2_of(double x0, double x1, double x2) {

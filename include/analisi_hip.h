@@ -38,7 +38,7 @@ extern "C" {
 #define ANL_GOFRT_SCREENED 1   /* 16-bit fixed-point screen of every pair, exact FP64
                                   evaluation of every candidate (same counts) */
 #define ANL_GOFRT_AUTO 2       /* SCREENED when its preconditions hold (in a changing cell: in every
-                                * frame's, from 256 atoms), else FP64 */
+                                * frame's, from 769 atoms), else FP64 */
 
 /* Message of the last failed call on this thread ("" if none). */
 const char *anl_last_error(void);
@@ -82,6 +82,8 @@ int anl_gofrt_reset(anl_gofrt *g, uint32_t n, uint32_t *leff_out);
 /* Gofrt::calculate(primo): whole (lags x t0 x ordered pairs) nest in one
  * launch; counts_host receives [leff][nch][nbin] uint64. */
 int anl_gofrt_calculate(anl_gofrt *g, uint64_t primo, uint64_t *counts_host);
+/* The same, out_host[k] = (double)counts[k] * scale. */
+int anl_gofrt_calculate_scaled(anl_gofrt *g, uint64_t primo, double scale, double *out_host);
 /* Same, device output (counts_dev zeroed and filled), enqueued on stream
  * (a hipStream_t, NULL = default stream), no host synchronisation. */
 int anl_gofrt_calculate_async(anl_gofrt *g, uint64_t primo, uint64_t *counts_dev, void *stream);

@@ -31,10 +31,10 @@ def _case(seed, N, F, L, tilt, fractions=(0.5, 0.3, 0.2), shift=0.0, breathe=0.0
     return ot, capi.DeviceTrajectory(ot.pos, ot.box, ot.type_id, ot.ntypes, ot.cm)
 
 
-@pytest.mark.parametrize("N", [256, 257, 319, 320, 511, 513, 1030])
+@pytest.mark.parametrize("N", [769, 831, 832, 1023, 1024, 1025])
 @pytest.mark.parametrize("tilt,shift", [(None, 0.0), (None, 41.0), ([1.5, -1.2, 0.9], 0.0), ([-1.4, 1.1, 1.3], -37.0)])
 def test_counts(N, tilt, shift):
-    ot, dt = _case(5, N, 12, 15.0, tilt, shift=shift)
+    ot, dt = _case(5, N, 12, 17.0, tilt, shift=shift)
     for rmin, rmax, nbin, skip, every, n, primo in [(0.0, 6.5, 71, 1, 1, 6, 0), (0.4, 5.0, 40, 2, 2, 7, 1)]:
         ref, _ = O.gofrt(ot, rmin, rmax, nbin, 5, 8, skip, every, n, primo, want_vdata=False)
         g = capi.DeviceGofrt(dt, rmin, rmax, nbin, 5, skip, every)
@@ -64,10 +64,10 @@ def test_far_groups_are_skipped():
 
 
 def test_atom_ranges_and_blocks():
-    ot, dt = _case(7, 400, 30, 16.0, [1.0, 0.8, -0.7])
+    ot, dt = _case(7, 800, 30, 16.0, [1.0, 0.8, -0.7])
     g = capi.DeviceGofrt(dt, 0.2, 6.0, 33, 6)
     g.reset(9)
-    for t, im, a0, a1 in [(0, 0, 0, 400), (3, 5, 17, 18), (5, 2, 100, 333), (1, 8, 399, 400), (2, 1, 50, 50)]:
+    for t, im, a0, a1 in [(0, 0, 0, 800), (3, 5, 17, 18), (5, 2, 100, 333), (1, 8, 799, 800), (2, 1, 50, 50)]:
         c = np.zeros((6, 12, 33), np.uint64)
         O.gofrt_single(ot, 0.2, 6.0, 33, 6, t, im, a0, a1, 2, c)
         assert np.array_equal(g.calc_single_th(t, im, a0, a1, 2), c), (t, im, a0, a1)
@@ -84,7 +84,7 @@ def test_atom_ranges_and_blocks():
 def test_pairs_at_bin_edges():
     """Pairs within ulps of every bin edge and of rmax, in a cell that differs
     from frame to frame."""
-    rmax, nbin, N = 5.0, 25, 300
+    rmax, nbin, N = 5.0, 25, 800
     rng = np.random.default_rng(8)
     box = np.tile(synth.lammps_box(14.0), (3, 1))
     box[1, 1] = 14.001
@@ -105,7 +105,7 @@ def test_pairs_at_bin_edges():
 
 
 def test_what_stays_with_the_plain_form():
-    ot, dt = _case(9, 300, 8, 12.0, None)
+    ot, dt = _case(9, 900, 8, 12.0, None)
     g = capi.DeviceGofrt(dt, 0.0, 6.2, 30, 2)       # over half of some frame's shortest edge
     g.reset(3)
     ref, _ = O.gofrt(ot, 0.0, 6.2, 30, 2, 4, 1, 1, 3, 0, want_vdata=False)
@@ -114,7 +114,7 @@ def test_what_stays_with_the_plain_form():
     s.reset(3)
     with pytest.raises(capi.AnlError, match="the cell changes along the trajectory"):
         s.calculate(0)
-    ot, dt = _case(9, 255, 8, 12.0, None)
+    ot, dt = _case(9, 768, 8, 12.0, None)
     g = capi.DeviceGofrt(dt, 0.0, 4.0, 30, 2)
     g.reset(3)
     ref, _ = O.gofrt(ot, 0.0, 4.0, 30, 2, 4, 1, 1, 3, 0, want_vdata=False)
