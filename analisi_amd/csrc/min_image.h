@@ -140,6 +140,15 @@ __device__ __forceinline__ void min_image_batch(double (&x0)[U], double (&x1)[U]
     } while (more && ++guard < (3 << 20));
 }
 
+template <bool TRI>
+__device__ __forceinline__ void min_image_one(double &x0, double &x1, double &x2, const DevCell &c) {
+    double a0[1] = {x0}, a1[1] = {x1}, a2[1] = {x2};
+    min_image_batch<TRI, 1>(a0, a1, a2, c);
+    x0 = a0[0];
+    x1 = a1[0];
+    x2 = a2[0];
+}
+
 // basetrajectory.h:200-219: x = xi - xj, minimum image, d2 = 0 + x0^2 + x1^2
 // + x2^2 with separate products and sums.
 __device__ __forceinline__ double d2_of(double x0, double x1, double x2) {

@@ -137,78 +137,84 @@ __device__ __forceinline__ void direction(double &x0, double &x1, double &x2) {
     x2 = sp;
 }
 
+// The expansion's loops are unrolled for two ranges of lmax: up to 6 (the order
+// parameters' usual l) and up to the largest.
+constexpr int SPH_LM_LOW = 6;
+
 // (specialfunctions.h:11-22, 262-360): P_l^m for l = m..lmax and
 // cos/sin(m phi), written to y[l*l + l + m] (cos) and y[l*l + l - m] (sin);
-// cf[l] is the coefficient of (l, m).  The loops run to the largest lmax with
-// the lane's own range as a predicate, so cf stays in registers.  The
-// recursion multiplies by 1/(l-m), which depends on l and m only, where the
+// cf[k] is the coefficient of (m + k, m).  Every lane steps k = l - m, so the
+// recursion's factors are the lane's 2m plus constants and only the writes
+// depend on the lane's range; the loops run to LM >= lmax without a test.  The
+// recursion multiplies by 1/(l-m) where the
 // reference divides by l-m: the division leaves the dependency chain of the
 // recursion, and each step changes by at most one rounding.
+template <int LM>
 __device__ __forceinline__ void put_harmonics(double *y, double ct, double cp, double sp, int m, int lmax,
-                                              const double (&cf)[ANL_SPH_LMAX_MAX + 1]) {
+                                              const double (&cf)[LM + 1]) {
+    asm volatile("" : "+v"(m));  // its comparisons stay here, where they cost one instruction, instead of in
+                                 // scalar registers across the whole atom (100 of them spilled)
     const double st = sqrt(1 - ct * ct);
-    double pmm = 1.0;
-#pragma unroll
-    for (int l = 1; l <= ANL_SPH_LMAX_MAX; ++l)
-        if (l <= m) pmm = (double)(-(2 * l - 1)) * st * pmm;
+    // the recursions in m, of which each lane keeps its own m's values
+    double pmm = 1.0, pm = 1.0;
     double cm = m > 0 ? cp : 1.0, sm = m > 0 ? sp : 0.0;
-    {
-        double c2 = 1.0, s2 = 0.0, c1 = cp, s1 = sp;
+    double c2 = 1.0, s2 = 0.0, c1 = cp, s1 = sp;
 #pragma unroll
-        for (int k = 2; k <= ANL_SPH_LMAX_MAX; ++k)
-            if (k <= m) {
-                const double cn = 2 * cp * c1 - c2;
-                const double sn = 2 * cp * s1 - s2;
-                c2 = c1;
-                s2 = s1;
-                c1 = cn;
-                s1 = sn;
-                cm = c1;
-                sm = s1;
-            }
-    }
-    double p1 = 0.0, p2 = 0.0;  // P_{l-1}^m, P_{l-2}^m
-#pragma unroll
-    for (int l = 0; l <= ANL_SPH_LMAX_MAX; ++l) {
-        if (l >= m && l <= lmax) {
-            double p;
-            if (l == m) p = pmm;
-            else if (l == m + 1) p = pmm * ct * (2 * m + 1);
-            else p = (p1 * ct * (2 * l - 1) - p2 * (l + m - 1)) * (1.0 / (double)(l - m));
-            const double v = p * cf[l];
-            y[l * l + l + m] = v * cm;
-            if (m > 0) y[l * l + l - m] = v * sm;
-            p2 = p1;
-            p1 = p;
+    for (int l = 1; l <= LM; ++l) {
+        pm = (double)(-(2 * l - 1)) * st * pm;
+        const bool own = l == m;
+        pmm = own ? pm : pmm;
+        if (l > 1) {
+            const double cn = 2 * cp * c1 - c2;
+            const double sn = 2 * cp * s1 - s2;
+            c2 = c1;
+            s2 = s1;
+            c1 = cn;
+            s1 = sn;
+            cm = own ? c1 : cm;
+            sm = own ? s1 : sm;
         }
+    }
+    const double m2 = (double)(2 * m);
+    double p1 = 0.0, p2 = 0.0;  // P_{l-1}^m, P_{l-2}^m
+    int at = m * m + m;         // l*l + l
+#pragma unroll
+    for (int k = 0; k <= LM; ++k) {
+        // k = 1: p2 is 0 and the factor 1, P_{m+1}^m = P_m^m ct (2m + 1)
+        const double p = k == 0 ? pmm : (p1 * ct * (m2 + (2 * k - 1)) - p2 * (m2 + (k - 1))) * (1.0 / (double)(k > 0 ? k : 1));
+        const double v = p * cf[k];
+        if (m + k <= lmax) {
+            y[at - m] = v * sm;  // m = 0: the same place, the cosine follows
+            y[at + m] = v * cm;
+        }
+        at += 2 * (m + k) + 2;
+        p2 = p1;
+        p1 = p;
     }
 }
 
-// Expands the nb oldest queue entries (entry k in lane k: direction, as
-// direction() leaves it, and type << 16 | bin - b0): lane (slot, m) puts entry
-// slot's harmonics into its staging block, the blocks are added into the
-// density block acc in queue order (each entry by one lane, in order), and the
-// queue moves down by nb.
-__device__ __forceinline__ void expand_queue(uint32_t nb, double &qx0, double &qx1, double &qx2, uint32_t &qcode,
-                                             uint32_t &qn, double *acc, double *stage, uint32_t nbc, uint32_t L2,
+// Expands the queue's qn entries (entry k in lane k: direction, as direction()
+// leaves it, and type << 16 | bin - b0), nc at a time: lane (slot, m) puts entry
+// slot's harmonics into its staging block, then the blocks are added into the
+// density block acc in queue order (each entry by one lane, in order).
+template <int LM>
+__device__ __forceinline__ void expand_queue(uint32_t nc, double qx0, double qx1, double qx2, uint32_t qcode,
+                                             uint32_t qn, double *acc, double *stage, uint32_t nbc, uint32_t L2,
                                              uint32_t lane, uint32_t slot, uint32_t m, int lmax,
-                                             const double (&cf)[ANL_SPH_LMAX_MAX + 1]) {
-    const int src = slot < nb ? (int)slot : 0;
-    const double y0 = __shfl(qx0, src), y1 = __shfl(qx1, src), y2 = __shfl(qx2, src);
-    if (slot < nb) put_harmonics(stage + slot * L2, y0, y1, y2, (int)m, lmax, cf);
-    wave_sync_lds();
-    for (uint32_t k = 0; k < nb; ++k) {
-        const uint32_t code = (uint32_t)__shfl((int)qcode, (int)k);
-        double *blk = acc + ((code >> 16) * nbc + (code & 0xFFFFu)) * L2;
-        for (uint32_t e = lane; e < L2; e += 64) blk[e] += stage[k * L2 + e];
+                                             const double (&cf)[LM + 1]) {
+    for (uint32_t q0 = 0; q0 < qn; q0 += nc) {
+        const uint32_t nb = min(qn - q0, nc);
+        const int src = (int)(q0 + (slot < nb ? slot : 0));
+        const double y0 = __shfl(qx0, src), y1 = __shfl(qx1, src), y2 = __shfl(qx2, src);
+        if (slot < nb) put_harmonics<LM>(stage + slot * L2, y0, y1, y2, (int)m, lmax, cf);
+        wave_sync_lds();
+        for (uint32_t k = 0; k < nb; ++k) {
+            const uint32_t code = (uint32_t)__builtin_amdgcn_readlane((int)qcode, (int)(q0 + k));
+            double *blk = acc + ((code >> 16) * nbc + (code & 0xFFFFu)) * L2;
+            for (uint32_t e = lane; e < L2; e += 64) blk[e] += stage[k * L2 + e];
+        }
+        wave_sync_lds();
     }
-    wave_sync_lds();
-    const int up = (int)min(lane + nb, 63u);
-    qx0 = __shfl(qx0, up);
-    qx1 = __shfl(qx1, up);
-    qx2 = __shfl(qx2, up);
-    qcode = (uint32_t)__shfl((int)qcode, up);
-    qn -= nb;
 }
 
 // Writes atom i's density block acc (bins b0 .. b0 + nbc - 1 of every type)
@@ -218,22 +224,28 @@ __device__ __forceinline__ void store_density(const SphDensArgs &a, const double
     const uint32_t L2 = (a.lmax + 1) * (a.lmax + 1);
     double *Sf = a.S + (uint64_t)fl * a.FS;
     const uint64_t ap = (uint64_t)a.aprime[i];
-    // blocks (type_j, bin) in a uniform loop, the (l, m) entries of a block
-    // across the lanes: no per-element division
-    for (uint32_t jt = 0; jt < a.nt; ++jt)
-        for (uint32_t bl = 0; bl < nbc && b0 + bl < a.nbin; ++bl) {
-            const double *src = acc + (jt * nbc + bl) * L2;
-            const uint64_t boff = (uint64_t)(jt * a.nbin + b0 + bl) * L2;
-            for (uint32_t e = lane; e < L2; e += 64) {
-                uint32_t l = (uint32_t)sqrtf((float)e);
-                while (l * l > e) --l;
-                while ((l + 1) * (l + 1) <= e) ++l;
-                Sf[(boff + l * l) * a.N + ap * (2 * l + 1) + (e - l * l)] = src[e];
-            }
-        }
+    // the (l, m) entries across the lanes, each with its place found once, and
+    // the blocks (type_j, bin) in a uniform loop
+    const uint64_t bstride = (uint64_t)L2 * a.N;
+    for (uint32_t e = lane; e < L2; e += 64) {
+        uint32_t l = (uint32_t)sqrtf((float)e);
+        while (l * l > e) --l;
+        while ((l + 1) * (l + 1) <= e) ++l;
+        double *o = Sf + (uint64_t)l * l * a.N + ap * (2 * l + 1) + (e - l * l) + (uint64_t)b0 * bstride;
+        const double *src = acc + e;
+        for (uint32_t jt = 0; jt < a.nt; ++jt, src += nbc * L2, o += (uint64_t)a.nbin * bstride)
+            for (uint32_t bl = 0; bl < nbc && b0 + bl < a.nbin; ++bl) o[bl * bstride] = src[bl * L2];
+    }
 }
 
-template <bool TRI>
+// Bound by VALU issue (two thirds of the cycles) at 3 wavefronts per SIMD (the
+// density blocks in LDS).  512 atoms x 295 frames, 4 shells, 2 types, lmax 10,
+// 19 neighbours: 1,521 -> 1,300 us with the recursions stepped in l - m without
+// per-lane ranges (their masks and constants no longer spill), entries read in
+// place instead of moved down the queue, (l, m) places found once, and the next
+// block loaded ahead; the densities written (1.2 GB) take 245 us at the rate of
+// a large copy.
+template <bool TRI, int LM>
 __global__ __launch_bounds__(256, 3) void sph_density_kernel(SphDensArgs a) {
     extern __shared__ double sph_lds[];
     const uint32_t wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -243,10 +255,10 @@ __global__ __launch_bounds__(256, 3) void sph_density_kernel(SphDensArgs a) {
     const uint32_t slot = lane / L1, m = lane - slot * L1;
     double *acc = sph_lds + wv * (accn + stage_doubles(a.lmax));
     double *stage = acc + accn;                        // [nc][L2] harmonics, or [64][4] new queue entries
-    double cf[ANL_SPH_LMAX_MAX + 1];                   // coefficients of (l, m) of this lane's m
+    double cf[LM + 1];                   // coefficients of (l, m) of this lane's m
 #pragma unroll
-    for (int l = 0; l <= ANL_SPH_LMAX_MAX; ++l)
-        cf[l] = (l >= (int)m && l <= (int)a.lmax) ? a.coef[l * L1 + m] : 0.0;
+    for (int k = 0; k <= LM; ++k)
+        cf[k] = m + k <= a.lmax ? a.coef[(m + k) * L1 + m] : 0.0;
     const uint32_t fl = blockIdx.x / a.ngroups;
     const uint64_t i = (uint64_t)(blockIdx.x % a.ngroups) * SPH_WAVES + wv;
     if (i >= a.N) return;  // the whole wavefront; no workgroup barrier below
@@ -281,6 +293,15 @@ __global__ __launch_bounds__(256, 3) void sph_density_kernel(SphDensArgs a) {
     double x0 = 0.0, x1 = 0.0, x2 = 0.0;
     uint32_t code = 0, cnt = 0;
     unsigned long long mask = 0;
+    // the first of `blocks` is loaded while the block before it is tested
+    uint64_t jn = 0;
+    double4 pn = pi;
+    uint32_t tn = 0;
+    auto fetch = [&] {
+        jn = (g + (uint64_t)(__ffsll(blocks) - 1)) * 64 + lane;
+        pn = P[min(jn, a.N - 1)];
+        tn = (uint32_t)a.type_slot[min(jn, a.N - 1)];
+    };
     for (;;) {
         if (!pending && !finished) {
             while (blocks == 0 && g < nblk) {
@@ -293,26 +314,27 @@ __global__ __launch_bounds__(256, 3) void sph_density_kernel(SphDensArgs a) {
                 }
                 blocks = __ballot(near);
                 if (blocks == 0) g += 64;
+                else fetch();
             }
             if (blocks == 0) {
                 finished = true;
             } else {
-                const uint64_t jb = (g + (uint64_t)(__ffsll(blocks) - 1)) * 64;
+                const uint64_t j = jn;
+                const double4 pj = pn;
+                const uint32_t tj = tn;
                 blocks &= blocks - 1;
                 if (blocks == 0) g += 64;
-                const uint64_t j = jb + lane;
+                else fetch();
                 in = false;
                 x0 = x1 = x2 = 0.0;
                 code = 0;
                 if (j < a.N && j != i) {
-                    const double4 pj = P[j];
                     x0 = pi.x - pj.x;
                     x1 = pi.y - pj.y;
                     x2 = pi.z - pj.z;
-                    min_image_ref<TRI>(x0, x1, x2, c);
+                    min_image_one<TRI>(x0, x1, x2, c);
                     const double d2 = d2_of(x0, x1, x2);
                     if (d2 >= a.d2lo && d2 < a.d2hi) {  // outer bounds over every type pair
-                        const uint32_t tj = (uint32_t)a.type_slot[j];
                         const double *T = thr_i + (size_t)tj * (a.nbin + 1);
                         if (d2 >= T[b0] && d2 < T[b1]) {
                             in = true;
@@ -350,9 +372,8 @@ __global__ __launch_bounds__(256, 3) void sph_density_kernel(SphDensArgs a) {
         }
         if (qn > 0 && (pending || finished)) {
             if (lane < qn) direction(qx0, qx1, qx2);
-            while (qn > 0)
-                expand_queue(min(qn, nc), qx0, qx1, qx2, qcode, qn, acc, stage, a.nbc, L2, lane, slot, m,
-                             (int)a.lmax, cf);
+            expand_queue<LM>(nc, qx0, qx1, qx2, qcode, qn, acc, stage, a.nbc, L2, lane, slot, m, (int)a.lmax, cf);
+            qn = 0;
         }
         if (finished) break;
     }
@@ -380,7 +401,10 @@ struct SannArgs {
 // first SANN-count of them (3, then more while the sum of the first m
 // distances exceeds r_m (m - 2)) are expanded into bin 0; the other bins are
 // zero.  The neighbour count is the l = 0 entry over Y_00.
-template <bool TRI>
+// 2,000 atoms x 30 frames, cutoff 4.5 in a 27 A cell, lmax 6: 985 -> 365 us; the
+// blocks out of reach skipped and the list lengths kept in registers 529, the
+// recursions as in sph_density_kernel 431, unrolled to lmax 6 only 365.
+template <bool TRI, int LM>
 __global__ __launch_bounds__(64) void sph_density_sann_kernel(SphDensArgs a, SannArgs s) {
     extern __shared__ double sann_lds[];
     const uint32_t lane = threadIdx.x;
@@ -393,52 +417,73 @@ __global__ __launch_bounds__(64) void sph_density_sann_kernel(SphDensArgs a, San
     double *rs = ru + s.total;                        // [capmax] sorted distances of one type
     int *ju = (int *)(rs + s.capmax);                 // [total] slots, in list order
     int *js = ju + s.total;                           // [capmax] sorted slots of one type
-    int *cnt = js + s.capmax;                         // [nt] list lengths (may exceed capacity)
-    double cf[ANL_SPH_LMAX_MAX + 1];
+    double cf[LM + 1];
 #pragma unroll
-    for (int l = 0; l <= ANL_SPH_LMAX_MAX; ++l)
-        cf[l] = (l >= (int)m && l <= (int)a.lmax) ? a.coef[l * L1 + m] : 0.0;
+    for (int k = 0; k <= LM; ++k)
+        cf[k] = m + k <= a.lmax ? a.coef[(m + k) * L1 + m] : 0.0;
     const uint32_t fl = (uint32_t)(blockIdx.x / a.N);
     const uint64_t i = blockIdx.x - (uint64_t)fl * a.N;
     for (uint32_t k = lane; k < a.nt * L2; k += 64) acc[k] = 0.0;
-    if (lane < a.nt) cnt[lane] = 0;
     wave_sync_lds();
     const uint64_t f = a.f0 + fl * a.fstride;
     const double4 *P = a.pos + f * a.N;
     const DevCell c = load_cell(a.box + f * 9);
     const double4 pi = P[i];
-    for (uint64_t jb = 0; jb < a.N; jb += 64) {
-        const uint64_t j = jb + lane;
-        bool ok = false;
-        uint32_t tj = 0;
-        double d2 = 0.0;
-        if (j < a.N && j != i) {
-            const double4 pj = P[j];
-            double x0 = pi.x - pj.x, x1 = pi.y - pj.y, x2 = pi.z - pj.z;
-            min_image_ref<TRI>(x0, x1, x2, c);
-            d2 = d2_of(x0, x1, x2);
-            tj = (uint32_t)a.type_slot[j];
-            ok = d2 <= s.cut2[tj];
+    // blocks of 64 slots, 64 blocks at a time, as in sph_density_kernel: a block
+    // whose bounding sphere is farther than the largest cutoff is skipped.  The
+    // length of type t's list is lane t's.
+    const double4 *rad = a.block_rad ? a.block_rad + (uint64_t)fl * ((a.N + 63) / 64) : nullptr;
+    const uint64_t nblk = (a.N + 63) / 64;
+    uint32_t cntv = 0;
+    for (uint64_t g = 0; g < nblk; g += 64) {
+        bool near = g + lane < nblk;
+        if (rad && near) {
+            const double4 bc = rad[g + lane];
+            double y0 = pi.x - bc.x, y1 = pi.y - bc.y, y2 = pi.z - bc.z;
+            min_image_ref<false>(y0, y1, y2, c);
+            near = !(sqrt(d2_of(y0, y1, y2)) > a.rcut + bc.w);
         }
-        for (uint32_t t = 0; t < a.nt; ++t) {
-            const unsigned long long mask = __ballot(ok && tj == t);
-            if (!mask) continue;
-            const uint32_t base = (uint32_t)cnt[t], add = (uint32_t)__popcll(mask);
-            if (ok && tj == t) {
-                const uint32_t pos = base + (uint32_t)__popcll(mask & ((1ull << lane) - 1));
-                if (pos < s.nn[t]) {
-                    ru[s.off[t] + pos] = sqrt(d2);
-                    ju[s.off[t] + pos] = (int)j;
+        unsigned long long blocks = __ballot(near);
+        // the next near block's atoms are loaded while this one's are tested
+        double4 pn = pi;
+        uint32_t tn = 0;
+        auto fetch = [&] {
+            const uint64_t j = (g + (uint64_t)(__ffsll(blocks) - 1)) * 64 + lane;
+            pn = P[min(j, a.N - 1)];
+            tn = (uint32_t)a.type_slot[min(j, a.N - 1)];
+        };
+        if (blocks) fetch();
+        while (blocks) {
+            const uint64_t j = (g + (uint64_t)(__ffsll(blocks) - 1)) * 64 + lane;
+            const double4 pj = pn;
+            const uint32_t tj = tn;
+            blocks &= blocks - 1;
+            if (blocks) fetch();
+            double x0 = pi.x - pj.x, x1 = pi.y - pj.y, x2 = pi.z - pj.z;
+            min_image_one<TRI>(x0, x1, x2, c);
+            const double d2 = d2_of(x0, x1, x2);
+            double cut2 = s.cut2[0];
+            for (uint32_t t = 1; t < a.nt; ++t) cut2 = tj == t ? s.cut2[t] : cut2;
+            const bool ok = j < a.N && j != i && d2 <= cut2;
+            if (!__ballot(ok)) continue;
+            for (uint32_t t = 0; t < a.nt; ++t) {
+                const unsigned long long mask = __ballot(ok && tj == t);
+                if (!mask) continue;
+                const uint32_t base = (uint32_t)__builtin_amdgcn_readlane((int)cntv, (int)t);
+                if (ok && tj == t) {
+                    const uint32_t pos = base + (uint32_t)__popcll(mask & ((1ull << lane) - 1));
+                    if (pos < s.nn[t]) {
+                        ru[s.off[t] + pos] = sqrt(d2);
+                        ju[s.off[t] + pos] = (int)j;
+                    }
                 }
+                if (lane == t) cntv += (uint32_t)__popcll(mask);
             }
-            wave_sync_lds();
-            if (lane == 0) {
-                cnt[t] = (int)(base + add);
-                if (base + add > s.nn[t]) atomicOr(s.overflow, 1);
-            }
-            wave_sync_lds();
         }
     }
+    for (uint32_t t = 0; t < a.nt; ++t)
+        if ((uint32_t)__builtin_amdgcn_readlane((int)cntv, (int)t) > s.nn[t] && lane == 0) atomicOr(s.overflow, 1);
+    wave_sync_lds();
     // neighbour.cpp:19-44 meets the pairs of atom i in increasing order of
     // the partner's index and throws when a pair within either type's cutoff
     // finds i's list for the partner's type already full.  Beyond a list that
@@ -449,7 +494,7 @@ __global__ __launch_bounds__(64) void sph_density_sann_kernel(SphDensArgs a, San
     {
         const uint32_t ti = (uint32_t)a.type_slot[i];
         for (uint32_t t = 0; t < a.nt; ++t) {
-            if (!((uint32_t)cnt[t] == s.nn[t] && s.cut2[ti] > s.cut2[t])) continue;  // uniform
+            if (!((uint32_t)__builtin_amdgcn_readlane((int)cntv, (int)t) == s.nn[t] && s.cut2[ti] > s.cut2[t])) continue;  // uniform
             int last = -1;
             for (uint32_t k = lane; k < s.nn[t]; k += 64) last = max(last, s.orig[ju[s.off[t] + k]]);
             for (int o = 32; o > 0; o >>= 1) last = max(last, __shfl_xor(last, o, 64));
@@ -470,26 +515,33 @@ __global__ __launch_bounds__(64) void sph_density_sann_kernel(SphDensArgs a, San
     double qx0 = 0.0, qx1 = 0.0, qx2 = 0.0;
     uint32_t qcode = 0, qn = 0;
     for (uint32_t t = 0; t < a.nt; ++t) {
-        const uint32_t n = min((uint32_t)cnt[t], s.nn[t]);
+        const uint32_t n = min((uint32_t)__builtin_amdgcn_readlane((int)cntv, (int)t), s.nn[t]);
         const double *r = ru + s.off[t];
         const int *jj = ju + s.off[t];
         for (uint32_t k = lane; k < n; k += 64) {
+            // the list is in slot order: among equal distances the earlier entry
             const double rk = r[k];
-            const int jk = jj[k];
             uint32_t rank = 0;
-            for (uint32_t q = 0; q < n; ++q) rank += (r[q] < rk || (r[q] == rk && jj[q] < jk)) ? 1u : 0u;
+#pragma unroll 8
+            for (uint32_t q = 0; q < n; ++q) rank += (r[q] < rk || (r[q] == rk && q < k)) ? 1u : 0u;
             rs[rank] = rk;
-            js[rank] = jk;
+            js[rank] = jj[k];
         }
         wave_sync_lds();
-        uint32_t ms = 0;  // neighbour.cpp:85-101
+        uint32_t ms = 0;  // neighbour.cpp:85-101, the distances 64 at a time from registers
         if (n >= 3) {
-            ms = 3;
-            double sum = rs[0] + rs[1] + rs[2];
-            while (ms < n) {
-                if (sum <= rs[ms] * (double)(ms - 2)) break;
-                sum += rs[ms];
-                ms++;
+            double v = rs[min(lane, n - 1)];
+            auto at = [&](uint32_t k) {
+                const int lo = __builtin_amdgcn_readlane(__double2loint(v), (int)(k & 63u));
+                const int hi = __builtin_amdgcn_readlane(__double2hiint(v), (int)(k & 63u));
+                return __hiloint2double(hi, lo);
+            };
+            double sum = at(0) + at(1) + at(2);
+            for (ms = 3; ms < n; ++ms) {
+                if ((ms & 63u) == 0) v = rs[min(ms + lane, n - 1)];
+                const double r1 = at(ms);
+                if (sum <= r1 * (double)(ms - 2)) break;
+                sum += r1;
             }
         }
         if (s.nbr) {
@@ -507,9 +559,7 @@ __global__ __launch_bounds__(64) void sph_density_sann_kernel(SphDensArgs a, San
                 qcode = t << 16;
             }
             if (lane < qn) direction(qx0, qx1, qx2);
-            while (qn > 0)
-                expand_queue(min(qn, nc), qx0, qx1, qx2, qcode, qn, acc, stage, 1, L2, lane, slot, m,
-                             (int)a.lmax, cf);
+            expand_queue<LM>(nc, qx0, qx1, qx2, qcode, qn, acc, stage, 1, L2, lane, slot, m, (int)a.lmax, cf);
         }
         wave_sync_lds();  // rs, js are reused by the next type
     }
@@ -518,14 +568,15 @@ __global__ __launch_bounds__(64) void sph_density_sann_kernel(SphDensArgs a, San
     // bins 1.. hold nothing with a neighbour list
     double *Sf = a.S + (uint64_t)fl * a.FS;
     const uint64_t ap = (uint64_t)a.aprime[i];
-    for (uint32_t t = 0; t < a.nt; ++t)
-        for (uint32_t b = 1; b < a.nbin; ++b)
-            for (uint32_t e = lane; e < L2; e += 64) {
-                uint32_t l = (uint32_t)sqrtf((float)e);
-                while (l * l > e) --l;
-                while ((l + 1) * (l + 1) <= e) ++l;
-                Sf[((uint64_t)(t * a.nbin + b) * L2 + l * l) * a.N + ap * (2 * l + 1) + (e - l * l)] = 0.0;
-            }
+    if (a.nbin > 1)
+        for (uint32_t e = lane; e < L2; e += 64) {
+            uint32_t l = (uint32_t)sqrtf((float)e);
+            while (l * l > e) --l;
+            while ((l + 1) * (l + 1) <= e) ++l;
+            double *o = Sf + (uint64_t)l * l * a.N + ap * (2 * l + 1) + (e - l * l);
+            for (uint32_t t = 0; t < a.nt; ++t)
+                for (uint32_t b = 1; b < a.nbin; ++b) o[(uint64_t)(t * a.nbin + b) * L2 * a.N] = 0.0;
+        }
 }
 
 struct SphGramArgs {
@@ -853,6 +904,15 @@ void launch_density(anl_sph *h, uint64_t f0, uint64_t fstride, uint32_t nfr, dou
     if (lm > h->lmax) lm = h->lmax;
     SphDensArgs a{};
     a.fstride = fstride;
+    a.block_rad = h->block_screen ? rad : nullptr;
+    auto block_spheres = [&] {
+        if (!a.block_rad) return;
+        const uint64_t nb = (uint64_t)nfr * ((h->tr->N + 63) / 64);
+        if (nb > 0x7fffffffull) fail(ANL_ERR_ARG, "too many (frame, atom block) pairs in one launch");
+        hipLaunchKernelGGL(sph_block_radius_kernel, dim3((uint32_t)nb), dim3(64), 0, s, h->tr->pos, h->tr->box,
+                           h->tr->N, f0, fstride, rad);
+        ANL_HIP(hipGetLastError());
+    };
     if (h->sann) {
         a.pos = h->tr->pos;
         a.box = h->tr->box;
@@ -871,14 +931,19 @@ void launch_density(anl_sph *h, uint64_t f0, uint64_t fstride, uint32_t nfr, dou
         if (gx > 0x7fffffffull) fail(ANL_ERR_ARG, "too many (frame, atom) pairs in one density launch");
         SannArgs sa = h->sann_args;
         sa.nbr = nbr;  // the chosen neighbours, for the averaged order parameter
+        double cut2 = 0.0;
+        for (uint32_t t = 0; t < h->nt; t++) cut2 = std::max(cut2, sa.cut2[t]);
+        a.rcut = std::sqrt(cut2) * (1.0 + 1e-9) + 1e-9;
+        block_spheres();
         const size_t lds = (size_t)(h->nt * (lm + 1) * (lm + 1) + stage_doubles(lm) + sa.total +
                                     sa.capmax) * sizeof(double) +
-                           (size_t)(sa.total + sa.capmax + SANN_MAXT) * sizeof(int);
+                           (size_t)(sa.total + sa.capmax) * sizeof(int);
         ANL_HIP(hipMemsetAsync(h->d_overflow, 0, sizeof(int), s));
-        if (h->tr->triclinic)
-            hipLaunchKernelGGL(sph_density_sann_kernel<true>, dim3((uint32_t)gx), dim3(64), lds, s, a, sa);
-        else
-            hipLaunchKernelGGL(sph_density_sann_kernel<false>, dim3((uint32_t)gx), dim3(64), lds, s, a, sa);
+        auto kernel = lm <= SPH_LM_LOW ? (h->tr->triclinic ? sph_density_sann_kernel<true, SPH_LM_LOW>
+                                                           : sph_density_sann_kernel<false, SPH_LM_LOW>)
+                                       : (h->tr->triclinic ? sph_density_sann_kernel<true, ANL_SPH_LMAX_MAX>
+                                                           : sph_density_sann_kernel<false, ANL_SPH_LMAX_MAX>);
+        hipLaunchKernelGGL(kernel, dim3((uint32_t)gx), dim3(64), lds, s, a, sa);
         ANL_HIP(hipGetLastError());
         int over = 0;
         ANL_HIP(hipMemcpyAsync(&over, h->d_overflow, sizeof(int), hipMemcpyDeviceToHost, s));
@@ -889,14 +954,7 @@ void launch_density(anl_sph *h, uint64_t f0, uint64_t fstride, uint32_t nfr, dou
     a.d2lo = h->d2lo;
     a.d2hi = h->d2hi;
     a.rcut = h->rcut;
-    a.block_rad = h->block_screen ? rad : nullptr;
-    if (a.block_rad) {
-        const uint64_t nb = (uint64_t)nfr * ((h->tr->N + 63) / 64);
-        if (nb > 0x7fffffffull) fail(ANL_ERR_ARG, "too many (frame, atom block) pairs in one launch");
-        hipLaunchKernelGGL(sph_block_radius_kernel, dim3((uint32_t)nb), dim3(64), 0, s, h->tr->pos, h->tr->box,
-                           h->tr->N, f0, fstride, rad);
-        ANL_HIP(hipGetLastError());
-    }
+    block_spheres();
     a.pos = h->tr->pos;
     a.box = h->tr->box;
     a.type_slot = h->tr->type_slot;
@@ -918,10 +976,10 @@ void launch_density(anl_sph *h, uint64_t f0, uint64_t fstride, uint32_t nfr, dou
     if (gx > 0x7fffffffull) fail(ANL_ERR_ARG, "too many (frame, atom) pairs in one density launch");
     if ((h->nbin + a.nbc - 1) / a.nbc > 65535) fail(ANL_ERR_ARG, "too many distance bins");
     dim3 grid((uint32_t)gx, (h->nbin + a.nbc - 1) / a.nbc);
-    if (h->tr->triclinic)
-        hipLaunchKernelGGL(sph_density_kernel<true>, grid, dim3(256), lds, s, a);
-    else
-        hipLaunchKernelGGL(sph_density_kernel<false>, grid, dim3(256), lds, s, a);
+    auto kernel = lm <= SPH_LM_LOW ? (h->tr->triclinic ? sph_density_kernel<true, SPH_LM_LOW> : sph_density_kernel<false, SPH_LM_LOW>)
+                                   : (h->tr->triclinic ? sph_density_kernel<true, ANL_SPH_LMAX_MAX>
+                                                       : sph_density_kernel<false, ANL_SPH_LMAX_MAX>);
+    hipLaunchKernelGGL(kernel, grid, dim3(256), lds, s, a);
     ANL_HIP(hipGetLastError());
 }
 
