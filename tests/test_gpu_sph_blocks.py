@@ -48,3 +48,21 @@ def test_blocks_and_lists(N, L, tri):
         s = capi.DeviceSph(dt, rm, 1, 4)
         s.set_neighbours(spec)
         _close(s.snapshot(1), O.sph_density_sann(ot, 1, spec, 1, 4)[0])
+
+
+@pytest.mark.parametrize("tri", [False, True])
+@pytest.mark.parametrize("N,lmax,ll", [(21, 1, [1]), (64, 10, [2, 10]), (65, 7, [7]), (150, 10, [4, 6, 9])])
+def test_averaged_order_parameter(N, lmax, ll, tri):
+    """One wavefront per item: l values of one to all entries of two per lane,
+    item counts around the 64 of a workgroup."""
+    ot, dt = _case(23, N, 7.0 if N < 100 else 9.0, tri)
+    spec = [(200, 3.4 ** 2, 0.0), (200, 3.1 ** 2, 0.0)]
+    s = capi.DeviceSph(dt, np.tile([0.5, 2.6], (4, 1)), 1, lmax)
+    s.set_neighbours(spec)
+    q = s.steinhardt(3, 1, 0, ll, 12, do_histogram=False, averaged=True)
+    want = O.steinhardt_sann(ot, spec, lmax, 12, ll, 1, 3, 0, False, averaged=True)
+    same_nan = np.isnan(q) == np.isnan(want)
+    assert same_nan.all() and np.nanmax(np.abs(q - want)) <= 1e-12
+    h = s.steinhardt(3, 1, 0, ll, 12, averaged=True)
+    hw = O.steinhardt_sann(ot, spec, lmax, 12, ll, 1, 3, 0, True, averaged=True)
+    np.testing.assert_allclose(h, hw, rtol=1e-13, atol=0)
