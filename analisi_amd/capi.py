@@ -44,6 +44,7 @@ SIGNATURES = [
     ("anl_gofrt_destroy", _i, [_vp]),
     ("anl_gofrt_reset", _i, [_vp, _u32, ctypes.POINTER(_u32)]),
     ("anl_gofrt_calculate", _i, [_vp, _u64, _vp]),
+    ("anl_gofrt_calculate_scaled", _i, [_vp, _u64, ctypes.c_double, _vp]),
     ("anl_gofrt_calculate_async", _i, [_vp, _u64, _vp, _vp]),
     ("anl_gofrt_calc_single_th", _i, [_vp, _i, _i, _i, _i, _u64, _vp]),
     ("anl_gofrt_calculate_blocks_async", _i, [_vp, _vp, _vp, _u32, _vp, _vp]),

@@ -1169,7 +1169,7 @@ template <bool TRI>
 __global__ __launch_bounds__(WG, 4) void gofrt_cells_kernel(const GofrtCellArgs ca) {
     constexpr int QC = SQCAP;
     const GofrtArgs &a = ca.g;
-    extern __shared__ __align__(16) unsigned char smem[];
+    extern __shared__ unsigned char smem[];
     const WgId id = decode_wg(a.ntiles, a.nlag, a.nwork, a.per_xcd);
     if (!id.valid) return;
     BlockInfo b;
