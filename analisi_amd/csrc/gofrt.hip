@@ -1941,7 +1941,7 @@ struct anl_gofrt {
     int32_t *d_chan = nullptr;
     unsigned long long *d_ncand = nullptr;   // [NSTAT] statistics of the last launch (Stat)
     int last_form = -1;
-    // a changing cell: the screen of every frame's cell (prepare_cells)
+    // a changing cell: the screen of every frame's cell (use_cells)
     CellScreen *d_cells = nullptr;
     int cells = -1;               // -1 not looked at, 0 the screen does not apply, 1 it does
     // scratch for the work list
