@@ -1977,10 +1977,11 @@ constexpr uint64_t CELLS_MIN_ATOMS = 769;
 bool use_cells(anl_gofrt *g) {
     anl_traj *tr = g->tr;
     if (g->form != ANL_GOFRT_AUTO || tr->box_const || tr->N < CELLS_MIN_ATOMS) return false;
+    std::lock_guard<std::mutex> lock(tr->screen_mutex);
     if (g->cells < 0) {
         std::vector<CellScreen> cells(tr->F);
-        g->cells = 1;
-        for (uint64_t f = 0; f < tr->F && g->cells; f++) {
+        bool ok = true;
+        for (uint64_t f = 0; f < tr->F && ok; f++) {
             const Cell c = cell_of(&tr->box_host[f * 9]);
             double wd[3];
             const Screen s = make_screen(c, true, tr->nt, g->rmax, wd);
@@ -1990,8 +1991,9 @@ bool use_cells(anl_gofrt *g) {
             const double tilt = std::max(std::fabs(c.xy), std::max(std::fabs(c.xz), std::fabs(c.yz))) / lmin;
             const double lo = std::max(std::fabs(c.lo[0]), std::max(std::fabs(c.lo[1]), std::fabs(c.lo[2])));
             const double e_s = 16.0 * std::ldexp(1.0, -53) * (1.0 + tilt) * (1.0 + tilt) * ((tr->pos_max + lo) / lmin + 1.0);
-            if (!s.valid || !(e_s < std::ldexp(1.0, -33))) {
-                g->cells = 0;
+            const bool finite = std::isfinite(c.lo[0]) && std::isfinite(c.lo[1]) && std::isfinite(c.lo[2]);
+            if (!s.valid || !finite || !(e_s < std::ldexp(1.0, -33))) {
+                ok = false;
                 break;
             }
             uint32_t gap[3];
@@ -2003,10 +2005,11 @@ bool use_cells(anl_gofrt *g) {
                                   (float)(c.yz * sc), (float)(c.L[2] * sc),
                                   du_window(s, tr->triclinic, g->rmin, g->rmax, g->dr, g->nbin), 0.0f};
         }
-        if (g->cells) {
-            ANL_HIP(hipMalloc(&g->d_cells, cells.size() * sizeof(CellScreen)));
+        if (ok) {
+            if (!g->d_cells) ANL_HIP(hipMalloc(&g->d_cells, cells.size() * sizeof(CellScreen)));
             ANL_HIP(hipMemcpy(g->d_cells, cells.data(), cells.size() * sizeof(CellScreen), hipMemcpyHostToDevice));
         }
+        g->cells = ok ? 1 : 0;
     }
     return g->cells == 1;
 }
