@@ -169,11 +169,16 @@ struct anl_series {
     uint32_t ncols = 0;
     double *data = nullptr;
     double2 *rec = nullptr;  // [nrows] 1/c, c = 1 .. nrows, in two parts (gk_reciprocals)
-    // Green-Kubo scratch (splits, partial sums, output staging), grow-only;
-    // calls on one series are stream-ordered on the caller's stream.
+    // scratch of the MFMA form (splits, partial sums), grow-only; its calls on
+    // one series are stream-ordered on the caller's stream.
     void *work = nullptr;
     size_t work_cap = 0;
-    anl::ScratchPool scratch;  // outputs of anl_gk_calculate_blocks
+    anl::ScratchPool scratch;  // of the synchronous calls: outputs, segment means of the FP64 form
+    // segment means of the asynchronous FP64 calls, in turn (GkSegments)
+    std::mutex seg_mutex;
+    void *seg = nullptr;
+    size_t seg_cap = 0;
+    hipEvent_t seg_done = nullptr;  // the last call's end
     // launch shape of the MFMA lag products: tiles per wavefront, MFMA steps
     // per FP32 chunk, wavefronts per workgroup (anl_gk_set_tuning)
     uint32_t gk_q = 8, gk_cs = 16, gk_wg = 4;
@@ -227,7 +232,6 @@ void gk_reciprocals(double2 *rec, uint64_t n, hipStream_t s);
 void gk_mfma_enqueue_blocks(anl_series *s, const uint32_t *idx_j, uint32_t ncur, uint32_t skip, uint32_t leff,
                             uint32_t n_seg, const uint64_t *primo, const uint32_t *n, uint32_t nblocks, double *d,
                             hipStream_t st);
-size_t gk_mfma_scratch_bytes(const anl_series *s, uint32_t ncur, uint32_t leff, uint32_t n);
 bool gkm_shape_ok(uint32_t q, uint32_t cs, uint32_t wg);
 // MediaVar over blocks (calcoliblocchi.h:21-65) of x_b = counts_b * incr_b or
 // values_b, element-parallel, Welford steps in block order.

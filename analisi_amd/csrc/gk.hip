@@ -14,6 +14,7 @@
 #include <algorithm>
 #include <atomic>
 #include <cstring>
+#include <optional>
 #include <thread>
 #include <type_traits>
 
@@ -1020,20 +1021,19 @@ void gk_epilogue(double *d, uint32_t narr, uint32_t ncur, uint32_t leff, int sub
     gk_schur_launch(d, narr, ncur, leff, s, nblocks, stride);
 }
 
-size_t gk_fp64_scratch_bytes(uint32_t ncur, uint32_t leff, uint32_t n_seg, uint32_t nblocks) {
-    return n_seg > 1 ? (size_t)std::min(GK_MAXB, nblocks) * n_seg * ncur * ncur * leff * sizeof(double) : 0;
+// Bytes of the segment means of a call, 0 where it keeps none: more than the
+// cap, or one segment.
+constexpr size_t GK_SEG_BYTES = 1ull << 30;
+static size_t gk_segment_bytes(uint32_t ncur, uint32_t leff, uint32_t n_seg, uint32_t nblocks) {
+    if (n_seg < 2 || n_seg > 65535) return 0;
+    const size_t need = (size_t)std::min(GK_MAXB, nblocks) * n_seg * ncur * ncur * leff * sizeof(double);
+    return need <= GK_SEG_BYTES ? need : 0;
 }
 
 void gk_reciprocals(double2 *rec, uint64_t n, hipStream_t s) {
     hipLaunchKernelGGL(gk_reciprocal_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, rec, n);
     ANL_HIP(hipGetLastError());
 }
-
-// The segments of a block run side by side into scratch of the series and
-// are folded afterwards, when the scratch is there or can be had; else (more
-// scratch than the cap, or a stream under capture, where nothing can be
-// allocated) one launch per segment folds into the output.
-constexpr size_t GK_SEG_BYTES = 1ull << 30;
 
 // Wavefronts of 64 means from which a stride 1 launch takes gk_dense_kernel:
 // gk_chain_kernel's time for 20,000 t0 grows by 0.48 ms per 256 (one
@@ -1049,15 +1049,14 @@ static bool gk_can_allocate(hipStream_t st) {
     return c == hipStreamCaptureStatusNone;
 }
 
-void gk_fp64_enqueue_blocks(anl_series *s, const uint32_t *idx_j, uint32_t ncur, uint32_t skip, uint32_t leff,
-                            uint32_t n_seg, const uint64_t *primo, const uint32_t *n, uint32_t nblocks, double *d,
-                            hipStream_t st) {
+// The segments of a block run side by side into segm (gk_segment_bytes) and
+// are folded afterwards; without it one launch per segment folds into the
+// output.
+static void gk_fp64_enqueue_blocks(anl_series *s, const uint32_t *idx_j, uint32_t ncur, uint32_t skip, uint32_t leff,
+                                   uint32_t n_seg, const uint64_t *primo, const uint32_t *n, uint32_t nblocks,
+                                   double *d, double *segm, hipStream_t st) {
     const uint32_t narr = 3 * ncur * ncur + 2;
     const uint64_t stride = (uint64_t)leff * narr;
-    const size_t need = gk_fp64_scratch_bytes(ncur, leff, n_seg, nblocks);
-    double *segm = nullptr;
-    if (need && need <= GK_SEG_BYTES && n_seg <= 65535 && (need <= s->work_cap || gk_can_allocate(st)))
-        segm = (double *)series_workspace(s, need);
     for (uint32_t b0 = 0; b0 < nblocks; b0 += GK_MAXB) {
         const uint32_t nb = std::min(GK_MAXB, nblocks - b0);
         GkArgs a{};
@@ -1125,6 +1124,89 @@ uint32_t gk_block_checks(anl_series *s, const uint32_t *idx_j, uint32_t ncur, ui
     return leff0;
 }
 
+static void gk_enqueue_checks(int form, uint32_t nblocks, const double *mean, const double *var) {
+    if ((mean || var) && (!mean || !var || nblocks < 2))
+        fail(ANL_ERR_ARG, "block mean and variance need both outputs and at least two blocks");
+    if (form != ANL_GK_FP64 && form != ANL_GK_MFMA) fail(ANL_ERR_ARG, "unknown Green-Kubo form");
+}
+
+// A checked call (gk_block_checks, gk_enqueue_checks, leff > 0) on stream st;
+// segm: the FP64 form's segment means, or null.
+static void gk_enqueue(anl_series *s, const uint32_t *idx_j, uint32_t ncur, uint32_t skip, uint32_t leff, uint32_t n_seg,
+                       int subtract_mean, uint32_t start_mean, const uint64_t *primo, const uint32_t *n,
+                       uint32_t nblocks, int form, double *out_dev, double *mean_dev, double *var_dev, double *segm,
+                       hipStream_t st) {
+    if (n_seg < 1) n_seg = 1;  // greenkubo...cpp:50-53
+    if (skip == 0) skip = 1;
+    const uint32_t narr = 3 * ncur * ncur + 2;
+    const uint64_t stride = (uint64_t)leff * narr;
+    if (form == ANL_GK_MFMA) gk_mfma_enqueue_blocks(s, idx_j, ncur, skip, leff, n_seg, primo, n, nblocks, out_dev, st);
+    else gk_fp64_enqueue_blocks(s, idx_j, ncur, skip, leff, n_seg, primo, n, nblocks, out_dev, segm, st);
+    // the FP64 form keeps the reference's serial scans (bit-identical results)
+    gk_epilogue(out_dev, narr, ncur, leff, subtract_mean, start_mean, st, nblocks, stride, form == ANL_GK_FP64, s->rec);
+    if (mean_dev) mediavar_blocks(nullptr, out_dev, nullptr, nblocks, stride, mean_dev, var_dev, st);
+}
+
+// The series' segment means for one asynchronous call: calls from any threads
+// and on any streams take them in turn, each stream waiting for the call
+// before.  p is null, and the call folds segment by segment, where they would
+// take more than a kept workspace may, where the memory cannot be had, and on
+// a stream under capture (a graph would keep an address that a later call may
+// free).
+struct GkSegments {
+    anl_series *s;
+    hipStream_t st;
+    std::unique_lock<std::mutex> lock;
+    double *p = nullptr;
+    GkSegments(anl_series *s, size_t need, hipStream_t st) : s(s), st(st) {
+        if (need == 0 || need > SCRATCH_KEEP || !gk_can_allocate(st)) return;
+        lock = std::unique_lock<std::mutex>(s->seg_mutex);
+        if (!s->seg_done) ANL_HIP(hipEventCreateWithFlags(&s->seg_done, hipEventDisableTiming));
+        if (need > s->seg_cap) {
+            if (s->seg) ANL_HIP(hipEventSynchronize(s->seg_done));
+            (void)hipFree(s->seg);
+            s->seg = nullptr;
+            s->seg_cap = 0;
+            if (hipMalloc(&s->seg, need) != hipSuccess) {
+                (void)hipGetLastError();
+                s->seg = nullptr;
+                return;
+            }
+            s->seg_cap = need;
+        } else {
+            ANL_HIP(hipStreamWaitEvent(st, s->seg_done, 0));
+        }
+        p = (double *)s->seg;
+    }
+    ~GkSegments() {
+        // if the record fails the next call must not go on without it
+        if (p && hipEventRecord(s->seg_done, st) != hipSuccess) (void)hipStreamSynchronize(st);
+    }
+    GkSegments(const GkSegments &) = delete;
+    GkSegments &operator=(const GkSegments &) = delete;
+};
+
+// A pooled workspace of `bytes` for a synchronous call, with room for the
+// segment means behind them if that can be had.
+struct GkWorkspace {
+    std::optional<ScratchLease> w;
+    double *segm = nullptr;
+    GkWorkspace(anl_series *s, size_t bytes, size_t seg, size_t pin) {
+        bytes = (std::max<size_t>(bytes, 8) + 255) / 256 * 256;
+        if (seg) {
+            try {
+                w.emplace(s->scratch, bytes + seg, pin);
+                segm = (double *)((char *)w->s.dev + bytes);
+                return;
+            } catch (const Error &) {
+                (void)hipGetLastError();
+            }
+        }
+        w.emplace(s->scratch, bytes, pin);
+    }
+    double *dev() const { return (double *)w->s.dev; }
+};
+
 }  // namespace anl
 
 using namespace anl;
@@ -1138,22 +1220,14 @@ int anl_gk_calculate_blocks_async(anl_series *s, const uint32_t *idx_j, uint32_t
     return guard([&] {
         const uint32_t leff = gk_block_checks(s, idx_j, ncur, tmax, primo, n, nblocks);
         if (!out_dev) fail(ANL_ERR_ARG, "null output passed to anl_gk_calculate_blocks_async");
-        if ((mean_dev || var_dev) && (!mean_dev || !var_dev || nblocks < 2))
-            fail(ANL_ERR_ARG, "block mean and variance need both outputs and at least two blocks");
-        if (form != ANL_GK_FP64 && form != ANL_GK_MFMA) fail(ANL_ERR_ARG, "unknown Green-Kubo form");
-        if (n_seg < 1) n_seg = 1;  // greenkubo...cpp:50-53
-        if (skip == 0) skip = 1;
+        gk_enqueue_checks(form, nblocks, mean_dev, var_dev);
         if (leff == 0) return;
         ensure_device();
-        const uint32_t narr = 3 * ncur * ncur + 2;
-        const uint64_t stride = (uint64_t)leff * narr;
         hipStream_t st = (hipStream_t)stream;
-        if (form == ANL_GK_MFMA) gk_mfma_enqueue_blocks(s, idx_j, ncur, skip, leff, n_seg, primo, n, nblocks, out_dev, st);
-        else gk_fp64_enqueue_blocks(s, idx_j, ncur, skip, leff, n_seg, primo, n, nblocks, out_dev, st);
-        // the FP64 form keeps the reference's serial scans (bit-identical results)
-        gk_epilogue(out_dev, narr, ncur, leff, subtract_mean, start_mean, st, nblocks, stride, form == ANL_GK_FP64,
-                    s->rec);
-        if (mean_dev) mediavar_blocks(nullptr, out_dev, nullptr, nblocks, stride, mean_dev, var_dev, st);
+        const size_t need = form == ANL_GK_FP64 ? gk_segment_bytes(ncur, leff, n_seg, nblocks) : 0;
+        GkSegments seg(s, need, st);
+        gk_enqueue(s, idx_j, ncur, skip, leff, n_seg, subtract_mean, start_mean, primo, n, nblocks, form, out_dev,
+                   mean_dev, var_dev, seg.p, st);
     });
 }
 
@@ -1171,13 +1245,18 @@ int anl_gk_calculate_blocks(anl_series *s, const uint32_t *idx_j, uint32_t ncur,
     return guard([&] {
         const uint32_t leff = gk_block_checks(s, idx_j, ncur, tmax, primo, n, nblocks);
         if (!out_host) fail(ANL_ERR_ARG, "null output passed to anl_gk_calculate_blocks");
+        gk_enqueue_checks(form, nblocks, mean_host, var_host);
+        if (leff == 0) return;
         ensure_device();
         const size_t len = (size_t)leff * (3 * ncur * ncur + 2), all = len * nblocks, total = all * sizeof(double);
         constexpr size_t PIECE = 2u << 20, RING = 3;
         const size_t pieces = (total + PIECE - 1) / PIECE;
         const unsigned nth = pieces < 2 ? 0 : std::min(8u, std::max(1u, std::thread::hardware_concurrency()));
-        ScratchLease w(s->scratch, std::max<size_t>((all + 2 * len) * sizeof(double), 8), nth ? RING * PIECE : 0);
-        double *d = (double *)w.s.dev;
+        const GkWorkspace w(s, (all + 2 * len) * sizeof(double),
+                            form == ANL_GK_FP64 ? gk_segment_bytes(ncur, leff, n_seg, nblocks) : 0,
+                            nth ? RING * PIECE : 0);
+        double *d = w.dev();
+        char *ring = (char *)w.w->s.pin;
         constexpr int64_t NOT_YET = -1, GIVE_UP = -2;  // no kernels yet; there will be no output
         std::atomic<int64_t> arrived{NOT_YET};         // pieces in the ring so far
         std::atomic<uint64_t> copied[RING] = {};       // shares copied out of each of its slots
@@ -1195,7 +1274,7 @@ int anl_gk_calculate_blocks(anl_series *s, const uint32_t *idx_j, uint32_t ncur,
                 while ((a = arrived.load(std::memory_order_acquire)) <= (int64_t)p && a != GIVE_UP) std::this_thread::yield();
                 if (a == GIVE_UP) return;
                 const size_t b0 = share(p, k), b1 = share(p, k + 1);
-                std::memcpy((char *)out_host + b0, (const char *)w.s.pin + p % RING * PIECE + (b0 - p * PIECE), b1 - b0);
+                std::memcpy((char *)out_host + b0, ring + p % RING * PIECE + (b0 - p * PIECE), b1 - b0);
                 copied[p % RING].fetch_add(1, std::memory_order_release);
             }
         };
@@ -1207,10 +1286,8 @@ int anl_gk_calculate_blocks(anl_series *s, const uint32_t *idx_j, uint32_t ncur,
                 if (e) (void)hipEventDestroy(e);
         };
         try {
-            int rc = anl_gk_calculate_blocks_async(s, idx_j, ncur, skip, tmax, n_seg, subtract_mean, start_mean, primo, n,
-                                                   nblocks, form, d, mean_host ? d + all : nullptr,
-                                                   var_host ? d + all + len : nullptr, 0);
-            if (rc != ANL_OK) throw Error{rc, anl_last_error()};
+            gk_enqueue(s, idx_j, ncur, skip, leff, n_seg, subtract_mean, start_mean, primo, n, nblocks, form, d,
+                       mean_host ? d + all : nullptr, var_host ? d + all + len : nullptr, w.segm, 0);
             if (nth) {
                 pool.reserve(nth);
                 for (unsigned k = 0; k < nth; k++) pool.emplace_back(work, k);
@@ -1221,7 +1298,7 @@ int anl_gk_calculate_blocks(anl_series *s, const uint32_t *idx_j, uint32_t ncur,
                         // the slot is free once every share of its earlier pieces has left it
                         while (copied[p % RING].load(std::memory_order_acquire) < nth * (p / RING))
                             std::this_thread::yield();
-                        ANL_HIP(hipMemcpyAsync((char *)w.s.pin + p % RING * PIECE, (const char *)d + p * PIECE,
+                        ANL_HIP(hipMemcpyAsync(ring + p % RING * PIECE, (const char *)d + p * PIECE,
                                                std::min(PIECE, total - p * PIECE), hipMemcpyDeviceToHost, 0));
                         ANL_HIP(hipEventRecord(ev[p % RING], 0));
                     }
@@ -1259,8 +1336,7 @@ int anl_gk_calculate_mfma_async(anl_series *s, const uint32_t *idx_j, uint32_t n
                                          ANL_GK_MFMA, out_dev, nullptr, nullptr, stream);
 }
 
-// Synchronous host-output form: the output is staged in the series scratch,
-// after the space the MFMA form needs.
+// Synchronous host-output form.
 static int gk_calculate_host(anl_series *s, const uint32_t *idx_j, uint32_t ncur, uint32_t skip, uint32_t tmax,
                              uint32_t n, uint32_t n_seg, int subtract_mean, uint32_t start_mean, uint64_t primo,
                              double *out_host, int form) {
@@ -1270,17 +1346,15 @@ static int gk_calculate_host(anl_series *s, const uint32_t *idx_j, uint32_t ncur
         if (leff == 0) return;
         ensure_device();
         const size_t bytes = (size_t)leff * (3 * ncur * ncur + 2) * sizeof(double);
-        size_t front = form == ANL_GK_MFMA ? gk_mfma_scratch_bytes(s, ncur, leff, n)
-                                           : gk_fp64_scratch_bytes(ncur, leff, n_seg, 1);
-        if (form == ANL_GK_FP64 && front > GK_SEG_BYTES) front = 0;  // not used then
-        front = (front + 255) / 256 * 256;
-        char *w = (char *)series_workspace(s, front + bytes);
-        double *d = (double *)(w + front);
-        // both forms take their scratch from the front of the series scratch
-        int rc = anl_gk_calculate_blocks_async(s, idx_j, ncur, skip, tmax, n_seg, subtract_mean, start_mean, &primo,
-                                               &n, 1, form, d, nullptr, nullptr, 0);
-        if (rc != ANL_OK) throw Error{rc, anl_last_error()};
-        ANL_HIP(hipMemcpy(out_host, d, bytes, hipMemcpyDeviceToHost));
+        const GkWorkspace w(s, bytes, form == ANL_GK_FP64 ? gk_segment_bytes(ncur, leff, n_seg, 1) : 0, 0);
+        try {
+            gk_enqueue(s, idx_j, ncur, skip, leff, n_seg, subtract_mean, start_mean, &primo, &n, 1, form,
+                       w.dev(), nullptr, nullptr, w.segm, 0);
+            ANL_HIP(hipMemcpy(out_host, w.dev(), bytes, hipMemcpyDeviceToHost));
+        } catch (...) {
+            (void)hipStreamSynchronize(0);  // the workspace goes back unused
+            throw;
+        }
     });
 }
 

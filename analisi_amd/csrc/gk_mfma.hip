@@ -507,12 +507,6 @@ bool gkm_shape_ok(uint32_t q, uint32_t cs, uint32_t wg) {
     return (q == 4 || q == 8) && (cs == 8 || cs == 16) && (wg == 2 || wg == 4);
 }
 
-size_t gk_mfma_scratch_bytes(const anl_series *s, uint32_t ncur, uint32_t leff, uint32_t n) {
-    uint64_t bytes = 0;
-    gkm_batch_end(ncur, leff, &n, 1, 0, gkm_shape_of(s), &bytes);
-    return bytes;
-}
-
 void gk_mfma_enqueue_blocks(anl_series *s, const uint32_t *idx_j, uint32_t ncur, uint32_t skip, uint32_t leff,
                             uint32_t n_seg, const uint64_t *primo, const uint32_t *n, uint32_t nblocks, double *d,
                             hipStream_t st) {

@@ -574,6 +574,8 @@ int anl_series_destroy(anl_series *s) {
         if (!s) return;
         (void)hipDeviceSynchronize();
         (void)hipFree(s->work);
+        (void)hipFree(s->seg);
+        if (s->seg_done) (void)hipEventDestroy(s->seg_done);
         (void)hipFree(s->rec);
         (void)hipFree(s->data);
         delete s;

@@ -314,8 +314,12 @@ int anl_gk_calculate_blocks(anl_series *s, const uint32_t *idx_j, uint32_t ncur,
                             const uint32_t *n, uint32_t nblocks, int form, double *out_host, double *mean_host,
                             double *var_host);
 /* Stream-ordered variants writing [leff][3*ncur^2+2] FP64 to device memory.
- * Scratch lives in the series (grow-only; growing synchronises the device),
- * so the calls on one series must be ordered on one stream. */
+ * The MFMA form's scratch lives in the series (grow-only; growing
+ * synchronises the device), so its calls on one series must be ordered on one
+ * stream.  FP64 calls may come from any threads and go to any streams: those
+ * with n_seg > 1 take the series' segment means in turn, or do without them
+ * (their segments one after the other, same values) where they would exceed
+ * 64 MiB or the memory cannot be had, and on a stream under capture. */
 int anl_gk_calculate_async(anl_series *s, const uint32_t *idx_j, uint32_t ncur, uint32_t skip,
                            uint32_t tmax, uint32_t n, uint32_t n_seg, int subtract_mean,
                            uint32_t start_mean, uint64_t primo, double *out_dev, void *stream);

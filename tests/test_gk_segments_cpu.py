@@ -1,0 +1,105 @@
+"""The segment means of the FP64 Green-Kubo form (n_seg > 1) on a HIP runtime
+without kernels: which memory each launch is given.  Calls that run at once do
+not share it, a stream waits for the call that used it before, a captured
+launch holds no address of it, and a call that cannot have it does without."""
+import fake_hip
+
+SEGM = 11  # the word of GkArgs that holds the segment means
+
+_SETUP = """
+def seg_of(entries):
+    l = launches(entries, "gk_chain_kernel") + launches(entries, "gk_dense_kernel")
+    return [dict(x.split(":") for x in e[6:]).get("%d") for e in l]
+import ctypes
+J = np.zeros((9000, 6))
+s = capi.DeviceSeries(J)
+idx = np.array([0, 3], np.uint32)
+def run_async(out, tmax, n, stream=None):
+    p, k = np.zeros(1, np.uint64), np.full(1, n, np.uint32)
+    capi.check(capi.lib().anl_gk_calculate_blocks_async(s.handle, capi._ptr(idx), 2, 1, tmax, 4, 0, 0, capi._ptr(p),
+               capi._ptr(k), 1, capi.GK_FP64, out, None, None, stream))
+def device(nbytes):
+    p = ctypes.c_void_p()
+    assert fake.hipMalloc(ctypes.byref(p), ctypes.c_size_t(nbytes)) == 0
+    return p
+log()
+""" % SEGM
+
+
+def test_synchronous_calls_that_overlap(tmp_path_factory):
+    """A second, larger call made while the first has not ended: memory of its
+    own, and the first one's is not freed."""
+    fake_hip.run(_SETUP + """
+for blocks in (False, True):
+    inner = []
+    outer = []
+    def other():
+        outer.extend(log() if not inner else [])
+        if not inner and launches(outer, "gk_"):
+            s.gk([0, 3], 1, 3000, 5000, 4, False, 0, 0) if not blocks else s.gk_blocks(
+                [0, 3], 1, 2000, 4, False, 0, [0, 100], [4000, 4000])
+            inner.extend(log())
+    cb = WAIT(other)
+    fake.fake_wait(0, ctypes.cast(cb, ctypes.c_void_p))
+    s.gk([0, 3], 1, 500, 3000, 4, False, 0, 0) if not blocks else s.gk_blocks(
+        [0, 3], 1, 300, 4, False, 0, [0, 100], [2000, 2000])
+    fake.fake_wait(0, None)
+    a, b = seg_of(outer), seg_of(inner)
+    assert len(a) == 1 and len(b) == 1 and a[0] and b[0], (a, b)
+    assert a[0] != b[0]
+    first = [e[6:] for e in launches(outer, "gk_chain")]
+    held = {x.split(":")[1] for l in first for x in l}
+    assert not [e for e in inner if e[1] == "free" and e[2] in held]
+""", tmp_path_factory)
+
+
+def test_asynchronous_calls_on_two_streams(tmp_path_factory):
+    fake_hip.run(_SETUP + """
+st = [ctypes.c_void_p(0xa0), ctypes.c_void_p(0xb0)]
+out = device(3000 * 14 * 8)
+run_async(out, 3000, 5000, st[0])
+run_async(out, 400, 900, st[1])
+e = log()
+assert len(set(seg_of(e))) == 1 and seg_of(e)[0]      # the same memory,
+last = max(i for i, x in enumerate(e) if x[1] == "launch" and x[2] == "0xa0")
+first = min(i for i, x in enumerate(e) if x[1] == "launch" and x[2] == "0xb0")
+rec = [x for x in e[last:first] if x[1] == "record" and x[3] == "0xa0"]
+wait = [x for x in e[last:first] if x[1] == "waitevent" and x[2] == "0xb0"]
+assert rec and wait and rec[-1][2] == wait[-1][3]     # after the first call's end
+""", tmp_path_factory)
+
+
+def test_captured_call_keeps_no_address(tmp_path_factory):
+    fake_hip.run(_SETUP + """
+s.gk([0, 3], 1, 3000, 5000, 4, False, 0, 0)
+out = device(3000 * 14 * 8)
+run_async(out, 3000, 5000)
+log()
+fake.fake_capture(1)
+run_async(out, 400, 900)
+fake.fake_capture(0)
+e = log()
+assert seg_of(e) == [None] * 4 and not launches(e, "gk_segments_kernel"), e
+assert not [x for x in e if x[1] in ("malloc", "free", "record", "waitevent")]
+""", tmp_path_factory)
+
+
+def test_no_memory_for_the_segments(tmp_path_factory):
+    """A device with room for the outputs only."""
+    fake_hip.run(_SETUP + """
+seg = 3000 * 14 * 8 + 256                 # more than the output
+out = device(3000 * 14 * 8)
+fake.fake_refuse(seg, NEVER)
+r = s.gk([0, 3], 1, 3000, 5000, 4, False, 0, 0)
+e = log()
+assert seg_of(e) == [None] * 4 and not launches(e, "gk_segments_kernel")
+run_async(out, 3000, 5000)
+e = log()
+assert seg_of(e) == [None] * 4
+r = s.gk_blocks([0, 3], 1, 300, 4, False, 0, [0, 100, 200], [2000, 2000, 2000])
+e = log()
+assert len(seg_of(e)) == 1 and seg_of(e)[0]           # these fit
+fake.fake_refuse(NEVER, NEVER)
+r = s.gk([0, 3], 1, 3000, 5000, 4, False, 0, 0)
+assert seg_of(log())[0]
+""", tmp_path_factory)
