@@ -170,7 +170,9 @@ struct anl_series {
     double *data = nullptr;
     double2 *rec = nullptr;  // [nrows] 1/c, c = 1 .. nrows, in two parts (gk_reciprocals)
     // scratch of the MFMA form (splits, partial sums), grow-only; its calls on
-    // one series are stream-ordered on the caller's stream.
+    // one series are stream-ordered on the caller's stream, and each enqueues
+    // all that uses the scratch under the lock
+    std::mutex work_mutex;
     void *work = nullptr;
     size_t work_cap = 0;
     anl::ScratchPool scratch;  // of the synchronous calls: outputs, segment means of the FP64 form

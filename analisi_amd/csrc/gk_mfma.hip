@@ -517,6 +517,7 @@ void gk_mfma_enqueue_blocks(anl_series *s, const uint32_t *idx_j, uint32_t ncur,
         b0 = gkm_batch_end(ncur, leff, n, nblocks, b0, sh, &bytes);
         need = std::max(need, bytes);
     }
+    std::lock_guard<std::mutex> lock(s->work_mutex);
     char *work = (char *)series_workspace(s, need);
     const uint64_t stride = (uint64_t)leff * (3 * ncur * ncur + 2);
     // batches run one after the other on st, sharing the scratch

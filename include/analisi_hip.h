@@ -315,8 +315,8 @@ int anl_gk_calculate_blocks(anl_series *s, const uint32_t *idx_j, uint32_t ncur,
                             double *var_host);
 /* Stream-ordered variants writing [leff][3*ncur^2+2] FP64 to device memory.
  * The MFMA form's scratch lives in the series (grow-only; growing
- * synchronises the device), so its calls on one series must be ordered on one
- * stream.  FP64 calls may come from any threads and go to any streams: those
+ * synchronises the device), so its calls on one series must go to one stream
+ * (from any threads).  FP64 calls may come from any threads and go to any streams: those
  * with n_seg > 1 take the series' segment means in turn, or do without them
  * (their segments one after the other, same values) where they would exceed
  * 64 MiB or the memory cannot be had, and on a stream under capture. */

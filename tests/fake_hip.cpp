@@ -22,6 +22,7 @@ std::string lines;                           // the log
 uint64_t refuse_from = UINT64_MAX;           // bytes of a device allocation that is refused
 uint64_t refuse_after = UINT64_MAX;          // device allocations that still succeed
 unsigned wait_us = 0;                        // of every wait of the host
+unsigned launch_us = 0;                      // of every launch
 bool capturing = false;
 void (*on_wait)() = nullptr;                 // called at every wait of the host
 thread_local bool in_wait = false;
@@ -63,6 +64,7 @@ void fake_wait(unsigned us, void (*callback)()) {
     wait_us = us;
     on_wait = callback;
 }
+void fake_launch_time(unsigned us) { launch_us = us; }
 void fake_capture(int on) { capturing = on != 0; }
 size_t fake_log(char *out, size_t cap) {  // takes the log when it fits
     std::lock_guard<std::mutex> l(mu);
@@ -123,6 +125,7 @@ hipError_t hipLaunchKernel(const void *f, dim3 g, dim3 b, void **args, size_t, h
         bufs = (names.count(f) ? names[f] : "?") + bufs;
     }
     log("launch %p %u,%u,%u %u %s", (void *)s, g.x, g.y, g.z, b.x * b.y * b.z, bufs.c_str());
+    if (launch_us) usleep(launch_us);
     // the runtime's limits
     const bool bad = (uint64_t)g.x * b.x > UINT32_MAX || (uint64_t)g.y * b.y > UINT32_MAX ||
                      (uint64_t)g.z * b.z > UINT32_MAX || g.x == 0 || g.y == 0 || g.z == 0 || g.y > 65535 * 1024u;

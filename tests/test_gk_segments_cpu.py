@@ -103,3 +103,31 @@ fake.fake_refuse(NEVER, NEVER)
 r = s.gk([0, 3], 1, 3000, 5000, 4, False, 0, 0)
 assert seg_of(log())[0]
 """, tmp_path_factory)
+
+
+def test_matrix_form_from_two_threads(tmp_path_factory):
+    """The MFMA form's scratch: what one call enqueues on it is not mixed with
+    another thread's."""
+    fake_hip.run(_SETUP + """
+import threading
+fake.fake_launch_time(2000)
+go = threading.Barrier(2)
+def work(tmax):
+    go.wait()
+    for _ in range(5):
+        s.gk([0, 3], 1, tmax, 2000, 2, False, 0, 0, mfma=True)
+ts = [threading.Thread(target=work, args=(t,)) for t in (300, 500)]
+[t.start() for t in ts]
+[t.join() for t in ts]
+e = launches(log(), "gkm_")
+runs = [e[0][0]]
+for x in e:
+    if x[0] != runs[-1]:
+        runs.append(x[0])
+per_call = len(e) // 10
+assert per_call >= 4 and len(runs) <= 10, (per_call, len(runs))
+at = 0
+while at < len(e):                        # whole calls, one after the other
+    assert len({x[0] for x in e[at:at + per_call]}) == 1
+    at += per_call
+""", tmp_path_factory)
