@@ -242,25 +242,38 @@ void build_screen_order(anl_traj *tr) {
     tr->frac_order = d;
 }
 
+// The fractions and groups are the trajectory's only when all of them are on
+// the device: a call that fails on the way leaves nothing for the next one.
 void build_frac16(anl_traj *tr, hipStream_t s) {
     build_screen_order(tr);
     std::lock_guard<std::mutex> lock(tr->screen_mutex);
     if (tr->frac16) return;
-    uint64_t total = tr->F * tr->N;
-    ANL_HIP(hipMalloc(&tr->frac16, total * sizeof(uint2)));
-    ANL_HIP(hipMalloc(&tr->frac32, total * sizeof(uint4)));
-    ANL_HIP(hipMalloc(&tr->pos_scr, total * sizeof(double4)));
+    const uint64_t total = tr->F * tr->N;
     const uint32_t ngroups = (uint32_t)((tr->N + 31) / 32);
     const uint64_t gtotal = tr->F * ngroups;
-    ANL_HIP(hipMalloc(&tr->jgroups, gtotal * sizeof(uint4)));
-    unsigned blocks = (unsigned)((total + 255) / 256);
-    hipLaunchKernelGGL(frac_kernel, dim3(blocks), dim3(256), 0, s, tr->pos, tr->type_slot, tr->frac_order, tr->N,
-                       tr->frac16, tr->frac32, tr->pos_scr, total, tr->cell0);
+    struct Built {
+        uint2 *frac16 = nullptr;
+        uint4 *frac32 = nullptr, *jgroups = nullptr;
+        double4 *pos_scr = nullptr;
+        ~Built() {
+            for (void *p : {(void *)frac16, (void *)frac32, (void *)jgroups, (void *)pos_scr}) (void)hipFree(p);
+        }
+    } b;
+    ANL_HIP(hipMalloc(&b.frac16, total * sizeof(uint2)));
+    ANL_HIP(hipMalloc(&b.frac32, total * sizeof(uint4)));
+    ANL_HIP(hipMalloc(&b.pos_scr, total * sizeof(double4)));
+    ANL_HIP(hipMalloc(&b.jgroups, gtotal * sizeof(uint4)));
+    hipLaunchKernelGGL(frac_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, tr->pos, tr->type_slot,
+                       tr->frac_order, tr->N, b.frac16, b.frac32, b.pos_scr, total, tr->cell0);
     ANL_HIP(hipGetLastError());
-    hipLaunchKernelGGL(jgroup_kernel, dim3((unsigned)((gtotal + 255) / 256)), dim3(256), 0, s, tr->frac16, tr->N,
-                       ngroups, gtotal, tr->cell0, tr->jgroups);
+    hipLaunchKernelGGL(jgroup_kernel, dim3((unsigned)((gtotal + 255) / 256)), dim3(256), 0, s, b.frac16, tr->N, ngroups,
+                       gtotal, tr->cell0, b.jgroups);
     ANL_HIP(hipGetLastError());
     ANL_HIP(hipStreamSynchronize(s));
+    std::swap(tr->frac16, b.frac16);
+    std::swap(tr->frac32, b.frac32);
+    std::swap(tr->pos_scr, b.pos_scr);
+    std::swap(tr->jgroups, b.jgroups);
     (void)hipFree(tr->frac_order);  // the fractions hold the order from now on
     tr->frac_order = nullptr;
 }

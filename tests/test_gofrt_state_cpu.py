@@ -1,0 +1,56 @@
+"""State that g(r,t) calculations of one trajectory share, on a HIP runtime
+without kernels: what a failed call leaves behind, and what each launch is
+given while other calculations run."""
+import fake_hip
+
+_SETUP = """
+rng = np.random.default_rng(3)
+def trajectory(N=500, F=12, L=20.0, varying=False):
+    pos = rng.uniform(0, L, (F, N, 3))
+    box = np.zeros((F, 9))
+    box[:, 3:6] = L / 2
+    if varying:
+        box[:, 3] += 0.01 * np.arange(F)
+    return capi.DeviceTrajectory(pos, box[:, :6].copy(), np.zeros(N, np.int32), 1)
+def words(entry):
+    return {x.split(":")[0] for x in entry[6:]}
+"""
+
+
+def test_fractions_after_a_failed_allocation(tmp_path_factory):
+    """Each of the allocations of the screen's fractions refused once: the call
+    fails, frees what it had, and the next one builds all of them."""
+    fake_hip.run(_SETUP + """
+def new():
+    t = trajectory()
+    g = capi.DeviceGofrt(t, 0.0, 4.0, 20, 4)
+    g.reset(6)
+    return t, g
+t, g = new()
+log()
+g.calculate(0)
+e = log()
+want = words(launches(e, "gofrt_screened_kernel")[0])
+assert len(want) >= 8
+refused = 0
+for after in range(8):
+    t, g = new()
+    live = fake.fake_live()
+    fake.fake_refuse(NEVER, after)
+    try:
+        g.calculate(0)
+        ok = True
+    except capi.AnlError as err:
+        ok = False
+    fake.fake_refuse(NEVER, NEVER)
+    if ok:
+        break
+    refused += 1
+    log()
+    left = fake.fake_live()
+    g.calculate(0)
+    got = launches(log(), "gofrt_screened_kernel")[0]
+    assert words(got) == want, (after, sorted(got[6:]))
+    assert left <= live + (after > 0)                 # at most the pooled workspace
+assert refused >= 4
+""", tmp_path_factory)
