@@ -155,8 +155,6 @@ struct anl_traj {
     std::vector<int32_t> type_of_slot;  // host copy
     std::vector<uint64_t> type_count;   // atoms per type
     anl::Cell cell0;                    // cell of frame 0
-    anl::Screen screen_cache;
-    double screen_rmax = -1.0;
     uint32_t msd_tile = 16;             // lag tile of the MSD window kernel (anl_msd_set_tuning)
     uint32_t msd_waves = 4;             // its wavefronts per workgroup
     bool msd_auto = true;               // neither was chosen: each calculation takes its own lag tile

@@ -1935,6 +1935,7 @@ struct anl_gofrt {
     uint32_t nbin = 0, lmax = 0, skip = 1, every = 1;
     int form = ANL_GOFRT_AUTO;
     uint32_t n = 0, leff = 0;     // from reset()
+    Screen screen;                // of the trajectory's (constant) cell and rmax
     std::vector<double> thr;      // T[0..nbin]
     double lo = 0;
     double *d_thr = nullptr;
@@ -1956,13 +1957,9 @@ uint32_t nch_of(const anl_traj *tr) { return tr->nt * (tr->nt + 1); }
 
 int choose_form(anl_gofrt *g) {
     if (g->form == ANL_GOFRT_FP64) return ANL_GOFRT_FP64;
-    if (g->tr->screen_rmax != g->rmax) {
-        g->tr->screen_cache = make_screen(g->tr->cell0, g->tr->box_const, g->tr->nt, g->rmax);
-        g->tr->screen_rmax = g->rmax;
-    }
-    if (g->tr->screen_cache.valid) return ANL_GOFRT_SCREENED;
+    if (g->screen.valid) return ANL_GOFRT_SCREENED;
     if (g->form == ANL_GOFRT_SCREENED)
-        fail(ANL_ERR_ARG, "the screened g(r,t) form cannot be used: " + g->tr->screen_cache.why_not);
+        fail(ANL_ERR_ARG, "the screened g(r,t) form cannot be used: " + g->screen.why_not);
     return ANL_GOFRT_FP64;
 }
 
@@ -2249,7 +2246,7 @@ GofrtPrepared gofrt_prepare(anl_gofrt *g, const Launch &L, uint64_t out_len, int
     a.zero_d2 = g->rmin == 0.0 && g->thr[1] > 0x1p-140 ? 0.0f : -1.0f;
     a.rminf = (float)g->rmin;
     a.inv_drf = (float)(1.0 / g->dr);
-    a.threshold = form == ANL_GOFRT_SCREENED ? tr->screen_cache.threshold : 0;
+    a.threshold = form == ANL_GOFRT_SCREENED ? g->screen.threshold : 0;
     a.a0 = a0;
     a.a1 = a1;
     a.frac32 = tr->frac32;
@@ -2263,10 +2260,10 @@ GofrtPrepared gofrt_prepare(anl_gofrt *g, const Launch &L, uint64_t out_len, int
         a.cy = (float)(cl.L[1] * sc);
         a.cyz = (float)(cl.yz * sc);
         a.cz = (float)(cl.L[2] * sc);
-        a.du_margin = form == ANL_GOFRT_SCREENED ? du_window(tr->screen_cache, tr->triclinic, g->rmin, g->rmax, g->dr, g->nbin) : 0.0f;
+        a.du_margin = form == ANL_GOFRT_SCREENED ? du_window(g->screen, tr->triclinic, g->rmin, g->rmax, g->dr, g->nbin) : 0.0f;
         a.du_m0 = a.du_m1 = 0.0f;
         if (form == ANL_GOFRT_SCREENED)
-            du_window_offsets(tr->screen_cache, g->rmin, g->rmax, g->dr, g->nbin, &a.du_m0, &a.du_m1);
+            du_window_offsets(g->screen, g->rmin, g->rmax, g->dr, g->nbin, &a.du_m0, &a.du_m1);
         // cluster screen: cell entries times 2^-16, quantisation bound,
         // largest usable wavefront radius (cluster_params)
         const double sh = std::ldexp(1.0, -16);
@@ -2276,14 +2273,14 @@ GofrtPrepared gofrt_prepare(anl_gofrt *g, const Launch &L, uint64_t out_len, int
         a.hy = (float)(cl.L[1] * sh);
         a.hyz = (float)(cl.yz * sh);
         a.hz = (float)(cl.L[2] * sh);
-        const ClusterParams cp = cluster_params(tr->screen_cache, g->rmax);
+        const ClusterParams cp = cluster_params(g->screen, g->rmax);
         a.dq = (float)cp.dq;
         a.rmaxf = (float)cp.rmaxf;
         a.rho_cap = form == ANL_GOFRT_SCREENED ? (float)cp.rho_cap : 0.0f;
         a.jgroups = tr->jgroups;
         a.ngroups = (uint32_t)((tr->N + 31) / 32);
-        a.inv_w16 = form == ANL_GOFRT_SCREENED ? (float)(65536.0 / tr->screen_cache.wmin * (1 + 1e-6)) : 0.0f;
-        a.smin16 = form == ANL_GOFRT_SCREENED ? (float)(tr->screen_cache.smin * std::ldexp(1.0, -16) * (1 - 1e-6)) : 0.0f;
+        a.inv_w16 = form == ANL_GOFRT_SCREENED ? (float)(65536.0 / g->screen.wmin * (1 + 1e-6)) : 0.0f;
+        a.smin16 = form == ANL_GOFRT_SCREENED ? (float)(g->screen.smin * std::ldexp(1.0, -16) * (1 - 1e-6)) : 0.0f;
     }
     const uint32_t ntiles = (uint32_t)((tr->N + L.tile - 1) / L.tile);
     P.split = L.tile != WG;
@@ -2500,7 +2497,8 @@ int anl_gofrt_create(anl_traj *tr, double rmin, double rmax, uint32_t nbin, uint
             // (zero when the screen does not apply to this cell and rmax)
             std::vector<double> t(g->thr);
             t.resize(nbin + 1 + NFP64K, 0.0);
-            const Screen sc = make_screen(tr->cell0, tr->box_const, tr->nt, rmax);
+            g->screen = make_screen(tr->cell0, tr->box_const, tr->nt, rmax);
+            const Screen &sc = g->screen;
             if (sc.valid) {
                 const Cell &cl = tr->cell0;
                 const double f = std::ldexp(1.0, -32);

@@ -23,6 +23,7 @@ uint64_t refuse_from = UINT64_MAX;           // bytes of a device allocation tha
 uint64_t refuse_after = UINT64_MAX;          // device allocations that still succeed
 unsigned wait_us = 0;                        // of every wait of the host
 unsigned launch_us = 0;                      // of every launch
+unsigned dump = 0;                           // bytes of a launch's first argument in the log
 bool capturing = false;
 void (*on_wait)() = nullptr;                 // called at every wait of the host
 thread_local bool in_wait = false;
@@ -36,7 +37,7 @@ thread_local Config config;
 unsigned long tid() { return (unsigned long)std::hash<std::thread::id>()(std::this_thread::get_id()); }
 template <class... A>
 void log(const char *fmt, A... a) {
-    char s[1024];
+    char s[4096];
     std::snprintf(s, sizeof s, fmt, a...);
     std::lock_guard<std::mutex> l(mu);
     lines += std::to_string(tid()) + " " + s + "\n";
@@ -65,6 +66,7 @@ void fake_wait(unsigned us, void (*callback)()) {
     on_wait = callback;
 }
 void fake_launch_time(unsigned us) { launch_us = us; }
+void fake_dump(unsigned bytes) { dump = bytes; }
 void fake_capture(int on) { capturing = on != 0; }
 size_t fake_log(char *out, size_t cap) {  // takes the log when it fits
     std::lock_guard<std::mutex> l(mu);
@@ -123,6 +125,11 @@ hipError_t hipLaunchKernel(const void *f, dim3 g, dim3 b, void **args, size_t, h
             }
         }
         bufs = (names.count(f) ? names[f] : "?") + bufs;
+        if (dump) bufs += " =";
+        for (unsigned k = 0; args && k < dump; k++) {
+            std::snprintf(p, sizeof p, "%02x", ((unsigned char *)args[0])[k]);
+            bufs += p;
+        }
     }
     log("launch %p %u,%u,%u %u %s", (void *)s, g.x, g.y, g.z, b.x * b.y * b.z, bufs.c_str());
     if (launch_us) usleep(launch_us);

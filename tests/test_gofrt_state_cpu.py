@@ -54,3 +54,40 @@ for after in range(8):
     assert left <= live + (after > 0)                 # at most the pooled workspace
 assert refused >= 4
 """, tmp_path_factory)
+
+
+def test_two_cutoffs_at_once(tmp_path_factory):
+    """A calculation that another handle of the trajectory, with another rmax,
+    runs in the middle of is launched with its own screen."""
+    fake_hip.run(_SETUP + """
+t = trajectory()
+a, b = [capi.DeviceGofrt(t, 0.0, r, 20, 4) for r in (7.0, 2.0)]
+a.reset(6)
+b.reset(6)
+a.calculate(0)
+b.calculate(0)
+def values(entries):                     # of the launch, without its addresses
+    e = launches(entries, "gofrt_screened_kernel")
+    assert len(e) == 1
+    raw = bytes.fromhex(e[0][-1][1:])
+    ptr = {int(x.split(":")[0]) for x in e[0][6:-1]}
+    return [raw[8 * k:8 * k + 8] for k in range(len(raw) // 8) if k not in ptr]
+fake.fake_dump(480)
+log()
+a.calculate(0)
+alone = values(log())
+seen = []
+def other():
+    if not seen:
+        seen.append(log())
+        b.calculate(0)
+        seen.append(values(log()))
+cb = WAIT(other)
+fake.fake_wait(0, ctypes.cast(cb, ctypes.c_void_p))
+a.calculate(0)
+fake.fake_wait(0, None)
+e = log()
+assert len(seen) == 2 and not launches(seen[0], "gofrt_screened_kernel")
+assert seen[1] != alone
+assert values(e) == alone
+""", tmp_path_factory)
