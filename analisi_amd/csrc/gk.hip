@@ -335,6 +335,12 @@ __global__ __launch_bounds__(256, 1) void gk_chain_kernel(const GkArgs a) {
         for (uint32_t k = np; k < a.narr; k++) o[k] = 0.0;
 }
 
+__device__ __forceinline__ void wave_sync_lds() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // The same chains for launches that fill the chip, t0 stride 1: one wavefront
 // = 64 lags of CH pairs (ja, jb0 ..) or, with one current, CH x 64 lags, CH
 // running means per lane that share Ja and 1/cont.  What bounds it is the
@@ -474,12 +480,19 @@ __global__ __launch_bounds__(64, 3) void gk_dense_kernel(const GkArgs a) {
     };
     Lane f0{}, f1{};
     if (nst) fetch(f0);
+    // the rows pass between lanes: neither the stage's reads nor the next
+    // stage's stores may move across (the hardware keeps their order, the
+    // compiler would not have to)
     for (uint32_t k = 0; k < nst; k += 2) {
+        wave_sync_lds();
         stash();
+        wave_sync_lds();
         if (k + 1 < nst) fetch(f1);
         stage(k, f0);
         if (k + 1 < nst) {
+            wave_sync_lds();
             stash();
+            wave_sync_lds();
             if (k + 2 < nst) fetch(f0);
             stage(k + 1, f1);
         }
