@@ -13,6 +13,8 @@
 //    Schur complement of the symmetrised integral matrix.
 #include <algorithm>
 #include <atomic>
+#include <chrono>
+#include <condition_variable>
 #include <cstring>
 #include <optional>
 #include <thread>
@@ -1273,19 +1275,41 @@ int anl_gk_calculate_blocks(anl_series *s, const uint32_t *idx_j, uint32_t ncur,
         constexpr int64_t NOT_YET = -1, GIVE_UP = -2;  // no kernels yet; there will be no output
         std::atomic<int64_t> arrived{NOT_YET};         // pieces in the ring so far
         std::atomic<uint64_t> copied[RING] = {};       // shares copied out of each of its slots
+        std::mutex mu;
+        std::condition_variable news;
+        auto publish = [&](int64_t v) {
+            {
+                std::lock_guard<std::mutex> lock(mu);
+                arrived.store(v, std::memory_order_release);
+            }
+            news.notify_all();
+        };
+        // more than v pieces (false: there will be none).  Pieces follow each
+        // other in tens of us, less than a thread takes to wake, so it looks
+        // for them for a while before it sleeps; the kernels may take seconds.
+        auto await = [&](int64_t v) {
+            const auto until = std::chrono::steady_clock::now() + std::chrono::microseconds(200);
+            int64_t a;
+            while ((a = arrived.load(std::memory_order_acquire)) <= v && a != GIVE_UP) {
+                if (std::chrono::steady_clock::now() < until) {
+                    std::this_thread::yield();
+                } else {
+                    std::unique_lock<std::mutex> lock(mu);
+                    news.wait(lock, [&] { return arrived.load() > v || arrived.load() == GIVE_UP; });
+                }
+            }
+            return a != GIVE_UP;
+        };
         // thread k's share of piece p: [first, last) of the output
         auto share = [&](size_t p, unsigned k) {
             return p * PIECE + std::min(PIECE, total - p * PIECE) * k / nth;
         };
         auto work = [&](unsigned k) {
-            int64_t a;
-            while ((a = arrived.load(std::memory_order_acquire)) == NOT_YET) std::this_thread::yield();
-            if (a == GIVE_UP) return;
+            if (!await(NOT_YET)) return;
             for (size_t p = 0; p < pieces; p++)
                 for (size_t b = share(p, k); b < share(p, k + 1); b += 4096) ((volatile char *)out_host)[b] = 0;
             for (size_t p = 0; p < pieces; p++) {
-                while ((a = arrived.load(std::memory_order_acquire)) <= (int64_t)p && a != GIVE_UP) std::this_thread::yield();
-                if (a == GIVE_UP) return;
+                if (!await((int64_t)p)) return;
                 const size_t b0 = share(p, k), b1 = share(p, k + 1);
                 std::memcpy((char *)out_host + b0, ring + p % RING * PIECE + (b0 - p * PIECE), b1 - b0);
                 copied[p % RING].fetch_add(1, std::memory_order_release);
@@ -1304,7 +1328,7 @@ int anl_gk_calculate_blocks(anl_series *s, const uint32_t *idx_j, uint32_t ncur,
             if (nth) {
                 pool.reserve(nth);
                 for (unsigned k = 0; k < nth; k++) pool.emplace_back(work, k);
-                arrived.store(0, std::memory_order_release);
+                publish(0);
                 for (hipEvent_t &e : ev) ANL_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
                 for (size_t p = 0; p <= pieces; p++) {
                     if (p < pieces) {
@@ -1317,7 +1341,7 @@ int anl_gk_calculate_blocks(anl_series *s, const uint32_t *idx_j, uint32_t ncur,
                     }
                     if (p) {
                         ANL_HIP(hipEventSynchronize(ev[(p - 1) % RING]));
-                        arrived.store((int64_t)p, std::memory_order_release);
+                        publish((int64_t)p);
                     }
                 }
             } else if (total) {
@@ -1327,7 +1351,7 @@ int anl_gk_calculate_blocks(anl_series *s, const uint32_t *idx_j, uint32_t ncur,
             if (var_host && len) ANL_HIP(hipMemcpy(var_host, d + all + len, len * sizeof(double), hipMemcpyDeviceToHost));
         } catch (...) {
             (void)hipStreamSynchronize(0);  // the workspace goes back unused
-            arrived.store(GIVE_UP, std::memory_order_release);
+            publish(GIVE_UP);
             end();
             throw;
         }

@@ -131,3 +131,24 @@ while at < len(e):                        # whole calls, one after the other
     assert len({x[0] for x in e[at:at + per_call]}) == 1
     at += per_call
 """, tmp_path_factory)
+
+
+def test_copy_threads_sleep_while_the_kernels_run(tmp_path_factory):
+    """gk_blocks' copy threads: a device that takes two seconds keeps less
+    than half a core of the host busy (eight when the threads look all the time;
+    the kernel counts their time in ticks, which is coarse)."""
+    fake_hip.run(_SETUP + """
+import resource, time
+def cpu():
+    r = resource.getrusage(resource.RUSAGE_SELF)
+    return r.ru_utime + r.ru_stime
+primo = list(range(0, 1400, 50))
+used = []
+for wait in (0, 0, 1000000):
+    fake.fake_wait(wait, None)
+    c, t = cpu(), time.perf_counter()
+    s.gk_blocks([0, 3], 500, 1000, 1, False, 0, primo, [2000] * len(primo), stats=False)  # 3 MB, two pieces
+    used.append(cpu() - c)
+    t = time.perf_counter() - t
+assert t > 1.9 and used[2] < t / 2, (used, t)
+""", tmp_path_factory)
