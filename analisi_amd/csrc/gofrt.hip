@@ -2477,13 +2477,15 @@ int anl_gofrt_create(anl_traj *tr, double rmin, double rmax, uint32_t nbin, uint
         g->skip = skip == 0 ? 1 : skip;     // calculatemultithread.h:43-46
         g->every = every == 0 ? 1 : every;
         g->form = form;
-        if (const char *e = std::getenv("ANL_GOFRT_UNROLL")) g->tune.unroll = std::atoi(e) == 8 ? 8 : 4;
-        if (const char *e = std::getenv("ANL_GOFRT_XCD")) g->tune.xcd = std::atoi(e) != 0;
-        if (const char *e = std::getenv("ANL_GOFRT_CLUSTER")) {
-            g->tune.cluster = std::min(4, std::max(0, std::atoi(e)));
-            g->tuned = true;
-        }
-        if (const char *e = std::getenv("ANL_GOFRT_PAIRS_PER_WG")) {
+        auto chosen = [&](const char *name) {
+            const char *e = std::getenv(name);
+            g->tuned |= e != nullptr;
+            return e;
+        };
+        if (const char *e = chosen("ANL_GOFRT_UNROLL")) g->tune.unroll = std::atoi(e) == 8 ? 8 : 4;
+        if (const char *e = chosen("ANL_GOFRT_XCD")) g->tune.xcd = std::atoi(e) != 0;
+        if (const char *e = chosen("ANL_GOFRT_CLUSTER")) g->tune.cluster = std::min(4, std::max(0, std::atoi(e)));
+        if (const char *e = chosen("ANL_GOFRT_PAIRS_PER_WG")) {
             long long v = std::atoll(e);
             if (v > 0) g->tune.pairs_per_wg = (uint64_t)v;
         }

@@ -23,6 +23,7 @@ uint64_t refuse_from = UINT64_MAX;           // bytes of a device allocation tha
 uint64_t refuse_after = UINT64_MAX;          // device allocations that still succeed
 unsigned wait_us = 0;                        // of every wait of the host
 unsigned launch_us = 0;                      // of every launch
+int fill = 0;                                // byte that device memory is filled with
 unsigned dump = 0;                           // bytes of a launch's first argument in the log
 bool capturing = false;
 void (*on_wait)() = nullptr;                 // called at every wait of the host
@@ -67,6 +68,7 @@ void fake_wait(unsigned us, void (*callback)()) {
 }
 void fake_launch_time(unsigned us) { launch_us = us; }
 void fake_dump(unsigned bytes) { dump = bytes; }
+void fake_fill(int byte) { fill = byte; }
 void fake_capture(int on) { capturing = on != 0; }
 size_t fake_log(char *out, size_t cap) {  // takes the log when it fits
     std::lock_guard<std::mutex> l(mu);
@@ -147,6 +149,7 @@ hipError_t hipMalloc(void **p, size_t n) {
     if (refuse_after != UINT64_MAX) refuse_after--;
     char *q = (char *)std::calloc(1, n + 64);
     if (!q) return last = hipErrorOutOfMemory;
+    if (fill) std::memset(q, fill, n);
     blocks[q] = n;
     *p = q;
     return hipSuccess;

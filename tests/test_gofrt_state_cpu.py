@@ -91,3 +91,31 @@ assert len(seen) == 2 and not launches(seen[0], "gofrt_screened_kernel")
 assert seen[1] != alone
 assert values(e) == alone
 """, tmp_path_factory)
+
+
+def test_shape_from_the_environment(tmp_path_factory):
+    """Each of the environment's launch settings, like anl_gofrt_set_tuning, is a
+    choice of the shape: the default cluster mode is then kept where an untuned
+    calculation would leave it (here groups 12 A wide in a cell of 40)."""
+    fake_hip.run(_SETUP + """
+import os
+fake.fake_fill(0x41)                      # 0x41414141: a radius of 12.1 A
+t = trajectory(L=40.0)
+def kernel(env, tune=None):
+    os.environ.update(env)
+    g = capi.DeviceGofrt(t, 0.0, 4.0, 20, 4)
+    for k in env:
+        del os.environ[k]
+    if tune:
+        g.set_tuning(*tune)
+    g.reset(6)
+    log()
+    g.calculate(0)
+    return launches(log(), "gofrt_screened_kernel")[0][5]
+untuned = kernel({})
+chosen = kernel({}, (4, 1, 1 << 26, 2))
+assert untuned != chosen
+for env in (dict(ANL_GOFRT_UNROLL="4"), dict(ANL_GOFRT_XCD="1"), dict(ANL_GOFRT_PAIRS_PER_WG=str(1 << 26)),
+            dict(ANL_GOFRT_CLUSTER="2")):
+    assert kernel(env) == chosen, env
+""", tmp_path_factory)
