@@ -40,6 +40,7 @@ SIGNATURES = [
     ("anl_info", ctypes.c_char_p, []),
     ("anl_traj_create", _i, [_vp, _vp, _u32, _vp, _u32, _vp, _u64, _u64, _pp]),
     ("anl_traj_destroy", _i, [_vp]),
+    ("anl_traj_prepare_gofrt", _i, [_vp, _vp, ctypes.c_double]),
     ("anl_gofrt_create", _i, [_vp, _d, _d, _u32, _u32, _u32, _u32, _i, _pp]),
     ("anl_gofrt_destroy", _i, [_vp]),
     ("anl_gofrt_reset", _i, [_vp, _u32, ctypes.POINTER(_u32)]),

@@ -153,6 +153,7 @@ struct anl_traj {
                                         // {centre a | b << 16, centre c, radius (float bits, A), 0}
     std::vector<double> box_host;       // [F][9]
     std::vector<int32_t> type_of_slot;  // host copy
+    std::vector<int32_t> orig_of_slot;  // host copy
     std::vector<uint64_t> type_count;   // atoms per type
     anl::Cell cell0;                    // cell of frame 0
     uint32_t msd_tile = 16;             // lag tile of the MSD window kernel (anl_msd_set_tuning)
@@ -190,7 +191,7 @@ Cell cell_of(const double *box9);
 // (int)floorf((float)((sqrt(d2) - rmin) / dr)) is >= k, computed on the host
 // with IEEE double arithmetic (gofrt.cpp:114-115, sphericalbase.cpp:52-53).
 std::vector<double> bin_edges(double rmin, double rmax, uint32_t nbin, double dr);
-void build_screen_order(anl_traj *tr);
+void build_screen_order(anl_traj *tr, const double *pos);
 void build_frac16(anl_traj *tr, hipStream_t s);
 
 // Prepared launches for the block engine: all host work (checks, plans,

@@ -2512,7 +2512,7 @@ int anl_gofrt_create(anl_traj *tr, double rmin, double rmax, uint32_t nbin, uint
                 k[FP64K_YZ] = cl.yz * f;
                 k[FP64K_Z] = cl.L[2] * f;
                 k[FP64K_EPS] = d2_window_fp64(sc, cl, tr->pos_max, rmax);
-                if (form != ANL_GOFRT_FP64) build_screen_order(tr);
+                if (form != ANL_GOFRT_FP64) build_screen_order(tr, nullptr);
             }
             ANL_HIP(hipMalloc(&g->d_thr, t.size() * sizeof(double)));
             ANL_HIP(hipMemcpy(g->d_thr, t.data(), t.size() * sizeof(double), hipMemcpyHostToDevice));
@@ -2528,6 +2528,15 @@ int anl_gofrt_create(anl_traj *tr, double rmin, double rmax, uint32_t nbin, uint
         ANL_HIP(hipMemcpy(g->d_chan, chan.data(), chan.size() * sizeof(int32_t), hipMemcpyHostToDevice));
         ANL_HIP(hipMalloc(&g->d_ncand, NSTAT * sizeof(unsigned long long)));
         *out = owner.release();
+    });
+}
+
+int anl_traj_prepare_gofrt(anl_traj *tr, const double *pos, double rmax) {
+    return guard([&] {
+        if (!tr || !pos) fail(ANL_ERR_ARG, "null pointer passed to anl_traj_prepare_gofrt");
+        if (!make_screen(tr->cell0, tr->box_const, tr->nt, rmax).valid) return;
+        ensure_device();
+        build_screen_order(tr, pos);
     });
 }
 

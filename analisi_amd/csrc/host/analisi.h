@@ -301,6 +301,8 @@ class Trajectory_numpy {
         }
         return dev;
     }
+    // the positions of device()'s frames
+    const double *device_positions() const { return pos_.data(); }
 
    private:
     struct Lcell {
@@ -494,6 +496,11 @@ class ReadLog_numpy {
 // ---------------------------------------------------------------------------
 // Gofrt (gofrt.h:28-107, gofrt.cpp)
 // ---------------------------------------------------------------------------
+// readers that prepare the windows they read ahead for the g(r,t) objects
+template <class X, class = void>
+struct prepares_ahead : std::false_type {};
+template <class X>
+struct prepares_ahead<X, std::void_t<decltype(std::declval<X &>().expect_gofrt(0.0))>> : std::true_type {};
 // whether a trajectory holds frames a device handle can be built over now:
 // a windowed trajectory only once its window has been read
 template <class X, class = void>
@@ -519,6 +526,8 @@ class Gofrt : public VectorOp<Gofrt<TFLOAT, T>, TFLOAT> {
           unsigned int skip = 1, unsigned int every = 1, bool debug = false, int form = ANL_GOFRT_AUTO)
         : traiettoria(t), rmin(rmin), rmax(rmax), nbin(nbin), lmax(tmax), nthreads(nthreads == 0 ? 1 : nthreads),
           skip(skip == 0 ? 1 : skip), every(every == 0 ? 1 : every), debug(debug), form(form) {
+        if constexpr (prepares_ahead<T>::value)
+            if (form != ANL_GOFRT_FP64) expected = t->expect_gofrt(rmax);
         if (has_frames(t)) h();  // argument errors surface here
     }
     ~Gofrt() {
@@ -601,6 +610,7 @@ class Gofrt : public VectorOp<Gofrt<TFLOAT, T>, TFLOAT> {
             anl_traj *d = traiettoria->device();
             if (g) anl_gofrt_destroy(g);
             g = nullptr;
+            if (form != ANL_GOFRT_FP64) anl_check(anl_traj_prepare_gofrt(d, traiettoria->device_positions(), rmax));
             anl_check(anl_gofrt_create(d, rmin, rmax, nbin, lmax, skip, every, form, &g));
             gen = traiettoria->generation();
             if (reset_done) anl_check(anl_gofrt_reset(g, ntimesteps, nullptr));
@@ -642,6 +652,7 @@ class Gofrt : public VectorOp<Gofrt<TFLOAT, T>, TFLOAT> {
     bool reset_done = false;
     uint64_t gen = 0;
     anl_gofrt *g = nullptr;
+    std::shared_ptr<const double> expected;  // rmax, for the reader, while this object exists
     std::string c_descr;
 };
 

@@ -139,7 +139,7 @@ class Trajectory {
     }
     ~Trajectory() {
         cancel_prefetch();
-        if (dev) anl_traj_destroy(dev);
+        drop_device();
         if (file) munmap((void *)file, fsize);
         if (fd != -1) close(fd);
     }
@@ -151,6 +151,7 @@ class Trajectory {
         if (!ok) return non_inizializzato;
         if (loaded_timesteps == n) return Ok;
         cancel_prefetch();
+        if (preparing.valid()) preparing.wait();  // it reads the positions
         dati_caricati = false;
         loaded_timesteps = n;
         pos_.assign(n * natoms * 3, 0.0);
@@ -175,7 +176,7 @@ class Trajectory {
                 adopt(w);
                 return Ok;
             }
-            if (w.dev) anl_traj_destroy(w.dev);
+            discard(w);
         }
         dati_caricati = false;
         Window w;
@@ -186,10 +187,12 @@ class Trajectory {
     }
 
     // Starts reading the window at ts, and building its device mirror, on a
-    // host thread: the reads, the host-side ordering and the uploads (on a
-    // stream of their own) overlap the work on the current window.  The next
-    // set_access_at(ts) adopts it; another prefetch or a window size change
-    // discards it.  A hint only: results never depend on it.
+    // host thread: the reads and the uploads (on a stream of their own) overlap
+    // the work on the current window.  Where a screened g(r,t) object waits for
+    // it, a second thread then orders the atoms of each frame, beside that work
+    // and beside the reading of the window after.  The next set_access_at(ts)
+    // adopts the window; another prefetch or a window size change discards it.
+    // A hint only: results never depend on it.
     void prefetch(size_t ts) {
         if (!ok || loaded_timesteps == 0 || !prefetching) return;
         if (ts + loaded_timesteps > n_timesteps) return;
@@ -197,13 +200,21 @@ class Trajectory {
         cancel_prefetch();
         ahead_start = ts;
         std::vector<size_t> offs = window_offsets(ts);  // indexes the file here, not on the reader
-        ahead = std::async(std::launch::async, [this, ts, offs]() {
+        const double rmax = expected_rmax();
+        ahead = std::async(std::launch::async, [this, ts, offs, rmax]() {
             Window w;
             w.start = ts;
             load_window(offs, w);
             std::vector<int32_t> tid(type_id.begin(), type_id.end());
             anl_check(anl_traj_create(w.pos.data(), w.boxes.data(), (uint32_t)box_stride, tid.data(),
                                       (uint32_t)ntypes, w.pcm.data(), loaded_timesteps, natoms, &w.dev));
+            // an error of this is met again, and reported, by anl_gofrt_create
+            if (rmax > 0) try {
+                    w.preparing = std::async(std::launch::async, [d = w.dev, p = w.pos.data(), rmax] {
+                        (void)anl_traj_prepare_gofrt(d, p, rmax);
+                    });
+                } catch (...) {
+                }
             return w;
         });
     }
@@ -211,7 +222,7 @@ class Trajectory {
         if (!ahead.valid()) return;
         try {
             Window w = ahead.get();
-            if (w.dev) anl_traj_destroy(w.dev);
+            discard(w);
         } catch (...) {
             // a discarded window's error does not concern the caller
         }
@@ -318,6 +329,14 @@ class Trajectory {
         next_start = std::min(primo, n_timesteps - loaded_timesteps);  // window_offset's rule
         next_set = true;
     }
+    // While the returned pointer is held, windows read ahead are prepared for
+    // a screened g(r,t) up to rmax.
+    std::shared_ptr<const double> expect_gofrt(double rmax) {
+        (void)expected_rmax();  // drops those that have gone
+        auto p = std::make_shared<const double>(rmax);
+        gofrts.push_back(p);
+        return p;
+    }
     // changes whenever the window's contents change; operators rebuild their
     // device handles when it does
     uint64_t generation() const { return generation_; }
@@ -327,8 +346,7 @@ class Trajectory {
         if (!dati_caricati || loaded_timesteps == 0)
             throw std::runtime_error("no timesteps are loaded: call setAccessWindowSize and setAccessStart first");
         if (!dev || dev_generation != generation_) {
-            if (dev) anl_traj_destroy(dev);
-            dev = nullptr;
+            drop_device();
             std::vector<int32_t> tid(type_id.begin(), type_id.end());
             anl_check(anl_traj_create(pos_.data(), boxes.data(), (uint32_t)box_stride, tid.data(), (uint32_t)ntypes,
                                       pcm_.data(), loaded_timesteps, natoms, &dev));
@@ -336,14 +354,42 @@ class Trajectory {
         }
         return dev;
     }
+    // the positions of device()'s frames, once a thread that prepares them has ended
+    const double *device_positions() const {
+        if (preparing.valid()) preparing.wait();
+        return pos_.data();
+    }
 
    private:
+    // the smallest rmax that a g(r,t) object waits for, 0 without one (the
+    // order is the same for all, and the screen applies to small rmax first)
+    double expected_rmax() {
+        double rmax = 0;
+        auto end = std::remove_if(gofrts.begin(), gofrts.end(), [&](const std::weak_ptr<const double> &w) {
+            const auto p = w.lock();
+            if (p && (rmax == 0 || *p < rmax)) rmax = *p;
+            return !p;
+        });
+        gofrts.erase(end, gofrts.end());
+        return rmax;
+    }
     // one window's host arrays (and, when read ahead, its device mirror)
     struct Window {
         size_t start = 0;
         std::vector<double> pos, vel, pcm, vcm, boxes;
         anl_traj *dev = nullptr;
+        std::future<void> preparing;  // works on dev and reads pos (its own buffer, wherever the vector goes)
     };
+    static void discard(Window &w) {
+        if (w.preparing.valid()) w.preparing.wait();
+        if (w.dev) anl_traj_destroy(w.dev);
+        w.dev = nullptr;
+    }
+    void drop_device() {
+        if (preparing.valid()) preparing.wait();
+        if (dev) anl_traj_destroy(dev);
+        dev = nullptr;
+    }
     std::vector<size_t> window_offsets(size_t ts) {
         std::vector<size_t> offs(loaded_timesteps);
         for (size_t k = 0; k < loaded_timesteps; k++) offs[k] = offset_of(ts + k);
@@ -409,6 +455,7 @@ class Trajectory {
         }
     }
     void adopt(Window &w) {
+        if (preparing.valid()) preparing.wait();  // the positions go
         pos_.swap(w.pos);
         vel_.swap(w.vel);
         pcm_.swap(w.pcm);
@@ -418,8 +465,10 @@ class Trajectory {
         current_timestep = w.start;
         generation_++;
         if (w.dev) {
-            if (dev) anl_traj_destroy(dev);
+            drop_device();
             dev = w.dev;
+            w.dev = nullptr;
+            preparing = std::move(w.preparing);
             dev_generation = generation_;
         }
     }
@@ -545,7 +594,9 @@ class Trajectory {
     std::vector<double> pos_, vel_, pcm_, vcm_, boxes;
     uint64_t generation_ = 0, dev_generation = 0;
     anl_traj *dev = nullptr;
+    std::future<void> preparing;  // of dev, from pos_
     std::future<Window> ahead;  // window being read ahead by prefetch()
+    std::vector<std::weak_ptr<const double>> gofrts;  // see expect_gofrt
     size_t ahead_start = 0, next_start = 0;
     bool prefetching = true, next_set = false;
 };

@@ -202,29 +202,41 @@ static void kd_order(int32_t *order, const std::array<float, 3> *fr, size_t lo, 
 // Screen order, per frame: the bisection of the slot order applied to that
 // frame's positions, so that the atoms of one wavefront stay compact in every
 // frame while they diffuse.  frac_order[f][s] = slot of the atom at screen slot
-// s.  Only the screened g(r,t) needs it (constant cell): its handle builds it,
-// from the device's positions, and every other calculation does without (the
-// first MSD over a new trajectory, 8,192 atoms x 1,000 frames: 124 -> 32 ms, with the
-// checks and the staging of the positions on several threads).
-void build_screen_order(anl_traj *tr) {
+// s.  Only the screened g(r,t) needs it (constant cell), and every other
+// calculation does without (the first MSD over a new trajectory, 8,192 atoms x
+// 1,000 frames: 124 -> 32 ms, with the checks and the staging of the positions
+// on several threads).  pos: the positions as given to anl_traj_create, or null
+// to read them back; with them nothing here waits for the null stream's
+// kernels, so that a thread that reads ahead can do it beside them.
+void build_screen_order(anl_traj *tr, const double *pos) {
     std::lock_guard<std::mutex> lock(tr->screen_mutex);
     if (tr->frac16 || tr->frac_order) return;
     const uint64_t N = tr->N, F = tr->F;
     const double len[3] = {tr->cell0.L[0], tr->cell0.L[1], tr->cell0.L[2]};
-    const uint64_t chunk = std::min<uint64_t>(F, std::max<uint64_t>(1, (64u << 20) / (N * sizeof(double4))));
-    std::vector<double4> pos(chunk * N);
+    const uint64_t chunk = pos ? F : std::min<uint64_t>(F, std::max<uint64_t>(1, (64u << 20) / (N * sizeof(double4))));
+    std::vector<double4> back(pos ? 0 : chunk * N);
     std::vector<int32_t> ford(F * N);
     for (uint64_t f0 = 0; f0 < F; f0 += chunk) {
         const uint64_t nf = std::min(chunk, F - f0);
-        ANL_HIP(hipMemcpy(pos.data(), tr->pos + f0 * N, nf * N * sizeof(double4), hipMemcpyDeviceToHost));
+        if (!pos) ANL_HIP(hipMemcpy(back.data(), tr->pos + f0 * N, nf * N * sizeof(double4), hipMemcpyDeviceToHost));
         parallel(nf, 1, [&](unsigned, uint64_t i0, uint64_t i1) {
                 std::vector<std::array<float, 3>> fs(N);
                 for (uint64_t f = i0; f < i1; f++) {
                     for (uint64_t sl = 0; sl < N; sl++) {
-                        const double4 x = pos[f * N + sl];
-                        double s3[3];
-                        to_fractional(tr->cell0, x.x, x.y, x.z, s3);
-                        for (int c = 0; c < 3; c++) fs[sl][c] = (float)(s3[c] - std::floor(s3[c]));
+                        double x[3], s3[3];
+                        if (pos) {
+                            const double *q = pos + ((f0 + f) * N + (uint64_t)tr->orig_of_slot[sl]) * 3;
+                            for (int c = 0; c < 3; c++) x[c] = q[c];
+                        } else {
+                            const double4 q = back[f * N + sl];
+                            x[0] = q.x, x[1] = q.y, x[2] = q.z;
+                        }
+                        to_fractional(tr->cell0, x[0], x[1], x[2], s3);
+                        for (int c = 0; c < 3; c++) {
+                            // an order whatever the caller's array holds by now
+                            const float v = (float)(s3[c] - std::floor(s3[c]));
+                            fs[sl][c] = v >= 0.0f ? v : 0.0f;
+                        }
                     }
                     int32_t *o = ford.data() + (f0 + f) * N;
                     std::iota(o, o + N, 0);
@@ -232,20 +244,43 @@ void build_screen_order(anl_traj *tr) {
                 }
             });
     }
-    int32_t *d = nullptr;
-    ANL_HIP(hipMalloc(&d, F * N * sizeof(int32_t)));
-    const hipError_t e = hipMemcpy(d, ford.data(), F * N * sizeof(int32_t), hipMemcpyHostToDevice);
-    if (e != hipSuccess) {
-        (void)hipFree(d);
-        ANL_HIP(e);
+    // beside a running kernel: on a stream of its own, through the pinned memory
+    // that the trajectory's creation left (a copy from pageable memory waits
+    // until the kernel leaves room for it)
+    struct Up {
+        hipStream_t s = nullptr;
+        int32_t *d = nullptr;
+        ~Up() {
+            if (s) {
+                (void)hipStreamSynchronize(s);
+                (void)hipStreamDestroy(s);
+            }
+            (void)hipFree(d);
+        }
+    };
+    const size_t bytes = F * N * sizeof(int32_t);
+    Up up;
+    ANL_HIP(hipMalloc(&up.d, bytes));
+    if (pos) {
+        const size_t piece = std::min<size_t>(bytes, 4u << 20);
+        const ScratchLease w(tr->scratch, 0, piece);
+        ANL_HIP(hipStreamCreateWithFlags(&up.s, hipStreamNonBlocking));
+        for (size_t at = 0; at < bytes; at += piece) {
+            const size_t n = std::min(piece, bytes - at);
+            std::memcpy(w.s.pin, (const char *)ford.data() + at, n);
+            ANL_HIP(hipMemcpyAsync((char *)up.d + at, w.s.pin, n, hipMemcpyHostToDevice, up.s));
+            ANL_HIP(hipStreamSynchronize(up.s));
+        }
+    } else {
+        ANL_HIP(hipMemcpy(up.d, ford.data(), bytes, hipMemcpyHostToDevice));
     }
-    tr->frac_order = d;
+    std::swap(tr->frac_order, up.d);
 }
 
 // The fractions and groups are the trajectory's only when all of them are on
 // the device: a call that fails on the way leaves nothing for the next one.
 void build_frac16(anl_traj *tr, hipStream_t s) {
-    build_screen_order(tr);
+    build_screen_order(tr, nullptr);
     std::lock_guard<std::mutex> lock(tr->screen_mutex);
     if (tr->frac16) return;
     const uint64_t total = tr->F * tr->N;
@@ -416,15 +451,18 @@ struct Uploader {
         }
     }
     void finish() { ANL_HIP(hipStreamSynchronize(s)); }
-    // after finish(): one staging buffer becomes the first pinned workspace of
-    // the trajectory's calculations (allocating another would cost the first
-    // of them 0.35 ms)
+    // after finish(): the staging buffers become pinned workspaces of the
+    // trajectory's calculations.  Allocating another would cost the first of
+    // them 0.35 ms, and freeing one waits for every kernel that runs: a thread
+    // that reads ahead would wait out the calculation it works beside.
     void keep(ScratchPool &pool) {
-        Scratch w;
-        w.pin = stage[0];
-        w.pin_cap = cap;
-        stage[0] = nullptr;
-        pool.give(w);
+        for (void *&p : stage) {
+            Scratch w;
+            w.pin = p;
+            w.pin_cap = cap;
+            p = nullptr;
+            pool.give(w);
+        }
     }
 };
 
@@ -540,6 +578,7 @@ int anl_traj_create(const double *pos, const double *box, uint32_t box_stride, c
             up.put(tr->cm, pos_cm, nframes * ntypes * 3 * sizeof(double));
         }
         up.finish();
+        tr->orig_of_slot = std::move(order);
         up.keep(tr->scratch);
         *out = owner.release();
     });

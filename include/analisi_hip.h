@@ -66,6 +66,13 @@ int anl_traj_create(const double *pos, const double *box, uint32_t box_stride,
                     const int32_t *type_id, uint32_t ntypes, const double *pos_cm,
                     uint64_t nframes, uint64_t natoms, anl_traj **out);
 int anl_traj_destroy(anl_traj *tr);
+/* Host work of the first screened g(r,t) handle up to rmax over tr (a constant
+ * cell only; else no effect), which anl_gofrt_create does otherwise, after
+ * reading the positions back: an order of the atoms of every frame.  pos: the
+ * positions tr was created from.  Waits for no other stream, so that a thread
+ * that creates the next trajectory can do it while a calculation runs.  The
+ * order changes no result. */
+int anl_traj_prepare_gofrt(anl_traj *tr, const double *pos, double rmax);
 
 /* ---- g(r,t) ------------------------------------------------------------ */
 /* Replaces Gofrt<double,T> (gofrt.h:37-45, gofrt.cpp:22-155) driven by

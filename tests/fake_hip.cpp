@@ -167,6 +167,7 @@ hipError_t hipHostMalloc(void **p, size_t n, unsigned) {
     return *p ? hipSuccess : hipErrorOutOfMemory;
 }
 hipError_t hipHostFree(void *p) {
+    if (p) log("hostfree %p", p);
     std::free(p);
     return hipSuccess;
 }
