@@ -542,55 +542,64 @@ void *msd_prepare_blocks(anl_traj *tr, const uint64_t *primo, const uint32_t *n,
     return P;
 }
 
-// out: [nblocks][leff][fcm][nt]
+// out: [nblocks][leff][fcm][nt].  A launch holds less than 2^32 threads: more
+// blocks than that go one range after the other.
 void msd_enqueue_prepared(void *prep, double *out, hipStream_t s) {
     const MsdPrepared &P = *(const MsdPrepared *)prep;
     if (P.leff == 0) return;
     const anl_traj *tr = P.tr;
-    if (P.tile) {
-        const uint32_t span = P.waves * P.tile;  // lags per workgroup
-        const uint32_t nres = std::min(P.skip, P.leff), M = (P.leff + P.skip - 1) / P.skip;
-        const uint32_t ntiles = (M + span - 1) / span;
-        const uint64_t total = (uint64_t)ntiles * nres * P.maxseg * P.nchunks * P.nblocks, per = (total + 7) / 8;
-        if (8 * per >= (1ull << 32)) fail(ANL_ERR_ARG, "MSD launch too large (reduce the number of blocks)");
-        const dim3 grid((uint32_t)(8 * per));
+    const uint32_t span = P.waves * P.tile;  // lags per workgroup of the window kernel
+    const uint32_t nres = std::min(P.skip, P.leff), M = (P.leff + P.skip - 1) / P.skip;
+    const uint32_t ntiles = P.tile ? (M + span - 1) / span : 0, nlb = (P.leff + MSD_TL - 1) / MSD_TL;
+    const uint32_t ncm = P.cm_msd ? P.nt * ((P.leff + 63) / 64) : 0;
+    // threads of a block
+    const uint64_t wgs = P.tile ? (uint64_t)ntiles * nres * P.maxseg * P.nchunks : 0;
+    const uint64_t threads = std::max(wgs * 64 * P.waves, ((uint64_t)P.leff * P.nt / 4 + 1 + ncm) * 256);
+    constexpr uint64_t LIMIT = (1ull << 32) - (1u << 14);  // grids are rounded up to 8 workgroups
+    if (threads > LIMIT) fail(ANL_ERR_ARG, "MSD launch too large (reduce the number of lags)");
+    const uint32_t range = (uint32_t)std::min<uint64_t>(P.tile ? P.nblocks : std::min(P.nblocks, 65535u), LIMIT / threads);
+    for (uint32_t b0 = 0; b0 < P.nblocks; b0 += range) {
+        const uint32_t nb = std::min(range, P.nblocks - b0);
+        MsdTables tables = P.tables;
+        if (tables.blocks) tables.blocks += b0;
+        if (tables.count) tables.count += (uint64_t)b0 * P.nt;
+        double *partial = P.d_partial + (uint64_t)b0 * P.leff * P.maxseg * P.nchunks * P.nt;
+        if (P.tile) {
+            const uint64_t total = wgs * nb, per = (total + 7) / 8;
+            const dim3 grid((uint32_t)(8 * per));
 #define ANL_MSD_WIN(R, W, C)                                                                             \
     hipLaunchKernelGGL((msd_window_kernel<R, W, C>), grid, dim3(64 * W), 0, s, tr->pos, tr->cm, tr->type_slot, \
-                       tr->N, P.nt, P.tables, P.maxseg, P.skip, P.leff, P.nchunks, P.group, ntiles, nres,         \
-                       (uint32_t)per, (uint32_t)total, P.d_partial)
+                       tr->N, P.nt, tables, P.maxseg, P.skip, P.leff, P.nchunks, P.group, ntiles, nres,           \
+                       (uint32_t)per, (uint32_t)total, partial)
 #define ANL_MSD_CASE(R, W)                          \
     case (R) * 64 + (W) * 2: ANL_MSD_WIN(R, W, false); break; \
     case (R) * 64 + (W) * 2 + 1: ANL_MSD_WIN(R, W, true); break;
-        switch (P.tile * 64 + P.waves * 2 + (P.cm_self ? 1 : 0)) {
-            ANL_MSD_CASE(8, 4)
-            ANL_MSD_CASE(12, 4)
-            ANL_MSD_CASE(16, 4)
-            ANL_MSD_CASE(24, 4)
-            ANL_MSD_CASE(16, 8)
-            ANL_MSD_CASE(24, 8)
-            ANL_MSD_CASE(12, 12)
-            ANL_MSD_CASE(16, 12)
-            ANL_MSD_CASE(8, 16)
-            default: fail(ANL_ERR_ARG, "unsupported MSD launch shape");
-        }
+            switch (P.tile * 64 + P.waves * 2 + (P.cm_self ? 1 : 0)) {
+                ANL_MSD_CASE(8, 4)
+                ANL_MSD_CASE(12, 4)
+                ANL_MSD_CASE(16, 4)
+                ANL_MSD_CASE(24, 4)
+                ANL_MSD_CASE(16, 8)
+                ANL_MSD_CASE(24, 8)
+                ANL_MSD_CASE(12, 12)
+                ANL_MSD_CASE(16, 12)
+                ANL_MSD_CASE(8, 16)
+                default: fail(ANL_ERR_ARG, "unsupported MSD launch shape");
+            }
 #undef ANL_MSD_CASE
 #undef ANL_MSD_WIN
-    } else {
-        const uint32_t nlb = (P.leff + MSD_TL - 1) / MSD_TL;
-        dim3 grid(P.nchunks, nlb, P.nblocks);
-        if (P.cm_self)
-            hipLaunchKernelGGL(msd_atoms_kernel<true>, grid, dim3(MSD_WG), 0, s, tr->pos, tr->cm, tr->type_slot, tr->N,
-                               P.nt, P.tables, P.skip, P.leff, P.nchunks, P.d_partial);
-        else
-            hipLaunchKernelGGL(msd_atoms_kernel<false>, grid, dim3(MSD_WG), 0, s, tr->pos, tr->cm, tr->type_slot,
-                               tr->N, P.nt, P.tables, P.skip, P.leff, P.nchunks, P.d_partial);
+        } else {
+            auto kernel = P.cm_self ? msd_atoms_kernel<true> : msd_atoms_kernel<false>;
+            hipLaunchKernelGGL(kernel, dim3(P.nchunks, nlb, nb), dim3(MSD_WG), 0, s, tr->pos, tr->cm, tr->type_slot,
+                               tr->N, P.nt, tables, P.skip, P.leff, P.nchunks, partial);
+        }
+        ANL_HIP(hipGetLastError());
+        const uint32_t nfin = (uint32_t)(((uint64_t)nb * P.leff * P.nt + 3) / 4);
+        hipLaunchKernelGGL(msd_finish_kernel, dim3(nfin + nb * ncm), dim3(256), 0, s, partial, P.nchunks, P.maxseg, P.nt,
+                           P.leff, nb, tables, P.fcm, tr->cm, P.skip, nfin,
+                           out + (uint64_t)b0 * P.leff * P.nt * P.fcm);
+        ANL_HIP(hipGetLastError());
     }
-    ANL_HIP(hipGetLastError());
-    const uint32_t nfin = (uint32_t)(((uint64_t)P.nblocks * P.leff * P.nt + 3) / 4);
-    const uint32_t ncm = P.cm_msd ? P.nblocks * P.nt * ((P.leff + 63) / 64) : 0;
-    hipLaunchKernelGGL(msd_finish_kernel, dim3(nfin + ncm), dim3(256), 0, s, P.d_partial, P.nchunks, P.maxseg, P.nt,
-                       P.leff, P.nblocks, P.tables, P.fcm, tr->cm, P.skip, nfin, out);
-    ANL_HIP(hipGetLastError());
 }
 
 void msd_free_prepared(void *prep) { delete (MsdPrepared *)prep; }

@@ -135,7 +135,8 @@ hipError_t hipLaunchKernel(const void *f, dim3 g, dim3 b, void **args, size_t, h
     }
     log("launch %p %u,%u,%u %u %s", (void *)s, g.x, g.y, g.z, b.x * b.y * b.z, bufs.c_str());
     if (launch_us) usleep(launch_us);
-    // the runtime's limits
+    // the dispatch packet holds 32 bits of threads a dimension: the real runtime
+    // runs the number modulo 2^32
     const bool bad = (uint64_t)g.x * b.x > UINT32_MAX || (uint64_t)g.y * b.y > UINT32_MAX ||
                      (uint64_t)g.z * b.z > UINT32_MAX || g.x == 0 || g.y == 0 || g.z == 0 || g.y > 65535 * 1024u;
     return last = bad ? hipErrorInvalidConfiguration : hipSuccess;
