@@ -15,7 +15,8 @@
 // msd_window_kernel: a wavefront holds R frames of its 64 atoms in registers,
 // one per lag of its tile, and moving to the next t0 replaces one of them.
 // The launch shape (R, wavefronts per workgroup) is tunable; tile 0 runs
-// msd_atoms_kernel (eight lags per thread, every frame loaded).
+// msd_atoms_kernel (eight lags per thread, every frame loaded), which a
+// calculation with few lags per residue also takes by itself.
 // A small calculation splits its t0 range into segments (msd_segments), summed
 // in order by msd_finish_kernel; the split depends on the calculation alone,
 // so every launch shape gives the same bits.
@@ -70,11 +71,14 @@ __device__ __forceinline__ void msd_segment(const MsdBlock &b, uint32_t skip, ui
     nk = min(len, K - k0);
 }
 
+// A thread holds eight lags of one atom and loads every frame.  The same
+// operations in the same order as msd_window_kernel over one segment, and the
+// same partial sums: per 64 slots, or per 256 (group 4).
 template <bool CMSELF>
 __global__ __launch_bounds__(MSD_WG) void msd_atoms_kernel(const double4 *__restrict__ pos, const double *__restrict__ cm,
                                                           const int32_t *__restrict__ type_slot, uint64_t N, uint32_t nt,
-                                                          const MsdTables tb_, uint32_t skip,
-                                                          uint32_t leff, uint32_t nchunks, double *__restrict__ partial) {
+                                                          const MsdTables tb_, uint32_t skip, uint32_t leff,
+                                                          uint32_t nchunks, uint32_t group, double *__restrict__ partial) {
     __shared__ double acc_lds[MSD_TL][MSD_WG];
     __shared__ int type_lds[MSD_WG];
     const MsdBlock blk = tb_.block(blockIdx.z);
@@ -88,30 +92,23 @@ __global__ __launch_bounds__(MSD_WG) void msd_atoms_kernel(const double4 *__rest
     int ti = -1;
     if (slot < N) {
         ti = type_slot[slot];
+        auto frame = [&](uint64_t f) {
+            const double4 x = pos[f * N + slot];
+            if (!CMSELF) return make_double3(x.x, x.y, x.z);
+            const double *c = cm + (f * nt + ti) * 3;
+            return make_double3(x.x - c[0], x.y - c[1], x.z - c[2]);
+        };
         for (uint32_t t0 = 0; t0 < n; t0 += skip) {
-            const uint64_t fa = primo + t0;
-            const double4 xa = pos[fa * N + slot];
-            double ca0 = 0, ca1 = 0, ca2 = 0;
-            if (CMSELF) {
-                const double *c = cm + (fa * nt + ti) * 3;
-                ca0 = c[0];
-                ca1 = c[1];
-                ca2 = c[2];
-            }
+            const double3 y = frame(primo + t0);
 #pragma unroll
             for (int l = 0; l < MSD_TL; l++) {
                 const uint32_t t = tb + l;
                 if (t < leff) {
-                    const uint64_t fb = fa + t;
-                    const double4 xb = pos[fb * N + slot];
-                    double e0 = xa.x - xb.x, e1 = xa.y - xb.y, e2 = xa.z - xb.z;
-                    if (CMSELF) {
-                        const double *c = cm + (fb * nt + ti) * 3;
-                        e0 = e0 - (ca0 - c[0]);
-                        e1 = e1 - (ca1 - c[1]);
-                        e2 = e2 - (ca2 - c[2]);
-                    }
-                    acc[l] += (e0 * e0 + e1 * e1) + e2 * e2;
+                    const double3 z = frame(primo + t0 + t);
+                    const double e0 = y.x - z.x, e1 = y.y - z.y, e2 = y.z - z.z;
+                    acc[l] = fma(e0, e0, acc[l]);
+                    acc[l] = fma(e1, e1, acc[l]);
+                    acc[l] = fma(e2, e2, acc[l]);
                 }
             }
         }
@@ -120,15 +117,20 @@ __global__ __launch_bounds__(MSD_WG) void msd_atoms_kernel(const double4 *__rest
     for (int l = 0; l < MSD_TL; l++) acc_lds[l][threadIdx.x] = acc[l];
     type_lds[threadIdx.x] = ti;
     __syncthreads();
-    // thread (l, type) sums its lane set in slot order
-    for (uint32_t w = threadIdx.x; w < MSD_TL * nt; w += MSD_WG) {
-        const uint32_t l = w / nt, tt = w % nt;
-        const uint32_t t = tb + l;
-        if (t >= leff) continue;
+    // thread (chunk, lag, type) sums 64 slots in order, or (lag, type) four such sums
+    const uint32_t parts = 4 / group;
+    for (uint32_t w = threadIdx.x; w < parts * MSD_TL * nt; w += MSD_WG) {
+        const uint32_t p = w / (MSD_TL * nt), r = w % (MSD_TL * nt), l = r / nt, tt = r % nt;
+        const uint32_t t = tb + l, chunk = blockIdx.x * parts + p;
+        if (t >= leff || chunk >= nchunks) continue;
         double s = 0.0;
-        for (int k = 0; k < MSD_WG; k++)
-            if (type_lds[k] == (int)tt) s += acc_lds[l][k];
-        partial[(((uint64_t)blockIdx.z * leff + t) * nchunks + blockIdx.x) * nt + tt] = s;  // one segment
+        for (uint32_t g = 0; g < group; g++) {
+            double sum = 0.0;
+            for (uint32_t k = 64 * (p + g); k < 64 * (p + g) + 64; k++)
+                if (type_lds[k] == (int)tt) sum += acc_lds[l][k];
+            s = g == 0 ? sum : s + sum;
+        }
+        partial[(((uint64_t)blockIdx.z * leff + t) * nchunks + chunk) * nt + tt] = s;  // one segment
     }
 }
 
@@ -448,6 +450,30 @@ static uint32_t msd_auto_tile(uint64_t units, uint32_t M, bool cm_self) {
     return best;
 }
 
+// Whether the shape chosen with anl_msd_set_tuning runs this calculation: at t0
+// strides above 1 only where the lags of a residue fill its workgroups.  Else
+// wavefronts, or most of their windows, would work for no lag: 8,000 atoms,
+// stride 300, one lag per residue, shape (24, 8) 1,120 us, the calculation's
+// own 49.
+static bool msd_chosen_shape(const anl_traj *tr, uint32_t skip, uint32_t leff) {
+    if (tr->msd_auto) return false;
+    return skip == 1 || tr->msd_tile == 0 || (leff + skip - 1) / skip >= tr->msd_tile * tr->msd_waves;
+}
+
+// Whether msd_atoms_kernel is the faster one: few lags per residue (M) and few
+// t0 (K), in a launch that fills the chip.  A wavefront of the window kernel
+// then fills a window of 8 frames and uses M of them, msd_atoms_kernel forms 8
+// lags of any residues in a thread.  20,000 atoms, stride 100 (us, window and
+// atoms, without drift removal): M 1, K 2 143 and 55, K 20 389 and 249; M 2, K 8
+// 217 and 198, K 20 401 and 453; M 3, K 4 182 and 152, K 6 203 and 209; with
+// it M 2, K 20 635 and 451, M 3, K 20 639 and 672, M 4, K 6 322 and 272, K 12
+// 466 and 540.  The line is where 10.7 M K + 33 meets 13.7 (K + 8), with drift
+// removal 25 (K + 5).  Launches of 3,000 to 4,700 workgroups break even.
+static bool msd_few_lags(uint64_t N, uint32_t nblocks, uint32_t n, uint32_t skip, uint32_t leff, bool cm_self) {
+    const double M = (leff + skip - 1) / skip, K = (n + skip - 1) / skip;
+    return skip > 1 && (N + 63) / 64 * std::min(skip, leff) * nblocks >= 8192 && (M - (cm_self ? 2.34 : 1.28)) * K < 8;
+}
+
 // msd.cpp:52-61 checks (leff is common to all blocks: min(n_b, tmax) must
 // agree); fills P's sizes and the host tables of the block list and the
 // term counts.  Touches no device memory.
@@ -478,30 +504,34 @@ static void msd_plan(anl_traj *tr, const uint64_t *primo, const uint32_t *n, uin
     P->fcm = cm_msd ? 2 : 1;
     P->cm_msd = cm_msd;
     P->cm_self = cm_self;
+    const bool own = !msd_chosen_shape(tr, skip, leff);
     P->tile = tr->msd_tile;
     P->waves = tr->msd_waves;
-    // a partial sum per 64 atoms; per 256 in msd_atoms_kernel and, at strides
-    // that msd_atoms_kernel once ran alone, where 64 would take more than 8 MiB
-    // (what fits a caller's scratch stays what it was)
+    // a partial sum per 64 atoms; per 256 at the strides and in the kernel that
+    // once had them all, where 64 would take more than 8 MiB (what fits a
+    // caller's scratch stays what it was)
     const uint64_t c64 = (tr->N + 63) / 64;
-    P->group = P->tile && skip > 1 && (uint64_t)leff * c64 * tr->nt * sizeof(double) > (8ull << 20) ? 4 : 1;
-    P->nchunks = (uint32_t)(P->tile ? (c64 + P->group - 1) / P->group : (tr->N + MSD_WG - 1) / MSD_WG);
+    P->group = (P->tile == 0 || skip > 1) && (uint64_t)leff * c64 * tr->nt * sizeof(double) > (8ull << 20) ? 4 : 1;
+    P->nchunks = (uint32_t)((c64 + P->group - 1) / P->group);
     P->maxseg = 1;
     hb->assign(nblocks, MsdBlock{});
     hc->assign((size_t)nblocks * tr->nt, 0);
     uint64_t segs = 0;
+    uint32_t nmax = 0;
     for (uint32_t b = 0; b < nblocks; b++) {
         const uint32_t nseg = P->tile && leff ? msd_segments(tr->N, tr->nt, n[b], skip, leff) : 1;
         P->maxseg = std::max(P->maxseg, nseg);
         segs += nseg;
+        nmax = std::max(nmax, n[b]);
         (*hb)[b] = MsdBlock{primo[b], n[b], nseg};
         const uint64_t n0 = (n[b] + skip - 1) / skip;
         for (uint32_t k = 0; k < tr->nt; k++) (*hc)[(size_t)b * tr->nt + k] = n0 * tr->type_count[k];
     }
-    if (P->tile && tr->msd_auto && leff) {
+    if (P->tile && own && leff) {
         const uint32_t M = (leff + skip - 1) / skip;
         P->tile = msd_auto_tile((uint64_t)P->nchunks * std::min(skip, leff) * segs, M, cm_self);
         P->waves = 4;
+        if (P->maxseg == 1 && msd_few_lags(tr->N, nblocks, nmax, skip, leff, cm_self)) P->tile = 0;
     }
     if (nblocks == 1 && tr->nt <= MSD_INL) {
         P->tables.one = (*hb)[0];
@@ -590,8 +620,9 @@ void msd_enqueue_prepared(void *prep, double *out, hipStream_t s) {
 #undef ANL_MSD_WIN
         } else {
             auto kernel = P.cm_self ? msd_atoms_kernel<true> : msd_atoms_kernel<false>;
-            hipLaunchKernelGGL(kernel, dim3(P.nchunks, nlb, nb), dim3(MSD_WG), 0, s, tr->pos, tr->cm, tr->type_slot,
-                               tr->N, P.nt, tables, P.skip, P.leff, P.nchunks, partial);
+            hipLaunchKernelGGL(kernel, dim3((uint32_t)((tr->N + MSD_WG - 1) / MSD_WG), nlb, nb), dim3(MSD_WG), 0, s,
+                               tr->pos, tr->cm, tr->type_slot, tr->N, P.nt, tables, P.skip, P.leff, P.nchunks, P.group,
+                               partial);
         }
         ANL_HIP(hipGetLastError());
         const uint32_t nfin = (uint32_t)(((uint64_t)nb * P.leff * P.nt + 3) / 4);

@@ -259,13 +259,16 @@ int anl_msd_calculate_noalloc(anl_traj *tr, uint32_t skip, uint32_t tmax, int cm
  * updates, and its wavefronts per workgroup W (a workgroup covers R * W lags
  * of 64 atoms; at t0 stride s > 1, R * W of the lags that are equal modulo
  * s).  (R, W) is one of (8,4) (12,4) (16,4) (24,4) (16,8) (24,8) (12,12)
- * (16,12) (8,16).  Until one is set each calculation takes its own tile by
- * its sizes, and the shape reads as (16,4).  Lag tile 0 selects the
- * eight-lags-per-thread kernel (W ignored).
+ * (16,12) (8,16).  Until one is set each calculation takes its own shape by
+ * its sizes, and the shape reads as (16,4); at strides above 1 it also does
+ * where fewer than R * W lags are equal modulo the stride.  Lag tile 0 selects
+ * the eight-lags-per-thread kernel (W ignored), which at strides above 1 with
+ * few t0 and lags may also be a calculation's own.
  * All shapes with R > 0 give identical results (each (atom, lag) sum runs
  * over t0 in order with the same operations, and the workgroup sums its 64
- * atoms in slot order); tile 0 agrees with them to rounding (both within
- * 1e-10 of the reference).  anl_msd_autotune times each candidate shape
+ * atoms in slot order); so does tile 0, except for a small calculation whose
+ * t0 range the others split, to rounding there (both within 1e-10 of the
+ * reference).  anl_msd_autotune times each candidate shape
  * (cand[2c], cand[2c+1]; NULL = the nine shapes above and tile 0) on the
  * calculation reset(n) at primo and keeps the fastest; ms_out[c] (may be
  * NULL) receives the times.  The reference's equivalent knob is nthreads
