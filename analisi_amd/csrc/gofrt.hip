@@ -2140,7 +2140,7 @@ void check_lengths(anl_gofrt *g, const uint64_t *primo, const uint32_t *n, uint3
 // can be captured into a HIP graph and replayed.
 struct GofrtPrepared {
     GofrtArgs a{};
-    dim3 grid;
+    bool remap = false;  // workgroups numbered per XCD (decode_wg)
     size_t lds = 0;
     int form = ANL_GOFRT_FP64;
     uint64_t out_len = 0;
@@ -2157,9 +2157,9 @@ struct GofrtPrepared {
 // Clears the output and the launch counters (a kernel: the launch may be
 // captured into a graph).
 __global__ void clear_kernel(unsigned long long *__restrict__ p, uint64_t len, unsigned long long *__restrict__ stat) {
-    const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < len) p[i] = 0ull;
-    if (i < NSTAT) stat[i] = 0ull;
+    const uint64_t i0 = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    for (uint64_t i = i0; i < len; i += (uint64_t)gridDim.x * blockDim.x) p[i] = 0ull;
+    if (i0 < NSTAT) stat[i0] = 0ull;
 }
 
 // own = true: the work list and block table go to buffers owned by the
@@ -2287,8 +2287,7 @@ GofrtPrepared gofrt_prepare(anl_gofrt *g, const Launch &L, uint64_t out_len, int
     const uint32_t nlag = nlag_force ? nlag_force : (L.leff_max + g->every - 1) / g->every;
     a.lag0 = lag0;
     const uint64_t total = (uint64_t)ntiles * nlag * L.nwork;
-    const uint64_t per = (total + 7) / 8;
-    if (8 * per >= (1ull << 32)) fail(ANL_ERR_ARG, "too many workgroups (reduce the trajectory block)");
+    if ((total + 7) / 8 * 8 >= (1ull << 32)) fail(ANL_ERR_ARG, "too many workgroups (reduce the trajectory block)");
     // histogram-offset table (screened forms: two entries per type pair; the
     // plain form, whose room stays as it was, reads a.chan when it flushes),
     // bin-edge table, histogram
@@ -2304,9 +2303,7 @@ GofrtPrepared gofrt_prepare(anl_gofrt *g, const Launch &L, uint64_t out_len, int
     a.ntiles = ntiles;
     a.nlag = nlag;
     a.nwork = L.nwork;
-    const bool remap = g->tune.xcd && (form == ANL_GOFRT_SCREENED || cells);
-    a.per_xcd = remap ? (uint32_t)per : 0u;
-    P.grid = dim3((uint32_t)(remap ? 8 * per : total));
+    P.remap = g->tune.xcd && (form == ANL_GOFRT_SCREENED || cells);
     // the cluster screen needs the larger queue; without room it is not used
     const bool colc = g->tune.cluster == 2 || g->tune.cluster == 4;
     const int qcl = colc ? SQCAP_CLC : SQCAP_CL;
@@ -2332,24 +2329,22 @@ GofrtPrepared gofrt_prepare(anl_gofrt *g, const Launch &L, uint64_t out_len, int
     return P;
 }
 
-void gofrt_enqueue(anl_gofrt *g, const GofrtPrepared &P, unsigned long long *out, hipStream_t s) {
-    GofrtArgs a = P.a;
-    a.out = out;
-    hipLaunchKernelGGL(clear_kernel, dim3((unsigned)((std::max<uint64_t>(P.out_len, NSTAT) + 255) / 256)), dim3(256), 0, s,
-                       out, P.out_len, g->d_ncand);
-    ANL_HIP(hipGetLastError());
-    if (P.grid.x == 0) return;
+// The lags and work items of `a` in one launch.
+static void gofrt_launch(anl_gofrt *g, const GofrtPrepared &P, GofrtArgs a, hipStream_t s) {
+    const uint64_t total = (uint64_t)a.ntiles * a.nlag * a.nwork, per = (total + 7) / 8;
+    a.per_xcd = P.remap ? (uint32_t)per : 0u;
+    const dim3 grid((uint32_t)(P.remap ? 8 * per : total));
     if (P.cells) {
         const GofrtCellArgs c{a, g->d_cells};
-        if (P.triclinic) hipLaunchKernelGGL(gofrt_cells_kernel<true>, P.grid, dim3(WG), P.lds, s, c);
-        else hipLaunchKernelGGL(gofrt_cells_kernel<false>, P.grid, dim3(WG), P.lds, s, c);
+        if (P.triclinic) hipLaunchKernelGGL(gofrt_cells_kernel<true>, grid, dim3(WG), P.lds, s, c);
+        else hipLaunchKernelGGL(gofrt_cells_kernel<false>, grid, dim3(WG), P.lds, s, c);
     } else if (P.form == ANL_GOFRT_FP64) {
         auto kernel = P.triclinic ? (P.split ? gofrt_fp64_kernel<true, true> : gofrt_fp64_kernel<true, false>)
                                   : (P.split ? gofrt_fp64_kernel<false, true> : gofrt_fp64_kernel<false, false>);
-        hipLaunchKernelGGL(kernel, P.grid, dim3(P.split ? SPLIT_WG : WG), P.lds, s, a);
+        hipLaunchKernelGGL(kernel, grid, dim3(P.split ? SPLIT_WG : WG), P.lds, s, a);
     } else {
         const bool u8 = P.unroll == 8;
-#define ANL_SCREENED(T, U, C, K) hipLaunchKernelGGL((gofrt_screened_kernel<T, U, C, K>), P.grid, dim3(WG), P.lds, s, a)
+#define ANL_SCREENED(T, U, C, K) hipLaunchKernelGGL((gofrt_screened_kernel<T, U, C, K>), grid, dim3(WG), P.lds, s, a)
         if (P.cluster) {  // the 16-bit fallback of non-compact wavefronts takes 8 j per step
             switch (P.cluster * 2 + (P.triclinic ? 1 : 0)) {
                 case 2: ANL_SCREENED(false, 8, true, 1); break;
@@ -2373,6 +2368,30 @@ void gofrt_enqueue(anl_gofrt *g, const GofrtPrepared &P, unsigned long long *out
 #undef ANL_SCREENED
     }
     ANL_HIP(hipGetLastError());
+}
+
+// A launch holds less than 2^32 threads (it runs their number modulo 2^32
+// otherwise, without an error): longer calculations are launched in ranges of
+// lags, or of work items.
+void gofrt_enqueue(anl_gofrt *g, const GofrtPrepared &P, unsigned long long *out, hipStream_t s) {
+    GofrtArgs a = P.a;
+    a.out = out;
+    const uint64_t clear = std::min<uint64_t>((std::max<uint64_t>(P.out_len, NSTAT) + 255) / 256, 1u << 20);
+    hipLaunchKernelGGL(clear_kernel, dim3((unsigned)clear), dim3(256), 0, s, out, P.out_len, g->d_ncand);
+    ANL_HIP(hipGetLastError());
+    if ((uint64_t)a.ntiles * a.nlag * a.nwork == 0) return;
+    const uint64_t most = ((1ull << 32) - 1) / (P.split ? SPLIT_WG : WG) - 8;  // workgroups
+    const uint32_t works = (uint32_t)std::min<uint64_t>(a.nwork, std::max<uint64_t>(1, most / a.ntiles));
+    const uint32_t lags = (uint32_t)std::min<uint64_t>(a.nlag, std::max<uint64_t>(1, most / ((uint64_t)a.ntiles * works)));
+    for (uint32_t w = 0; w < P.a.nwork; w += works)
+        for (uint32_t l = 0; l < P.a.nlag; l += lags) {
+            a.nwork = std::min(works, P.a.nwork - w);
+            a.work = P.a.work ? P.a.work + w : nullptr;
+            a.wk0 = P.a.wk0 + w * P.a.chunk;
+            a.nlag = std::min(lags, P.a.nlag - l);
+            a.lag0 = P.a.lag0 + l * P.a.every;
+            gofrt_launch(g, P, a, s);
+        }
 }
 
 // Internal API of the block engine (blocks.hip), declared in anl_internal.h.
