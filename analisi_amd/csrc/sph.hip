@@ -711,6 +711,7 @@ struct SteinArgs {
     unsigned long long *hist;    // [nbin][nt][nt][hs] counts, or null
     double *q;                   // [nbin][nfs][N][nt][lmax] q_l, l = 1..lmax, or null
     uint64_t N, FS, hs;
+    uint64_t item0;              // first item of this launch
     uint32_t nt, nbin, lmax, nl, nbin_st, nfr, fidx0, nfs;
     uint32_t lmask;              // bit l set: q_l is needed
     double c00;                  // Y_00 of any direction: the density's l = 0 entry is (count) * c00
@@ -765,7 +766,7 @@ __global__ __launch_bounds__(256) void sph_steinhardt_kernel(SteinArgs a) {
     const uint64_t total = (uint64_t)a.nfr * a.nt * a.nbin * a.N;
     __shared__ double w[AVG ? 4 : 1][AVG ? NQ * NQ : 1];
     __shared__ double qs[AVG ? STEIN_ITEMS : 1][NQ];
-    uint64_t k = (uint64_t)blockIdx.x * 256 + threadIdx.x;
+    uint64_t k = a.item0 + (uint64_t)blockIdx.x * 256 + threadIdx.x;
     if constexpr (AVG) {
         const uint32_t lane = threadIdx.x & 63u, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
         // entry lane + 64 c: (l, position o in the order of the m sum); this lane's l among the sums
@@ -787,7 +788,7 @@ __global__ __launch_bounds__(256) void sph_steinhardt_kernel(SteinArgs a) {
             first += 2 * l + 1;
             nsel++;
         }
-        const uint64_t item0 = (uint64_t)blockIdx.x * STEIN_ITEMS;
+        const uint64_t item0 = a.item0 + (uint64_t)blockIdx.x * STEIN_ITEMS;
         for (uint32_t it = wave * (STEIN_ITEMS / 4); it < (wave + 1) * (STEIN_ITEMS / 4); ++it) {
             if (lane < NQ) qs[it][lane] = 0.0;
             if (item0 + it >= total) continue;  // uniform
@@ -902,8 +903,11 @@ __global__ __launch_bounds__(256) void sph_finish_kernel(const double *__restric
 }
 
 __global__ __launch_bounds__(256) void sph_zero_kernel(double *p, uint64_t n) {
-    const uint64_t k = (uint64_t)blockIdx.x * 256 + threadIdx.x;
-    if (k < n) p[k] = 0.0;
+    for (uint64_t k = (uint64_t)blockIdx.x * 256 + threadIdx.x; k < n; k += (uint64_t)gridDim.x * 256) p[k] = 0.0;
+}
+static void sph_zero(double *p, uint64_t n, hipStream_t s) {
+    hipLaunchKernelGGL(sph_zero_kernel, dim3((uint32_t)std::min<uint64_t>((n + 255) / 256, 1u << 20)), dim3(256), 0, s, p, n);
+    ANL_HIP(hipGetLastError());
 }
 
 // specialfunctions.h:33-49: sqrt((2l+1)/(4 pi)) for m = 0, else
@@ -988,19 +992,15 @@ uint64_t radius_bytes(const anl_sph *h, uint64_t nfr) {
     return h->block_screen ? nfr * ((h->tr->N + 63) / 64) * sizeof(double4) : 0;
 }
 
-// densities of frames f0 + k * fstride, k < nfr, of the device trajectory into
-// S, expanded up to l = lm (default lmax; the values of l <= lm do not depend
-// on it); rad holds radius_bytes(h, nfr)
-void launch_density(anl_sph *h, uint64_t f0, uint64_t fstride, uint32_t nfr, double *S, double4 *rad,
-                    hipStream_t s, int32_t *nbr = nullptr, uint32_t lm = ~0u) {
-    if (lm > h->lmax) lm = h->lmax;
+// one launch of launch_density, which checks the sizes and reads the overflow of the lists
+void launch_density_range(anl_sph *h, uint64_t f0, uint64_t fstride, uint32_t nfr, double *S, double4 *rad,
+                          hipStream_t s, int32_t *nbr, uint32_t lm) {
     SphDensArgs a{};
     a.fstride = fstride;
     a.block_rad = h->block_screen ? rad : nullptr;
     auto block_spheres = [&] {
         if (!a.block_rad) return;
         const uint64_t nb = (uint64_t)nfr * ((h->tr->N + 63) / 64);
-        if (nb > 0x7fffffffull) fail(ANL_ERR_ARG, "too many (frame, atom block) pairs in one launch");
         hipLaunchKernelGGL(sph_block_radius_kernel, dim3((uint32_t)nb), dim3(64), 0, s, h->tr->pos, h->tr->box,
                            h->tr->N, f0, fstride, rad);
         ANL_HIP(hipGetLastError());
@@ -1020,7 +1020,6 @@ void launch_density(anl_sph *h, uint64_t f0, uint64_t fstride, uint32_t nfr, dou
         a.lmax = lm;
         a.nbc = 1;
         const uint64_t gx = (uint64_t)nfr * a.N;
-        if (gx > 0x7fffffffull) fail(ANL_ERR_ARG, "too many (frame, atom) pairs in one density launch");
         SannArgs sa = h->sann_args;
         sa.nbr = nbr;  // the chosen neighbours, for the averaged order parameter
         double cut2 = 0.0;
@@ -1030,17 +1029,12 @@ void launch_density(anl_sph *h, uint64_t f0, uint64_t fstride, uint32_t nfr, dou
         const size_t lds = (size_t)(h->nt * (lm + 1) * (lm + 1) + stage_doubles(lm) + sa.total +
                                     sa.capmax) * sizeof(double) +
                            (size_t)(sa.total + sa.capmax) * sizeof(int);
-        ANL_HIP(hipMemsetAsync(h->d_overflow, 0, sizeof(int), s));
         auto kernel = lm <= SPH_LM_LOW ? (h->tr->triclinic ? sph_density_sann_kernel<true, SPH_LM_LOW>
                                                            : sph_density_sann_kernel<false, SPH_LM_LOW>)
                                        : (h->tr->triclinic ? sph_density_sann_kernel<true, ANL_SPH_LMAX_MAX>
                                                            : sph_density_sann_kernel<false, ANL_SPH_LMAX_MAX>);
         hipLaunchKernelGGL(kernel, dim3((uint32_t)gx), dim3(64), lds, s, a, sa);
         ANL_HIP(hipGetLastError());
-        int over = 0;
-        ANL_HIP(hipMemcpyAsync(&over, h->d_overflow, sizeof(int), hipMemcpyDeviceToHost, s));
-        ANL_HIP(hipStreamSynchronize(s));
-        if (over) fail(ANL_ERR_ARG, "Too many neighbours in shell!");  // neighbour.cpp:44-48
         return;
     }
     a.d2lo = h->d2lo;
@@ -1065,7 +1059,6 @@ void launch_density(anl_sph *h, uint64_t f0, uint64_t fstride, uint32_t nfr, dou
     const uint32_t accn = a.nt * a.nbc * (a.lmax + 1) * (a.lmax + 1);
     const size_t lds = (size_t)SPH_WAVES * (accn + stage_doubles(a.lmax)) * sizeof(double);
     const uint64_t gx = (uint64_t)nfr * a.ngroups;
-    if (gx > 0x7fffffffull) fail(ANL_ERR_ARG, "too many (frame, atom) pairs in one density launch");
     if ((h->nbin + a.nbc - 1) / a.nbc > 65535) fail(ANL_ERR_ARG, "too many distance bins");
     dim3 grid((uint32_t)gx, (h->nbin + a.nbc - 1) / a.nbc);
     auto kernel = lm <= SPH_LM_LOW ? (h->tr->triclinic ? sph_density_kernel<true, SPH_LM_LOW> : sph_density_kernel<false, SPH_LM_LOW>)
@@ -1075,6 +1068,29 @@ void launch_density(anl_sph *h, uint64_t f0, uint64_t fstride, uint32_t nfr, dou
     ANL_HIP(hipGetLastError());
 }
 
+// densities of frames f0 + k * fstride, k < nfr, of the device trajectory into
+// S, expanded up to l = lm (default lmax; the values of l <= lm do not depend
+// on it); rad holds radius_bytes(h, nfr)
+void launch_density(anl_sph *h, uint64_t f0, uint64_t fstride, uint32_t nfr, double *S, double4 *rad,
+                    hipStream_t s, int32_t *nbr = nullptr, uint32_t lm = ~0u) {
+    if (lm > h->lmax) lm = h->lmax;
+    const uint64_t N = h->tr->N;
+    if (nfr * (h->sann ? N : (N + SPH_WAVES - 1) / SPH_WAVES) > 0x7fffffffull)
+        fail(ANL_ERR_ARG, "too many (frame, atom) pairs in one density launch");
+    if (h->sann) ANL_HIP(hipMemsetAsync(h->d_overflow, 0, sizeof(int), s));
+    // a launch holds less than 2^32 threads, 64 an atom
+    const uint64_t most = std::max<uint64_t>(1, ((1ull << 32) - 1) / (64 * (N + SPH_WAVES)));
+    for (uint64_t k = 0; k < nfr; k += most)
+        launch_density_range(h, f0 + k * fstride, fstride, (uint32_t)std::min<uint64_t>(most, nfr - k),
+                             S + k * frame_doubles(h, lm), rad + radius_bytes(h, k) / sizeof(double4), s,
+                             nbr ? nbr + k * N * h->sann_args.total : nullptr, lm);
+    if (h->sann) {
+        int over = 0;
+        ANL_HIP(hipMemcpyAsync(&over, h->d_overflow, sizeof(int), hipMemcpyDeviceToHost, s));
+        ANL_HIP(hipStreamSynchronize(s));
+        if (over) fail(ANL_ERR_ARG, "Too many neighbours in shell!");  // neighbour.cpp:44-48
+    }
+}
 void sph_calculate(anl_sph *h, uint64_t primo, uint32_t n, uint32_t tmax, uint32_t skip, double *out_host) {
     anl_traj *tr = h->tr;
     if (skip == 0) skip = 1;
@@ -1106,8 +1122,7 @@ void sph_calculate(anl_sph *h, uint64_t primo, uint32_t n, uint32_t tmax, uint32
     double4 *rad = (double4 *)(w + offQ);
     hipStream_t s = nullptr;
     const uint64_t nR = (uint64_t)nprob * leff;
-    hipLaunchKernelGGL(sph_zero_kernel, dim3((uint32_t)((nR + 255) / 256)), dim3(256), 0, s, R, nR);
-    ANL_HIP(hipGetLastError());
+    sph_zero(R, nR, s);
     for (uint64_t e0 = 0; e0 < n0; e0 += rc) {
         const uint32_t n0c = (uint32_t)std::min<uint64_t>(rc, n0 - e0);
         const uint64_t t1_first = e0 * skip;
@@ -1189,8 +1204,7 @@ void steinhardt_calculate(anl_sph *h, uint64_t primo, uint32_t n, uint32_t skip,
     double *outd = (double *)(w + offO);
     int32_t *nbr = averaged ? (int32_t *)(w + offN) : nullptr;
     hipStream_t s = nullptr;
-    hipLaunchKernelGGL(sph_zero_kernel, dim3((uint32_t)((len + 255) / 256)), dim3(256), 0, s, outd, len);
-    ANL_HIP(hipGetLastError());
+    sph_zero(outd, len, s);
     SteinArgs a{};
     a.S = S;
     a.type_ap = h->d_type_ap;
@@ -1221,12 +1235,17 @@ void steinhardt_calculate(anl_sph *h, uint64_t primo, uint32_t n, uint32_t skip,
         a.fidx0 = (uint32_t)f0;
         const uint64_t nth = (uint64_t)nfc * nt * nbin * N;
         if ((nth + 255) / 256 > 0x7fffffffull) fail(ANL_ERR_ARG, "too many (frame, atom) pairs in one launch");
-        if (nbr)  // the densities of 2^31 workgroups' items would not fit the memory
-            hipLaunchKernelGGL(sph_steinhardt_kernel<true>, dim3((uint32_t)((nth + STEIN_ITEMS - 1) / STEIN_ITEMS)),
-                               dim3(256), 0, s, a);
-        else
-            hipLaunchKernelGGL(sph_steinhardt_kernel<false>, dim3((uint32_t)((nth + 255) / 256)), dim3(256), 0, s, a);
-        ANL_HIP(hipGetLastError());
+        // a launch holds less than 2^32 threads, four an item in the averaged form
+        constexpr uint64_t MOST = 1ull << 29;
+        for (a.item0 = 0; a.item0 < nth; a.item0 += MOST) {
+            const uint64_t items = std::min(MOST, nth - a.item0);
+            if (nbr)
+                hipLaunchKernelGGL(sph_steinhardt_kernel<true>, dim3((uint32_t)((items + STEIN_ITEMS - 1) / STEIN_ITEMS)),
+                                   dim3(256), 0, s, a);
+            else
+                hipLaunchKernelGGL(sph_steinhardt_kernel<false>, dim3((uint32_t)((items + 255) / 256)), dim3(256), 0, s, a);
+            ANL_HIP(hipGetLastError());
+        }
     }
     if (do_hist) {
         std::vector<unsigned long long> c(len);
