@@ -712,6 +712,7 @@ struct SteinArgs {
     double *q;                   // [nbin][nfs][N][nt][lmax] q_l, l = 1..lmax, or null
     uint64_t N, FS, hs;
     uint64_t item0;              // first item of this launch
+    uint32_t items;              // of a workgroup, averaged form
     uint32_t nt, nbin, lmax, nl, nbin_st, nfr, fidx0, nfs;
     uint32_t lmask;              // bit l set: q_l is needed
     double c00;                  // Y_00 of any direction: the density's l = 0 entry is (count) * c00
@@ -727,7 +728,6 @@ struct SteinItem {
     uint64_t ap;
     uint32_t b, jt, fl, ti;
     const double *Sb;  // the densities of (frame, type_j, bin)
-    double na;         // the neighbour count, recovered exactly from the l = 0 entry
 };
 __device__ __forceinline__ SteinItem stein_item(const SteinArgs &a, uint64_t k) {
     SteinItem t;
@@ -738,28 +738,35 @@ __device__ __forceinline__ SteinItem stein_item(const SteinArgs &a, uint64_t k) 
     t.jt = (uint32_t)(k % a.nt);
     t.fl = (uint32_t)(k / a.nt);
     t.Sb = a.S + (uint64_t)t.fl * a.FS + (uint64_t)(t.jt * a.nbin + t.b) * (a.lmax + 1) * (a.lmax + 1) * a.N;
-    t.na = rint(t.Sb[t.ap] / a.c00);
     t.ti = (uint32_t)a.type_ap[t.ap];
     return t;
 }
+// the neighbour count, recovered exactly from the l = 0 entry
+__device__ __forceinline__ double stein_count(const SteinArgs &a, const SteinItem &t) { return rint(t.Sb[t.ap] / a.c00); }
 __device__ __forceinline__ double stein_q(double v, double na, int l) {
     const double pi = 3.14159265358979323846264338327950288419716939937510;
     return sqrt(v / na / na * 4 * pi / (2 * l + 1));
 }
 
-constexpr int STEIN_ITEMS = 64;  // items of a workgroup of the averaged form
+// Items of a workgroup of the averaged form, at most: fewer where that leaves
+// the launch below STEIN_WGS workgroups (8 per CU), since a wavefront takes its
+// items one after the other (200 atoms, 20 frames, l = 0, us a call: 107 with 64
+// items, 71 with 4; 100 atoms, l = 4 and 6, 121 and 65).
+constexpr int STEIN_ITEMS = 64;
+constexpr uint64_t STEIN_WGS = 2048;
 
 // steinhardt.cpp:166-225.  q_l = sqrt(sum_m S_lm^2 / n / n * 4 pi / (2l+1)), the
 // m sum in the reference's order (m = 0, -1..-l, 1..l), n the neighbour count.
 // Plain: one thread per item.  AVG, the averaged order parameter
 // (steinhardt.cpp:128-173): qbar = S(i)/n(i) for the atom's own type, plus
-// S(k)/n(k) of its SANN neighbours k in order.  A wavefront takes 16 items one
-// after the other: a lane owns one or two (l, m) and adds the neighbours in
-// order, so that a neighbour's m run is one coalesced read and its count one
-// division for all; the squares meet in LDS, one lane per l sums them; then the
-// first wavefront finishes the 64 items.  With one thread per item (too few
-// wavefronts, a scattered read and a division per value) 2,000 atoms x 30
-// frames, l = 4 and 6, took 322 us; this takes 190.
+// S(k)/n(k) of its SANN neighbours k in order.  A wavefront takes its items with
+// neighbours (their counts are read together) one after the other: a lane owns
+// one or two (l, m) and adds the neighbours in order, so that a neighbour's m
+// run is one coalesced read and its count one division for all; the squares
+// meet in LDS, one lane per l sums them; then the first wavefront finishes the
+// workgroup's items.  With one thread per item (too few wavefronts, a scattered
+// read and a division per value) 2,000 atoms x 30 frames, l = 4 and 6, took 322
+// us; this takes 160 (190 with the items counted one by one).
 template <bool AVG>
 __global__ __launch_bounds__(256) void sph_steinhardt_kernel(SteinArgs a) {
     constexpr int NQ = ANL_SPH_LMAX_MAX + 1;
@@ -788,14 +795,19 @@ __global__ __launch_bounds__(256) void sph_steinhardt_kernel(SteinArgs a) {
             first += 2 * l + 1;
             nsel++;
         }
-        const uint64_t item0 = a.item0 + (uint64_t)blockIdx.x * STEIN_ITEMS;
-        for (uint32_t it = wave * (STEIN_ITEMS / 4); it < (wave + 1) * (STEIN_ITEMS / 4); ++it) {
-            if (lane < NQ) qs[it][lane] = 0.0;
-            if (item0 + it >= total) continue;  // uniform
-            const SteinItem t = stein_item(a, item0 + it);
-            if (!(t.na > 0)) continue;
+        const uint64_t item0 = a.item0 + (uint64_t)blockIdx.x * a.items;
+        const uint32_t per = a.items / 4, it0 = wave * per;  // this wavefront's
+        double nav = 0.0;                                    // lane it: the count of item it0 + it
+        if (lane < per && item0 + it0 + lane < total) nav = stein_count(a, stein_item(a, item0 + it0 + lane));
+        for (uint32_t e = lane; e < per * NQ; e += 64) qs[it0 + e / NQ][e % NQ] = 0.0;
+        wave_sync_lds();
+        for (unsigned long long left = __ballot(nav > 0); left; left &= left - 1) {
+            const uint32_t it = (uint32_t)__ffsll(left) - 1;
+            const SteinItem t = stein_item(a, item0 + it0 + it);
+            const double na = __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(nav), (int)it),
+                                               __builtin_amdgcn_readlane(__double2loint(nav), (int)it));
             const int32_t *nb = a.nbr + ((uint64_t)t.fl * a.N + t.ap) * a.nbr_stride + a.nbr_off[t.jt];
-            const uint32_t nk = min((uint32_t)t.na, a.nbr_stride - a.nbr_off[t.jt]);
+            const uint32_t nk = min((uint32_t)na, a.nbr_stride - a.nbr_off[t.jt]);
             double qb[2] = {0.0, 0.0};
             const double *Se[2];
 #pragma unroll
@@ -803,7 +815,7 @@ __global__ __launch_bounds__(256) void sph_steinhardt_kernel(SteinArgs a) {
                 const int l = max(el[c], 0);
                 const int mi = eo[c] == 0 ? l : (eo[c] <= l ? l - eo[c] : eo[c]);  // index of (l, m) in the m-run
                 Se[c] = t.Sb + (uint64_t)(l * l) * a.N + mi;
-                if (el[c] >= 0 && t.ti == t.jt) qb[c] = Se[c][t.ap * (2 * l + 1)] / t.na;
+                if (el[c] >= 0 && t.ti == t.jt) qb[c] = Se[c][t.ap * (2 * l + 1)] / na;
             }
             for (uint32_t k0 = 0; k0 < nk; k0 += 64) {
                 const uint32_t n = min(64u, nk - k0);
@@ -825,19 +837,19 @@ __global__ __launch_bounds__(256) void sph_steinhardt_kernel(SteinArgs a) {
             if (sl >= 0) {
                 double v = w[wave][s0];
                 for (int o = 1; o <= 2 * sl; ++o) v += w[wave][s0 + o];
-                qs[it][sl] = stein_q(v, t.na, sl);
+                qs[it0 + it][sl] = stein_q(v, na, sl);
             }
             wave_sync_lds();
         }
         __syncthreads();
-        if (wave != 0) return;
+        if (wave != 0 || lane >= a.items) return;
         k = item0 + lane;
     }
     if (k >= total) return;
     const SteinItem t = stein_item(a, k);
     const uint64_t ap = t.ap;
     const uint32_t b = t.b, jt = t.jt, fl = t.fl, ti = t.ti;
-    const double na = t.na;
+    const double na = stein_count(a, t);
     double q[NQ];
 #pragma unroll
     for (int l = 0; l < NQ; ++l) {
@@ -1237,10 +1249,11 @@ void steinhardt_calculate(anl_sph *h, uint64_t primo, uint32_t n, uint32_t skip,
         if ((nth + 255) / 256 > 0x7fffffffull) fail(ANL_ERR_ARG, "too many (frame, atom) pairs in one launch");
         // a launch holds less than 2^32 threads, four an item in the averaged form
         constexpr uint64_t MOST = 1ull << 29;
+        a.items = (uint32_t)std::min<uint64_t>(STEIN_ITEMS, std::max<uint64_t>(4, nth / STEIN_WGS / 4 * 4));
         for (a.item0 = 0; a.item0 < nth; a.item0 += MOST) {
             const uint64_t items = std::min(MOST, nth - a.item0);
             if (nbr)
-                hipLaunchKernelGGL(sph_steinhardt_kernel<true>, dim3((uint32_t)((items + STEIN_ITEMS - 1) / STEIN_ITEMS)),
+                hipLaunchKernelGGL(sph_steinhardt_kernel<true>, dim3((uint32_t)((items + a.items - 1) / a.items)),
                                    dim3(256), 0, s, a);
             else
                 hipLaunchKernelGGL(sph_steinhardt_kernel<false>, dim3((uint32_t)((items + 255) / 256)), dim3(256), 0, s, a);

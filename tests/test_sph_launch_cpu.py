@@ -25,3 +25,27 @@ for sann in (False, True):
     assert threads == 64 * N * F
     assert len({x[6:][-1] for x in d}) == 2
 """, tmp_path_factory, timeout=300)
+
+
+_SMALL = """
+def system(N, F=30, nt=1, nbin=1, lmax=2):
+    box = np.tile(np.array([0, 0, 0, 5, 5, 5.0]), (F, 1))
+    t = capi.DeviceTrajectory(np.zeros((F, N, 3)), box, (np.arange(N) % nt).astype(np.int32), nt)
+    h = capi.DeviceSph(t, [(0.5, 3.0)] * nt ** 2, nbin, lmax)
+    h.set_neighbours([(8, 4.0, 4.0)] * nt)
+    log()
+    return h
+"""
+
+
+def test_averaged_form_fills_the_chip(tmp_path_factory):
+    """Items per workgroup of the averaged order parameter: 64 for a large
+    calculation, fewer where that leaves less than 2,048 workgroups."""
+    fake_hip.run(_SMALL + """
+for N, F, nt, nbin, want in ((10, 1, 1, 1, 3), (200, 20, 1, 1, 1000), (300, 20, 3, 6, 2077), (2000, 30, 2, 1, 2143),
+                             (20000, 20, 1, 1, 6250)):
+    h = system(N, F, nt, nbin)
+    h.steinhardt(F, 1, 0, [2], 4, averaged=True)
+    x = launches(log(), "sph_steinhardt_kernel")
+    assert len(x) == 1 and int(x[0][3].split(",")[0]) == want, (N, x[0][3])
+""", tmp_path_factory)
