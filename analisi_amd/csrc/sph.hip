@@ -28,8 +28,8 @@
 //     through LDS 32 at a time; entries with 0 <= t2 - t1 < leff go to
 //     G[problem][t1 index][t2 - t1].
 //  3. sph_reduce_kernel: R[problem][dt] += sum over t1 of G, in t1 order.
-// The host divides R by (number of t1) x (atoms of type_i) and writes the
-// reference layout [dt][type_i][type_j][bin][k] with k holding l = lmax - k.
+//     The last chunk's divides by (number of t1) x (atoms of type_i) and writes
+//     the reference layout [dt][type_i][type_j][bin][k], k holding l = lmax - k.
 // Every sum has a fixed order: results are deterministic.
 //
 // Steinhardt<lmax> (steinhardt.cpp:90-236) reuses step 1 on frames
@@ -690,16 +690,25 @@ __global__ __launch_bounds__(256) void sph_gram_mfma_kernel(SphGramArgs a) {
     }
 }
 
-// R[p][dt] += sum over the chunk's t1 (in order) of G[p][t1][dt]
+// R[p][dt] += sum over the chunk's t1 (in order) of G[p][t1][dt], p = ((ti nt +
+// tj) nbin + b) L1 + l.  After the last chunk (out) R / N_ti / n0 goes to
+// out[dt][ti][tj][b][lmax - l] instead (per = nt nbin).
 __global__ __launch_bounds__(256) void sph_reduce_kernel(const double *G, double *R, uint32_t nprob, uint32_t n0c,
-                                                         uint32_t leff) {
+                                                         uint32_t leff, const uint32_t *tstart, uint32_t L1, uint32_t per,
+                                                         double n0, double *out) {
     const uint64_t k = (uint64_t)blockIdx.x * 256 + threadIdx.x;
     if (k >= (uint64_t)nprob * leff) return;
     const uint64_t p = k / leff, dt = k - p * leff;
     const double *g = G + p * n0c * leff + dt;
     double s = 0.0;
     for (uint32_t e = 0; e < n0c; ++e) s += g[(uint64_t)e * leff];
-    R[k] = R[k] + s;
+    const double r = R[k] + s;
+    if (!out) {
+        R[k] = r;
+        return;
+    }
+    const uint32_t q = (uint32_t)p / L1, l = (uint32_t)p - q * L1, ti = q / per;
+    out[dt * nprob + q * L1 + (L1 - 1 - l)] = r / (double)(tstart[ti + 1] - tstart[ti]) / n0;
 }
 
 constexpr uint32_t STEIN_MAXL = 16;  // l values of one histogram
@@ -900,20 +909,6 @@ __global__ __launch_bounds__(256) void sph_steinhardt_kernel(SteinArgs a) {
     }
 }
 
-// R[((ti*nt + tj)*nbin + b)*L1 + l][dt] / N_ti / n0 -> out[dt][ti][tj][b][lmax - l]
-// (per = nt*nbin).  One launch in place of a pass over the result on the host
-// with two divisions a value (26,400 values: 65 us less per call).
-__global__ __launch_bounds__(256) void sph_finish_kernel(const double *__restrict__ R, const uint32_t *__restrict__ tstart,
-                                                         uint32_t nprob, uint32_t leff, uint32_t L1, uint32_t per,
-                                                         double n0, double *__restrict__ out) {
-    const uint64_t k = (uint64_t)blockIdx.x * 256 + threadIdx.x;
-    if (k >= (uint64_t)nprob * leff) return;
-    const uint32_t dt = (uint32_t)(k / nprob), r = (uint32_t)(k - (uint64_t)dt * nprob);
-    const uint32_t q = r / L1, p = q * L1 + (L1 - 1 - (r - q * L1)), ti = q / per;
-    const double na = (double)(tstart[ti + 1] - tstart[ti]);
-    out[k] = R[(uint64_t)p * leff + dt] / na / n0;
-}
-
 __global__ __launch_bounds__(256) void sph_zero_kernel(double *p, uint64_t n) {
     for (uint64_t k = (uint64_t)blockIdx.x * 256 + threadIdx.x; k < n; k += (uint64_t)gridDim.x * 256) p[k] = 0.0;
 }
@@ -1004,12 +999,17 @@ uint64_t radius_bytes(const anl_sph *h, uint64_t nfr) {
     return h->block_screen ? nfr * ((h->tr->N + 63) / 64) * sizeof(double4) : 0;
 }
 
+// Atoms up to which the neighbour lists go through all blocks: their spheres are a
+// launch of their own, 5 us of a call (22 atoms, one frame: 80 us with them, 57
+// without; 200 atoms, 60 frames: no difference).
+constexpr uint64_t SANN_NO_SPHERES = 256;
+
 // one launch of launch_density, which checks the sizes and reads the overflow of the lists
 void launch_density_range(anl_sph *h, uint64_t f0, uint64_t fstride, uint32_t nfr, double *S, double4 *rad,
                           hipStream_t s, int32_t *nbr, uint32_t lm) {
     SphDensArgs a{};
     a.fstride = fstride;
-    a.block_rad = h->block_screen ? rad : nullptr;
+    a.block_rad = h->block_screen && !(h->sann && h->tr->N <= SANN_NO_SPHERES) ? rad : nullptr;
     auto block_spheres = [&] {
         if (!a.block_rad) return;
         const uint64_t nb = (uint64_t)nfr * ((h->tr->N + 63) / 64);
@@ -1128,9 +1128,9 @@ void sph_calculate(anl_sph *h, uint64_t primo, uint32_t n, uint32_t tmax, uint32
     if (nprob > 65535) fail(ANL_ERR_ARG, "too many (type, type, bin, l) channels for one launch (at most 65535)");
     const uint64_t nfr_max = (rc - 1) * skip + leff;
     const uint64_t offS = 0, offG = a256(nfr_max * fbytes), offR = offG + a256((uint64_t)nprob * rc * leff * 8);
-    const uint64_t offQ = offR + a256((uint64_t)nprob * leff * 8);
+    const uint64_t offO = offR + a256((uint64_t)nprob * leff * 8), offQ = offO + a256((uint64_t)nprob * leff * 8);
     char *w = (char *)workspace(h, offQ + a256(radius_bytes(h, nfr_max)));
-    double *S = (double *)(w + offS), *G = (double *)(w + offG), *R = (double *)(w + offR);
+    double *S = (double *)(w + offS), *G = (double *)(w + offG), *R = (double *)(w + offR), *out = (double *)(w + offO);
     double4 *rad = (double4 *)(w + offQ);
     hipStream_t s = nullptr;
     const uint64_t nR = (uint64_t)nprob * leff;
@@ -1162,14 +1162,10 @@ void sph_calculate(anl_sph *h, uint64_t primo, uint32_t n, uint32_t tmax, uint32
         hipLaunchKernelGGL(sph_gram_mfma_kernel, dim3((uint32_t)(ncb * g.ncol), nprob), dim3(256), 0, s, g);
         ANL_HIP(hipGetLastError());
         hipLaunchKernelGGL(sph_reduce_kernel, dim3((uint32_t)((nR + 255) / 256)), dim3(256), 0, s, G, R, nprob,
-                           n0c, leff);
+                           n0c, leff, h->d_tstart, L1, nt * h->nbin, (double)n0, e0 + rc < n0 ? nullptr : out);
         ANL_HIP(hipGetLastError());
     }
-    // the Gram values are no longer needed: the result takes their place
-    hipLaunchKernelGGL(sph_finish_kernel, dim3((uint32_t)((nR + 255) / 256)), dim3(256), 0, s, R, h->d_tstart, nprob,
-                       leff, L1, nt * h->nbin, (double)n0, G);
-    ANL_HIP(hipGetLastError());
-    ANL_HIP(hipMemcpy(out_host, G, nR * sizeof(double), hipMemcpyDeviceToHost));
+    ANL_HIP(hipMemcpy(out_host, out, nR * sizeof(double), hipMemcpyDeviceToHost));
 }
 
 // steinhardt.cpp:47-236 (no neighbour list, not averaged): frames primo + i,

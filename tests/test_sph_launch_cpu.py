@@ -49,3 +49,22 @@ for N, F, nt, nbin, want in ((10, 1, 1, 1, 3), (200, 20, 1, 1, 1000), (300, 20, 
     x = launches(log(), "sph_steinhardt_kernel")
     assert len(x) == 1 and int(x[0][3].split(",")[0]) == want, (N, x[0][3])
 """, tmp_path_factory)
+
+
+def test_small_calls_launch_no_more_than_they_need(tmp_path_factory):
+    """The densities' Gram values are reduced and laid out by one kernel, once a
+    chunk; neighbour lists of few atoms take no bounding spheres."""
+    fake_hip.run(_SMALL + """
+def names(e):
+    return [x[5].split("sph_")[1].split("_kernel")[0] for x in launches(e, "sph_")]
+h = system(100, 40)
+h.calculate(20, 10, 2, 0)
+assert names(log()) == ["zero", "density_sann", "gram_mfma", "reduce"]
+h = system(257, 40)
+h.calculate(20, 10, 2, 0)
+assert names(log()) == ["zero", "block_radius", "density_sann", "gram_mfma", "reduce"]
+h.set_budget(5 * 257 * 9 * 8)                         # densities of two t1 values and their lags
+h.calculate(4, 4, 1, 0)
+n = names(log())
+assert n.count("reduce") == n.count("gram_mfma") == 2 and n[-1] == "reduce", n
+""", tmp_path_factory)
