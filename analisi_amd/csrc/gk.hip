@@ -147,7 +147,7 @@ __global__ __launch_bounds__(256, 1) void gk_chain_kernel(const GkArgs a) {
     const uint64_t primo = a.bl.primo[blk];
     const uint32_t seg = a.bl.n[blk] / a.n_seg;
     const uint32_t first = seg * iseg + (seg * iseg) % a.skip, end = seg * (iseg + 1);  // :208
-    const uint32_t n0 = first < end ? (end - first + a.skip - 1) / a.skip : 0;
+    const uint32_t n0 = first < end ? (end - first - 1) / a.skip + 1 : 0;
     const uint32_t nst = (n0 + T - 1) / T;
     double JJ = 0.0;
     if (wave == 0) {
@@ -514,6 +514,46 @@ __global__ __launch_bounds__(64, 3) void gk_dense_kernel(const GkArgs a) {
         if (it == 0 && pair == 0)
             for (uint32_t k = np; k < a.narr; k++) o[k] = 0.0;
     }
+}
+
+// The same means where a lag has few t0 (gk_plan): a thread holds every pair of
+// one lag and takes the segments one after the other, with true divisions.  The
+// kernels above would fill their stages for a term or two, in a workgroup per
+// segment.
+template <int NC>
+__global__ __launch_bounds__(64) void gk_few_kernel(const GkArgs a) {
+    constexpr int NP = NC * NC;
+    const uint32_t it = blockIdx.x * 64 + threadIdx.x, blk = blockIdx.y;
+    if (it >= a.leff) return;
+    const double *d = a.data + a.bl.primo[blk] * a.ncols;
+    const uint32_t seg = a.bl.n[blk] / a.n_seg;
+    double v[NP] = {};
+    for (uint32_t iseg = 0; iseg < (seg ? a.n_seg : 0); iseg++) {  // empty segments: the mean of zeros
+        double JJ[NP] = {};
+        uint32_t cont = 0;
+        const uint32_t first = seg * iseg + (seg * iseg) % a.skip, end = seg * (iseg + 1);  // :208
+        for (uint64_t jm = first; jm < end; jm += a.skip) {
+            const double *la = d + jm * a.ncols, *lb = la + (uint64_t)it * a.ncols;
+            double A[NC][3], B[NC][3];
+#pragma unroll
+            for (int c = 0; c < NC; c++)
+#pragma unroll
+                for (int x = 0; x < 3; x++) A[c][x] = la[a.idx[c] + x], B[c][x] = lb[a.idx[c] + x];
+            const double dc = (double)++cont;
+#pragma unroll
+            for (int k = 0; k < NP; k++) {
+                const double q = (A[k / NC][0] * B[k % NC][0] + A[k / NC][1] * B[k % NC][1]) + A[k / NC][2] * B[k % NC][2];
+                JJ[k] = JJ[k] + (q / 3.0 - JJ[k]) / dc;  // :200-228
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < NP; k++) v[k] = v[k] + (JJ[k] - v[k]) / (double)(iseg + 1);  // :230-237
+    }
+    double *o = a.out + blk * a.out_stride + (uint64_t)it * a.narr;
+#pragma unroll
+    for (int k = 0; k < NP; k++) o[k] = v[k];
+    if (it == 0)  // the integrals start from zero
+        for (uint32_t k = NP; k < a.narr; k++) o[k] = 0.0;
 }
 
 // The running mean over the segments (:230-237) of the segment means.
@@ -1036,15 +1076,6 @@ void gk_epilogue(double *d, uint32_t narr, uint32_t ncur, uint32_t leff, int sub
     gk_schur_launch(d, narr, ncur, leff, s, nblocks, stride);
 }
 
-// Bytes of the segment means of a call, 0 where it keeps none: more than the
-// cap, or one segment.
-constexpr size_t GK_SEG_BYTES = 1ull << 30;
-static size_t gk_segment_bytes(uint32_t ncur, uint32_t leff, uint32_t n_seg, uint32_t nblocks) {
-    if (n_seg < 2 || n_seg > 65535) return 0;
-    const size_t need = (size_t)std::min(GK_MAXB, nblocks) * n_seg * ncur * ncur * leff * sizeof(double);
-    return need <= GK_SEG_BYTES ? need : 0;
-}
-
 void gk_reciprocals(double2 *rec, uint64_t n, hipStream_t s) {
     hipLaunchKernelGGL(gk_reciprocal_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, rec, n);
     ANL_HIP(hipGetLastError());
@@ -1055,6 +1086,7 @@ void gk_reciprocals(double2 *rec, uint64_t n, hipStream_t s) {
 // per CU), the dense kernel's by 0.2-0.3 ms from 1.4 ms on (2.0 against
 // 2.7 ms at 1,024 and 2 currents, 2.9 against 2.6 ms at 2,048 and 4).
 constexpr uint64_t GK_DENSE_CHAINS = 1792;
+
 static bool gk_can_allocate(hipStream_t st) {
     hipStreamCaptureStatus c = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(st, &c) != hipSuccess) {
@@ -1064,12 +1096,49 @@ static bool gk_can_allocate(hipStream_t st) {
     return c == hipStreamCaptureStatusNone;
 }
 
-// The segments of a block run side by side into segm (gk_segment_bytes) and
+// How the FP64 form runs a call.
+struct GkPlan {
+    bool few = false;      // gk_few_kernel
+    size_t seg_bytes = 0;  // of the segment means of segments side by side; 0: one segment, or more than the cap
+};
+constexpr size_t GK_SEG_BYTES = 1ull << 30;
+
+// The smaller of two estimates (us) decides for gk_few_kernel, which takes K
+// terms of a lag one after the other (at least one per segment), 0.16 to 1.3 us
+// each by the number of currents.  A workgroup of gk_chain_kernel takes 14 ns of
+// the chip before its first term, a wavefront of gk_dense_kernel 2; segments side
+// by side take a launch and a division each, one after the other a launch each.
+// Measured (us a call, chain or dense and few): 2 currents, one segment, 40
+// lags, K 4 25 and 23, K 16 25 and 28; 1,500 lags x 16 blocks, K 16 216 and 225,
+// K 64 239 and 229; in 16 segments K 16 536 and 225, K 100 580 and 250; 4
+// currents, 40 lags, 16 segments, K 16 35 and 57; 6,000 lags x 16 blocks, 64
+// segments, K 100 25,700 and 4,400.
+static GkPlan gk_plan(uint32_t ncur, uint32_t leff, uint32_t skip, uint32_t n_seg, const uint32_t *n, uint32_t nblocks,
+                      bool side_by_side = true) {
+    static const double term[GK_MAXC] = {0.16, 0.41, 0.8, 1.3};
+    GkPlan P;
+    const uint64_t nb = std::min(GK_MAXB, nblocks), pairs = ncur * ncur;
+    const uint64_t need = nb * n_seg * pairs * leff * sizeof(double);
+    if (side_by_side && n_seg > 1 && n_seg <= 65535 && need <= GK_SEG_BYTES) P.seg_bytes = need;
+    uint64_t seg = 0;
+    for (uint32_t b = 0; b < nblocks; b++) seg = std::max<uint64_t>(seg, n[b] / n_seg);
+    const double terms = (double)((seg + skip - 1) / skip), lags = (leff + 63) / 64;
+    const double chains = lags * pairs * n_seg * nb, waves = lags * nb;
+    const bool dense = skip == 1 && chains > GK_DENSE_CHAINS;
+    const double few = n_seg * terms * term[ncur - 1] * (1 + waves / 4096);
+    const double chain = 1.5 + 0.03 * terms + chains * (dense ? 0.002 : 0.0135) +
+                         (n_seg > 1 ? (P.seg_bytes ? 2.5 + 0.15 * n_seg : 4.0 * n_seg) : 0.0);
+    P.few = few < chain;
+    if (P.few) P.seg_bytes = 0;
+    return P;
+}
+
+// The segments of a block run side by side into segm (GkPlan::seg_bytes) and
 // are folded afterwards; without it one launch per segment folds into the
 // output.
 static void gk_fp64_enqueue_blocks(anl_series *s, const uint32_t *idx_j, uint32_t ncur, uint32_t skip, uint32_t leff,
                                    uint32_t n_seg, const uint64_t *primo, const uint32_t *n, uint32_t nblocks,
-                                   double *d, double *segm, hipStream_t st) {
+                                   double *d, const GkPlan &plan, double *segm, hipStream_t st) {
     const uint32_t narr = 3 * ncur * ncur + 2;
     const uint64_t stride = (uint64_t)leff * narr;
     for (uint32_t b0 = 0; b0 < nblocks; b0 += GK_MAXB) {
@@ -1091,6 +1160,17 @@ static void gk_fp64_enqueue_blocks(anl_series *s, const uint32_t *idx_j, uint32_
         for (uint32_t b = 0; b < nb; b++) {
             a.bl.primo[b] = primo[b0 + b];
             a.bl.n[b] = n[b0 + b];
+        }
+        if (plan.few) {
+            const dim3 grid((leff + 63) / 64, nb);
+            switch (ncur) {
+                case 1: hipLaunchKernelGGL(gk_few_kernel<1>, grid, dim3(64), 0, st, a); break;
+                case 2: hipLaunchKernelGGL(gk_few_kernel<2>, grid, dim3(64), 0, st, a); break;
+                case 3: hipLaunchKernelGGL(gk_few_kernel<3>, grid, dim3(64), 0, st, a); break;
+                default: hipLaunchKernelGGL(gk_few_kernel<4>, grid, dim3(64), 0, st, a); break;
+            }
+            ANL_HIP(hipGetLastError());
+            continue;
         }
         const dim3 grid((leff + 63) / 64 * ncur * ncur, segm ? n_seg : 1, nb);
         for (uint32_t k = 0; k < (segm ? 1 : n_seg); k++) {
@@ -1139,24 +1219,27 @@ uint32_t gk_block_checks(anl_series *s, const uint32_t *idx_j, uint32_t ncur, ui
     return leff0;
 }
 
+static void gk_defaults(uint32_t &n_seg, uint32_t &skip) {
+    n_seg = std::max(n_seg, 1u);  // greenkubo...cpp:50-53
+    skip = std::max(skip, 1u);
+}
 static void gk_enqueue_checks(int form, uint32_t nblocks, const double *mean, const double *var) {
     if ((mean || var) && (!mean || !var || nblocks < 2))
         fail(ANL_ERR_ARG, "block mean and variance need both outputs and at least two blocks");
     if (form != ANL_GK_FP64 && form != ANL_GK_MFMA) fail(ANL_ERR_ARG, "unknown Green-Kubo form");
 }
 
-// A checked call (gk_block_checks, gk_enqueue_checks, leff > 0) on stream st;
-// segm: the FP64 form's segment means, or null.
+// A checked call (gk_block_checks, gk_enqueue_checks, leff > 0; n_seg and skip at
+// least 1) on stream st; plan and segm (its segment means, or null) are the
+// FP64 form's.
 static void gk_enqueue(anl_series *s, const uint32_t *idx_j, uint32_t ncur, uint32_t skip, uint32_t leff, uint32_t n_seg,
                        int subtract_mean, uint32_t start_mean, const uint64_t *primo, const uint32_t *n,
-                       uint32_t nblocks, int form, double *out_dev, double *mean_dev, double *var_dev, double *segm,
-                       hipStream_t st) {
-    if (n_seg < 1) n_seg = 1;  // greenkubo...cpp:50-53
-    if (skip == 0) skip = 1;
+                       uint32_t nblocks, int form, double *out_dev, double *mean_dev, double *var_dev,
+                       const GkPlan &plan, double *segm, hipStream_t st) {
     const uint32_t narr = 3 * ncur * ncur + 2;
     const uint64_t stride = (uint64_t)leff * narr;
     if (form == ANL_GK_MFMA) gk_mfma_enqueue_blocks(s, idx_j, ncur, skip, leff, n_seg, primo, n, nblocks, out_dev, st);
-    else gk_fp64_enqueue_blocks(s, idx_j, ncur, skip, leff, n_seg, primo, n, nblocks, out_dev, segm, st);
+    else gk_fp64_enqueue_blocks(s, idx_j, ncur, skip, leff, n_seg, primo, n, nblocks, out_dev, plan, segm, st);
     // the FP64 form keeps the reference's serial scans (bit-identical results)
     gk_epilogue(out_dev, narr, ncur, leff, subtract_mean, start_mean, st, nblocks, stride, form == ANL_GK_FP64, s->rec);
     if (mean_dev) mediavar_blocks(nullptr, out_dev, nullptr, nblocks, stride, mean_dev, var_dev, st);
@@ -1239,10 +1322,12 @@ int anl_gk_calculate_blocks_async(anl_series *s, const uint32_t *idx_j, uint32_t
         if (leff == 0) return;
         ensure_device();
         hipStream_t st = (hipStream_t)stream;
-        const size_t need = form == ANL_GK_FP64 ? gk_segment_bytes(ncur, leff, n_seg, nblocks) : 0;
-        GkSegments seg(s, need, st);
+        gk_defaults(n_seg, skip);
+        GkPlan plan = form == ANL_GK_FP64 ? gk_plan(ncur, leff, skip, n_seg, n, nblocks) : GkPlan{};
+        GkSegments seg(s, plan.seg_bytes, st);
+        if (plan.seg_bytes && !seg.p) plan = gk_plan(ncur, leff, skip, n_seg, n, nblocks, false);
         gk_enqueue(s, idx_j, ncur, skip, leff, n_seg, subtract_mean, start_mean, primo, n, nblocks, form, out_dev,
-                   mean_dev, var_dev, seg.p, st);
+                   mean_dev, var_dev, plan, seg.p, st);
     });
 }
 
@@ -1267,9 +1352,10 @@ int anl_gk_calculate_blocks(anl_series *s, const uint32_t *idx_j, uint32_t ncur,
         constexpr size_t PIECE = 2u << 20, RING = 3;
         const size_t pieces = (total + PIECE - 1) / PIECE;
         const unsigned nth = pieces < 2 ? 0 : std::min(8u, std::max(1u, std::thread::hardware_concurrency()));
-        const GkWorkspace w(s, (all + 2 * len) * sizeof(double),
-                            form == ANL_GK_FP64 ? gk_segment_bytes(ncur, leff, n_seg, nblocks) : 0,
-                            nth ? RING * PIECE : 0);
+        gk_defaults(n_seg, skip);
+        GkPlan plan = form == ANL_GK_FP64 ? gk_plan(ncur, leff, skip, n_seg, n, nblocks) : GkPlan{};
+        const GkWorkspace w(s, (all + 2 * len) * sizeof(double), plan.seg_bytes, nth ? RING * PIECE : 0);
+        if (plan.seg_bytes && !w.segm) plan = gk_plan(ncur, leff, skip, n_seg, n, nblocks, false);
         double *d = w.dev();
         char *ring = (char *)w.w->s.pin;
         constexpr int64_t NOT_YET = -1, GIVE_UP = -2;  // no kernels yet; there will be no output
@@ -1324,7 +1410,7 @@ int anl_gk_calculate_blocks(anl_series *s, const uint32_t *idx_j, uint32_t ncur,
         };
         try {
             gk_enqueue(s, idx_j, ncur, skip, leff, n_seg, subtract_mean, start_mean, primo, n, nblocks, form, d,
-                       mean_host ? d + all : nullptr, var_host ? d + all + len : nullptr, w.segm, 0);
+                       mean_host ? d + all : nullptr, var_host ? d + all + len : nullptr, plan, w.segm, 0);
             if (nth) {
                 pool.reserve(nth);
                 for (unsigned k = 0; k < nth; k++) pool.emplace_back(work, k);
@@ -1383,10 +1469,13 @@ static int gk_calculate_host(anl_series *s, const uint32_t *idx_j, uint32_t ncur
         if (leff == 0) return;
         ensure_device();
         const size_t bytes = (size_t)leff * (3 * ncur * ncur + 2) * sizeof(double);
-        const GkWorkspace w(s, bytes, form == ANL_GK_FP64 ? gk_segment_bytes(ncur, leff, n_seg, 1) : 0, 0);
+        gk_defaults(n_seg, skip);
+        GkPlan plan = form == ANL_GK_FP64 ? gk_plan(ncur, leff, skip, n_seg, &n, 1) : GkPlan{};
+        const GkWorkspace w(s, bytes, plan.seg_bytes, 0);
+        if (plan.seg_bytes && !w.segm) plan = gk_plan(ncur, leff, skip, n_seg, &n, 1, false);
         try {
             gk_enqueue(s, idx_j, ncur, skip, leff, n_seg, subtract_mean, start_mean, &primo, &n, 1, form,
-                       w.dev(), nullptr, nullptr, w.segm, 0);
+                       w.dev(), nullptr, nullptr, plan, w.segm, 0);
             ANL_HIP(hipMemcpy(out_host, w.dev(), bytes, hipMemcpyDeviceToHost));
         } catch (...) {
             (void)hipStreamSynchronize(0);  // the workspace goes back unused

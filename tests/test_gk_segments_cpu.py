@@ -152,3 +152,26 @@ for wait in (0, 0, 1000000):
     t = time.perf_counter() - t
 assert t > 1.9 and used[2] < t / 2, (used, t)
 """, tmp_path_factory)
+
+
+def test_few_terms_a_lag(tmp_path_factory):
+    """Lags of few t0 take one launch of a thread each, however many segments and
+    whether or not their means could be kept; longer ones do not."""
+    fake_hip.run(_SETUP + """
+def names(f):
+    log()
+    f()
+    return [x[5].split("gk_")[1].split("_kernel")[0] for x in launches(log(), "gk_")][:-2]  # without the epilogue
+gk = lambda n, tmax, skip, g: names(lambda: s.gk([0, 3], skip, tmax, n, g, False, 0, 0))
+assert gk(2, 2, 1, 1) == ["few"]
+assert gk(31, 30, 1, 100) == gk(53, 53, 65, 2) == gk(50, 50, 1, 4000000) == ["few"]
+assert gk(3000, 2000, 1000, 30) == ["few"]
+assert gk(200, 100, 1, 1) == ["chain"]
+assert gk(4000, 2000, 1, 4) == ["chain", "segments"]
+fake.fake_capture(1)
+out = device(2000 * 14 * 8)
+assert names(lambda: run_async(out, 2000, 4000)) == ["chain"] * 4
+assert names(lambda: run_async(out, 10, 20)) == ["few"]
+fake.fake_capture(0)
+assert [len(gk(4500, 4000, 4294967280, 1)), len(gk(4500, 4500, 1, 1))] == [1, 1]
+""", tmp_path_factory)
