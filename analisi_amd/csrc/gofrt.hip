@@ -1930,7 +1930,7 @@ struct anl_gofrt {
     anl_traj *tr = nullptr;
     GofrtTuning tune;
     bool tuned = false;           // the caller or the environment set the shape, or the autotuner did
-    int fits = -1;                // clusters_fit, -1 not looked at
+    double crowd = -1;            // clusters_fit, -1 not looked at
     double rmin = 0, rmax = 0, dr = 0, rmin2 = 0, rmax2 = 0;
     uint32_t nbin = 0, lmax = 0, skip = 1, every = 1;
     int form = ANL_GOFRT_AUTO;
@@ -2011,19 +2011,30 @@ bool use_cells(anl_gofrt *g) {
     return g->cells == 1;
 }
 
-// Whether the cluster screen pays for a launch shape nobody chose, from frame
-// 0's groups: `unfit`, the share of wavefronts too wide for it (they fall back
-// to the 16-bit screen in a kernel with fewer registers left for it), and
-// `near`, the volume a compact wavefront cannot skip over that of the cell.  A
-// wavefront's radius is taken as half the extent of its two groups' spheres.
-// The line near + unfit = 0.9 is where 6 t0 x 6 lags of 4,000 to 40,000 atoms
-// and 40 x 10 of 1,000 to 8,000, rmax 0.04 to 0.35 of a cubic cell, broke
-// even.  Cluster against 16-bit: 4,000 atoms 290 / 325 us at 0.57, 476 / 428 at
-// 1.5; 12,000 1.61 / 1.75 ms at 0.85, 2.29 / 2.17 at 1.35; 24,000 6.08 / 6.97
-// at 0.82, 10.5 / 8.84 at 1.23; 1,000 atoms 547 / 411 us at 1.4 (rmax 0.1 of
-// the cell) and 635 / 477 at 2 and more.
-bool clusters_fit(anl_gofrt *g, float rho_cap) {
-    if (g->fits < 0) {
+// Whether the cluster screen pays for a launch shape nobody chose: `crowd`, from
+// frame 0's groups, below a line.  crowd is the volume that a compact wavefront
+// cannot skip over that of the cell, and half the share of wavefronts too wide
+// for the screen (they fall back to the 16-bit one in a kernel with fewer
+// registers left for it).  A wavefront's radius is taken as half the extent of
+// its two groups' spheres.  The lines are where cluster and 16-bit screen break
+// even for liquids of 1,000 to 30,000 atoms, rmax 0.05 to 0.4 of a cubic cell, 10
+// to 150 t0 x 6 to 50 lags: 2 up to 2,048 atoms, 1.15 to 1.25 above, 0.25 more
+// where many counters make the 16-bit kernel's rechecks slow; and 0.9 where the
+// chip is not full (U (workgroup, t0) pairs), as a workgroup's longer start is
+// not hidden there.  Cluster / 16-bit at crowd, 100 bins, us: 1,000 atoms 60 x 10
+// 306 / 355 at 1.66, 374 / 369 at 2.5, 10 x 10 160 / 136 at 1.66; 2,000 40 x 8 480 /
+// 672 at 1.77, 723 / 721 at 2.2, 10 x 10 287 / 255 at 0.95; 3,000 813 / 1,024 at
+// 0.83, 1,220 / 1,008 at 1.44; 4,000 8,851 / 9,372 at 1.26, 12,367 / 11,583 at 1.93;
+// 12,000 10,989 / 11,222 at 1.14, 17,120 / 14,138 at 1.72; 1,000 bins: 4,000 11,068 /
+// 13,512 at 1.26; 12,000 14,283 / 16,435 at 1.14.
+bool below_line(const anl_gofrt *g, double U) {
+    const uint64_t N = g->tr->N;
+    if (U < 2048) return g->crowd < 0.9;
+    if (N < 4000) return g->crowd < (N <= 2048 ? 2.0 : 1.15);
+    return g->crowd < (nch_of(g->tr) * (uint64_t)g->nbin >= 2000 ? 1.5 : 1.25);
+}
+bool clusters_fit(anl_gofrt *g, float rho_cap, double U) {
+    if (g->crowd < 0) {
         anl_traj *tr = g->tr;
         const uint64_t ng = (tr->N + 31) / 32;
         std::vector<uint4> gr(ng);
@@ -2046,14 +2057,15 @@ bool clusters_fit(anl_gofrt *g, float rho_cap) {
         reach /= (double)all;
         const double near = 4.0 / 3.0 * 3.14159265358979 * reach * reach * reach / (c.L[0] * c.L[1] * c.L[2]);
         const double unfit = 1.0 - (double)fit / (double)all;
-        g->fits = near + unfit < 0.9;
+        g->crowd = near + 0.5 * unfit;
     }
-    return g->fits == 1;
+    return below_line(g, U);
 }
 
 struct Launch {
     std::vector<BlockInfo> blocks;
     std::vector<WorkItem> work;   // empty for one block: [k0, k1) in chunks, from the arguments
+    double pairs = 0;             // (workgroup, t0) pairs
     uint32_t k0 = 0, k1 = 0, chunk = 1;
     uint32_t nwork = 0;
     uint32_t leff_max = 0;
@@ -2074,6 +2086,35 @@ size_t fp64_lds(const anl_gofrt *g) {
 }
 size_t fp64_stage(const anl_gofrt *g) { return (fp64_lds(g) + 15) / 16 * 16; }
 
+// t0 that a workgroup takes at least, where a launch is split finer to fill the
+// chip.  A workgroup costs the chip a us beside its t0: its start, the clearing
+// and reading of its counters, an atomic for each that was hit.  U (workgroup,
+// t0) pairs in workgroups of c t0 thus take a U / c us of that, beside U B / 1,000
+// of work (B us a t0; a thousand workgroups at once) and the last one's B c: the
+// smallest c that keeps the first below the others, as long as it leaves 512
+// workgroups (128 of the split plain form, which takes four t0 at once).
+// Us a call, c 1, 2, 4, 8, 16: 30 atoms, 200 t0 x 100 lags 2,444, 1,250, 659, 379,
+// 261; 300 atoms, 100 x 50 1,613, 892, 579, 474, 625; 1,000, 40 x 10, rmax 0.1 of
+// the cell 381, 272, 252, 360, 662; 4,000, 40 x 10 1,911, 1,158, 1,218, 1,382, 2,384;
+// 8,000 4,060, 4,226, 4,755, 5,383, 5,986; split plain form, 30 atoms as above 540,
+// 535, 531, 302, 221.  The cost of a start and of a t0 are fits to such rows.
+uint64_t flush_chunk(const anl_gofrt *g, uint32_t tile, int form, bool cells, double U) {
+    const Cell &cell = g->tr->cell0;
+    const bool split = tile < WG, screened = form == ANL_GOFRT_SCREENED;
+    const bool cluster = screened && g->tune.cluster != 0 && (g->tuned || below_line(g, U));
+    const double N = (double)g->tr->N, nt = g->tr->nt, nh = nt * (nt + 1) * g->nbin;
+    const double f = std::min(1.0, 4.19 * (g->rmax2 * g->rmax - g->rmin2 * g->rmin) / (cell.L[0] * cell.L[1] * cell.L[2]));
+    const double a = (cluster ? 0.45 : 0.1) + 1e-4 * std::min(nt * nt * g->nbin, tile * N * f) + 7e-6 * nh;
+    const double B = cells ? 6 + N * (0.048 + 0.6 * f) : screened ? 6 + N * (0.04 + 0.25 * f) : split ? 2.5 + 0.03 * N : 6 + 0.3 * N;
+    const double W = U * B / 1000;  // B c^2 + W c = a U
+    const double c = (std::sqrt(W * W + 4 * B * a * U) - W) / (2 * B);
+    if (split) return 4 * (uint64_t)std::min(c / 4 + 0.4, U / 128 / 4);
+    // the cluster screen's start wants two t0 in any full launch, and already in
+    // three quarters of one where they are short: 6,000 atoms, 16 t0 x 6 lags,
+    // rmax 0.1 of the cell 814 us at one t0, 647 at two; 8,000, 12 x 6 940 and 1,155
+    return (uint64_t)std::min(std::max(std::ceil(c - 0.3), cluster && (U >= 3600 || c > 1.18) ? 2.0 : 1.0), U / 512);
+}
+
 // Splits every block's t0 range into chunks: a chunk bounds the LDS counters
 // (each t0 adds at most 256*N to one bin: 256*N*chunk < 2^32) and sets the
 // work per workgroup (the tuned number of pair evaluations), finer where the
@@ -2081,8 +2122,9 @@ size_t fp64_stage(const anl_gofrt *g) { return (fp64_lds(g) + 15) / 16 * 16; }
 Launch plan(anl_gofrt *g, const uint64_t *primo, const uint32_t *n, uint32_t nblocks) {
     Launch L;
     const uint64_t N = g->tr->N;
-    const bool split = choose_form(g) == ANL_GOFRT_FP64 && N <= FP64_SPLIT_ATOMS &&
-                       fp64_stage(g) + SPLIT_WG / 64 * STAGE_J <= 160 * 1024 && !use_cells(g);
+    const int form = choose_form(g);
+    const bool plain = form == ANL_GOFRT_FP64, cells = plain && use_cells(g);
+    const bool split = plain && !cells && N <= FP64_SPLIT_ATOMS && fp64_stage(g) + SPLIT_WG / 64 * STAGE_J <= 160 * 1024;
     if (split) L.tile = 64;
     uint64_t cap = (0xFFFFFFFFull / ((uint64_t)WG * N));
     if (cap < 1) cap = 1;
@@ -2094,19 +2136,29 @@ Launch plan(anl_gofrt *g, const uint64_t *primo, const uint32_t *n, uint32_t nbl
     // its t0 range finer (the counts are sums of integers, so the split
     // changes no result).  2,048 -> 4,096, rounded up: 1,000 atoms, 150 t0, 51
     // lags 4.25 -> 4.02 ms; 3,000 atoms, 20 t0, 10 lags 2.16 -> 1.76; 8,192
-    // gains nothing more
+    // gains nothing more.  Not finer than the flushes allow (flush_chunk)
     const uint64_t ntiles = (N + L.tile - 1) / L.tile;
     const uint64_t want = (4096 + nblocks - 1) / nblocks;
+    auto lags_of = [&](uint32_t nb) {
+        const uint32_t leff = (nb < g->lmax || g->lmax == 0) ? nb : g->lmax;
+        return std::max<uint64_t>(1, (leff + g->every - 1) / g->every);
+    };
+    double U = 0;
+    for (uint32_t bi = 0; bi < nblocks; bi++)
+        U += (double)(ntiles * lags_of(n[bi])) * ((n[bi] + g->skip - 1) / g->skip);
+    L.pairs = U;
+    const uint64_t least = flush_chunk(g, L.tile, form, cells, U);
     for (uint32_t bi = 0; bi < nblocks; bi++) {
         uint32_t leff = (n[bi] < g->lmax || g->lmax == 0) ? n[bi] : g->lmax;
         L.blocks.push_back(BlockInfo{primo[bi], leff, 0});
         L.leff_max = std::max(L.leff_max, leff);
         uint32_t n0 = (n[bi] + g->skip - 1) / g->skip;  // t0 = 0, skip, ... < n
-        const uint64_t units = ntiles * std::max<uint64_t>(1, (leff + g->every - 1) / g->every);
+        const uint64_t units = ntiles * lags_of(n[bi]);
         uint64_t chunk_b = chunk;
         if (units * ((n0 + chunk - 1) / chunk) < want) {
             const uint64_t items = (want + units - 1) / units;
-            chunk_b = std::min(chunk, std::max<uint64_t>(split ? std::min<uint64_t>(4, n0) : 1, n0 / items));
+            chunk_b = std::min(chunk, std::max<uint64_t>(split ? std::min<uint64_t>(4, n0) : 1,
+                                                         std::max(n0 / items, std::min<uint64_t>(least, n0))));
         }
         if (nblocks == 1) {
             L.k1 = n0;
@@ -2308,7 +2360,7 @@ GofrtPrepared gofrt_prepare(anl_gofrt *g, const Launch &L, uint64_t out_len, int
     const bool colc = g->tune.cluster == 2 || g->tune.cluster == 4;
     const int qcl = colc ? SQCAP_CLC : SQCAP_CL;
     const bool cluster_ok = g->tune.cluster != 0 && form == ANL_GOFRT_SCREENED && a.rho_cap > 0 &&
-                            screened_lds(qcl, colc) <= 160 * 1024 && (g->tuned || clusters_fit(g, a.rho_cap));
+                            screened_lds(qcl, colc) <= 160 * 1024 && (g->tuned || clusters_fit(g, a.rho_cap, L.pairs));
     P.lds = form == ANL_GOFRT_FP64 ? common : (cluster_ok ? screened_lds(qcl, colc) : screened_lds(SQCAP, false));
     if (P.lds > 160 * 1024) fail(ANL_ERR_ARG, "histogram does not fit in LDS (reduce nbin or types)");
     P.lds = std::max<size_t>(P.lds, 64 * sizeof(unsigned));  // the plain form adds 0 to words 0 .. 63
