@@ -1965,11 +1965,14 @@ int choose_form(anl_gofrt *g) {
 
 // Whether the automatic form of a trajectory with a changing cell takes
 // gofrt_cells_kernel: the screen's preconditions hold in every frame's cell.
-// From 769 atoms (more than three tiles of i; 40 t0, 10 lags, plain -> this at
-// rmax 0.3 and 0.49 of the cell length: 600 atoms 243 -> 285 us (0.15) and 342
-// -> 442, 800 481 -> 389 and 504 -> 568, 1,000 658 -> 491 and 715 -> 679, 2,000
-// at 0.49 2.29 -> 1.84 ms, 3,000 tilted 6.16 -> 4.08, 10,000 at 0.2 42.5 ->
-// 11.2); below, the plain form's smaller tiles fill the chip better.
+// From 769 atoms (more than three tiles of i): there it is the faster one up to
+// rmax half the cell, but for few lags of that range (us, plain -> this at rmax
+// 0.3 and 0.49 of the cell length; 40 t0 x 10 lags: 769 atoms 512 -> 374 and 551
+// -> 516, 800 531 -> 378 and 570 -> 539, 1,000 633 -> 467 and 696 -> 651, 1,200
+// 849 -> 580 and 923 -> 783; 150 x 50, 1,000 atoms 9,221 -> 3,851 and 10,173 ->
+// 8,021; 60 x 4, 1,200 atoms 585 -> 446 and 634 -> 681; 10,000 atoms at 0.2 42.5
+// -> 11.2 ms).  Below, the plain form's smaller tiles fill the chip better: 600
+// atoms, 40 x 10 243 -> 285 and 342 -> 442.
 constexpr uint64_t CELLS_MIN_ATOMS = 769;
 bool use_cells(anl_gofrt *g) {
     anl_traj *tr = g->tr;
