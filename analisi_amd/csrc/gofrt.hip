@@ -645,7 +645,7 @@ __global__ __launch_bounds__(SPLIT ? SPLIT_WG : WG) void gofrt_fp64_kernel(const
         for (int v = 0; v < U; v++) {
             const float f2 = (float)d2[v], u = (__builtin_amdgcn_sqrtf(f2) - rminf) * inv_drf;
             const bool sure = (fabsf(u - rintf(u)) > margin) | (f2 <= zero_d2), count = in[v] & sure;
-            need |= in[v] & !sure ? 1u << v : 0u;
+            need |= (in[v] & !sure) ? 1u << v : 0u;
             const uint32_t at = (slot == js + v ? rowself : row0 + row[v]) + (uint32_t)floor_i32(u);
             atomicAdd(count ? &hist[at] : (unsigned *)smem + (threadIdx.x & 63u), count ? 1u : 0u);
         }

@@ -34,11 +34,14 @@ extern "C" {
 #define ANL_ERR_HEADER 6       /* GK header not found (greenkubo...cpp:62-69) */
 
 /* g(r,t) arithmetic forms */
-#define ANL_GOFRT_FP64 0       /* plain FP64 evaluation of every ordered pair */
+#define ANL_GOFRT_FP64 0       /* plain FP64 evaluation of every ordered pair; its bin by the FP64
+                                  edges, or by an FP32 quotient of the FP64 distance where that is
+                                  farther from an integer than twice its error (the same bin) */
 #define ANL_GOFRT_SCREENED 1   /* 16-bit fixed-point screen of every pair, exact FP64
                                   evaluation of every candidate (same counts) */
 #define ANL_GOFRT_AUTO 2       /* SCREENED when its preconditions hold (in a changing cell: in every
-                                * frame's, from 769 atoms), else FP64 */
+                                * frame's, from 769 atoms: there by FP32 products of 32-bit fractions,
+                                * FP64 wherever their error could change a count), else FP64 */
 
 /* Message of the last failed call on this thread ("" if none). */
 const char *anl_last_error(void);
