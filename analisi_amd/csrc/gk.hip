@@ -350,8 +350,8 @@ __device__ __forceinline__ void wave_sync_lds() {
 // LDS port is next (3 rows of 8 bytes per mean and t0: 12 of 16 clocks).  A
 // stage of 16 t0 goes through one LDS buffer: a wavefront's LDS operations
 // stay in order, so the next stage's values, loaded to registers while this
-// one is summed, are stored after its last read.  VALU busy 85% on 20,000
-// lags x 60,000 t0 x 8 blocks, 2 currents; 32 such blocks 95 ms per call
+// one is summed, are stored after its last read.  VALU busy 83% on 20,000
+// lags x 60,000 t0 x 8 blocks, 2 currents; 32 such blocks 90 ms per call
 // with its 72 MB copied to the host (186 ms with one thread per lag).
 template <int NCUR, int CH>
 __global__ __launch_bounds__(64, 3) void gk_dense_kernel(const GkArgs a) {
@@ -1336,7 +1336,7 @@ int anl_gk_calculate_blocks_async(anl_series *s, const uint32_t *idx_j, uint32_t
 // copy: while the kernels run, up to 8 threads write a byte of each page of
 // their share; then they copy their part of every piece that has arrived in
 // the ring while the next ones arrive.  16 blocks x 8,000 lags (14 MB), MFMA: a
-// call 1,310 us with a plain copy from memory allocated for it, 770 now, of
+// call 1,310 us with a plain copy from memory allocated for it, 820 now, of
 // which the kernels are 305.
 int anl_gk_calculate_blocks(anl_series *s, const uint32_t *idx_j, uint32_t ncur, uint32_t skip, uint32_t tmax,
                             uint32_t n_seg, int subtract_mean, uint32_t start_mean, const uint64_t *primo,
