@@ -999,17 +999,20 @@ uint64_t radius_bytes(const anl_sph *h, uint64_t nfr) {
     return h->block_screen ? nfr * ((h->tr->N + 63) / 64) * sizeof(double4) : 0;
 }
 
-// Atoms up to which the neighbour lists go through all blocks: their spheres are a
-// launch of their own, 5 us of a call (22 atoms, one frame: 80 us with them, 57
-// without; 200 atoms, 60 frames: no difference).
-constexpr uint64_t SANN_NO_SPHERES = 256;
+// Whether the neighbour lists skip blocks by their spheres: those are a launch of
+// their own, 3 to 16 us of a call, which few atoms do not earn back, nor a few
+// frames of not many more.  Us a call without and with them: 22 atoms, one frame 57
+// and 80; 300, 2 frames 70 and 86, 60 frames 147 and 164; 600, 8 102 and 118, 60
+// 256 and 267; 800, 8 121 and 135, 60 352 and 350; 1,200, 60 554 and 489; 2,000,
+// 2 153 and 155, 60 1,103 and 730.
+bool sann_spheres(uint64_t N, uint64_t nfr) { return N > 1024 || (N > 640 && N * nfr > 8192); }
 
 // one launch of launch_density, which checks the sizes and reads the overflow of the lists
 void launch_density_range(anl_sph *h, uint64_t f0, uint64_t fstride, uint32_t nfr, double *S, double4 *rad,
                           hipStream_t s, int32_t *nbr, uint32_t lm) {
     SphDensArgs a{};
     a.fstride = fstride;
-    a.block_rad = h->block_screen && !(h->sann && h->tr->N <= SANN_NO_SPHERES) ? rad : nullptr;
+    a.block_rad = h->block_screen && (!h->sann || sann_spheres(h->tr->N, nfr)) ? rad : nullptr;
     auto block_spheres = [&] {
         if (!a.block_rad) return;
         const uint64_t nb = (uint64_t)nfr * ((h->tr->N + 63) / 64);

@@ -60,10 +60,16 @@ def names(e):
 h = system(100, 40)
 h.calculate(20, 10, 2, 0)
 assert names(log()) == ["zero", "density_sann", "gram_mfma", "reduce"]
-h = system(257, 40)
+h = system(640, 40)
+h.calculate(20, 10, 2, 0)
+assert names(log()) == ["zero", "density_sann", "gram_mfma", "reduce"]
+h = system(1024, 8)                                   # few frames of more atoms
+h.calculate(4, 4, 1, 0)
+assert names(log()) == ["zero", "density_sann", "gram_mfma", "reduce"]
+h = system(641, 40)
 h.calculate(20, 10, 2, 0)
 assert names(log()) == ["zero", "block_radius", "density_sann", "gram_mfma", "reduce"]
-h.set_budget(5 * 257 * 9 * 8)                         # densities of two t1 values and their lags
+h.set_budget(5 * 641 * 9 * 8)                         # densities of two t1 values and their lags
 h.calculate(4, 4, 1, 0)
 n = names(log())
 assert n.count("reduce") == n.count("gram_mfma") == 2 and n[-1] == "reduce", n
